@@ -410,8 +410,8 @@ def main():
         ("row_max", "k_reduce_rows", n1 * 4 + ROWS * 4, n1, lambda: _lib.neural_reduce_max(T["Y"]._ptr, 1, T["rmax"]._ptr)),
         ("row_argmax", "k_reduce_rows", n1 * 4 + ROWS * 8, n1,
          lambda: _lib.neural_reduce_argmax(T["Y"]._ptr, 1, ctypes.c_void_p(ridx.data_ptr()))),
-        ("softmax", "k_softmax_wave_f32<false>", 2 * n2 * 4, n2, lambda: _lib.neural_softmax(T["P"]._ptr, T["S"]._ptr)),
-        ("log_softmax", "k_softmax_wave_f32<true>", 2 * n2 * 4, n2,
+        ("softmax", "k_softmax_rows<float, false>", 2 * n2 * 4, n2, lambda: _lib.neural_softmax(T["P"]._ptr, T["S"]._ptr)),
+        ("log_softmax", "k_softmax_rows<float, true>", 2 * n2 * 4, n2,
          lambda: _lib.neural_log_softmax(T["L"]._ptr, T["S"]._ptr)),
     ]
     step_bytes = sum(o[2] for o in step_ops)

@@ -17,8 +17,11 @@
 // softmax.  A NaN anywhere in a row makes the whole row NaN, as in the
 // reference (the NaN reaches the sum).
 //
-// Rows of up to 64*16 vectors (4096 f32 / 2048 f64 values) are register
-// resident: one wave per row, a single HBM read and a single write.
+// A row is held in registers by one group of lanes -- a wave up to 4096 f32 /
+// 2048 f64 values, a block of 256 to 1024 lanes beyond, up to 98304 / 49152
+// values -- so it is read once and written once at any width and alignment:
+// 16-byte accesses at the element's own alignment and one scalar per lane for
+// the last cols % VN values.  Wider rows are read twice.
 #include <cmath>
 
 #include <hip/hip_ext.h>
@@ -40,232 +43,288 @@ template <> NH_DEV double neg_inf<double>() { return -__builtin_inf(); }
 // passes through and makes the row's sum NaN, as in the reference.
 NH_DEV float exp_diff_f32(float x, double md) { return exp_d2f(double(x) - md); }
 
-// One wave per row (RPW rows per wave: all loads of the wave's rows issued
-// before any arithmetic).
-template <bool LOG, int VPL, bool FULL>
-NH_DEV void softmax_row_f32(f32x4 (&v)[VPL], f32x4 *__restrict__ yr, int64_t ncv, int lane)
-{
-    const auto in_row = [&](int k) { return FULL || lane + int64_t(k) * 64 < ncv; };
-    float m = -__builtin_inff();
+// Group-wide max (NaN-ignoring) and sum over the NT lanes that share a row:
+// 4, 16 or 32 lanes of a wave (DPP moves, and one swizzle across 16), one wave,
+// or a block of NT lanes through LDS.
+template <int NT>
+struct RowGrp {
+    static constexpr int kWaves = NT < 64 ? 1 : NT / 64;
+    template <typename T> NH_DEV static T dpp(T v, int step)
+    {
+        if constexpr (sizeof(T) == 4)
+            return step == 0 ? dpp_f<kDppXor1>(v) : step == 1 ? dpp_f<kDppXor2>(v)
+                 : step == 2 ? dpp_f<kDppHalfMirror>(v) : dpp_f<kDppMirror>(v);
+        else
+            return step == 0 ? dpp_d<kDppXor1>(v) : step == 1 ? dpp_d<kDppXor2>(v)
+                 : step == 2 ? dpp_d<kDppHalfMirror>(v) : dpp_d<kDppMirror>(v);
+    }
+    template <typename T, typename C>
+    NH_DEV static T part(T v, C comb)
+    {
 #pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        if (in_row(k)) {
+        for (int i = 0; i < (NT == 4 ? 2 : 4); i++) v = comb(v, dpp(v, i));
+        return NT == 32 ? comb(v, __shfl_xor(v, 16, 64)) : v;
+    }
+    template <typename T, typename C>
+    NH_DEV static T across(T w, T *lds, C comb)
+    {
+        if constexpr (kWaves == 1) {
+            return w;
+        } else {
+            if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = w;
+            __syncthreads();
+            T r = lds[0];
 #pragma unroll
-            for (int j = 0; j < 4; j++) m = __builtin_fmaxf(m, v[k][j]);
+            for (int i = 1; i < kWaves; i++) r = comb(r, lds[i]);
+            return r;
         }
     }
-    const double md = double(wave_fmax(m));
-    double s = 0.0;
-    if (!LOG) {
-        // e_j kept in the input registers, rounded to float as the reference does.
-#pragma unroll
-        for (int k = 0; k < VPL; k++) {
-            if (in_row(k)) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float e = exp_diff_f32(v[k][j], md);
-                    v[k][j] = e;
-                    s += double(e);
-                }
-            }
-        }
-        s = wave_dsum(s);
-        const float rs = 1.0f / float(s);
-#pragma unroll
-        for (int k = 0; k < VPL; k++)
-            if (in_row(k)) st_nt(yr + lane + k * 64, v[k] * rs);
-    } else {
-#pragma unroll
-        for (int k = 0; k < VPL; k++) {
-            if (in_row(k)) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) s += double(exp_diff_f32(v[k][j], md));
-            }
-        }
-        s = wave_dsum(s);
-        // y = (x - m) - lse in float: x - m <= 0 and lse >= 0, so the two
-        // terms never cancel and two float roundings (plus lse's) leave y
-        // within ~2e-7 relative of the double expression; NaN / Inf rows give
-        // the same NaNs as the double form.
-        const float lse = float(log_ge1(s));  // s >= 1: the row maximum contributes exp(0) = 1
-        const float mf = float(md);
-#pragma unroll
-        for (int k = 0; k < VPL; k++) {
-            if (in_row(k)) st_nt(yr + lane + k * 64, (v[k] - mf) - lse);
-        }
+    NH_DEV static float max(float v, float *lds)
+    {
+        if constexpr (NT < 64) return part(v, [](float a, float b) { return __builtin_fmaxf(a, b); });
+        else return across(wave_fmax(v), lds, [](float a, float b) { return __builtin_fmaxf(a, b); });
     }
-}
+    NH_DEV static double max(double v, double *lds)
+    {
+        if constexpr (NT < 64) return part(v, [](double a, double b) { return __builtin_fmax(a, b); });
+        else return across(wave_max_ignore_nan(v), lds, [](double a, double b) { return __builtin_fmax(a, b); });
+    }
+    NH_DEV static double sum(double v, double *lds)
+    {
+        if constexpr (NT < 64) return part(v, [](double a, double b) { return a + b; });
+        else return across(wave_dsum(v), lds, [](double a, double b) { return a + b; });
+    }
+};
 
-template <bool LOG, int VPL, bool FULL, int RPW>
-__global__ __launch_bounds__(kSmBlock) void k_softmax_wave_f32(const float *__restrict__ x, float *__restrict__ y,
-                                                               int64_t rows, int64_t cols, int64_t r_base)
-{
-    using V = f32x4;
-    const int lane = threadIdx.x & 63;
-    const int64_t r0 = r_base + (int64_t(blockIdx.x) * (kSmBlock / 64) + (threadIdx.x >> 6)) * RPW;
-    if (r0 >= rows) return;  // uniform per wave
-    const int64_t ncv = cols / 4;
-    V v[RPW][VPL];
-#pragma unroll
-    for (int q = 0; q < RPW; q++) {
-        if (r0 + q < rows) {
-            const V *xr = reinterpret_cast<const V *>(x + (r0 + q) * cols);
-#pragma unroll
-            for (int k = 0; k < VPL; k++)
-                if (FULL || lane + int64_t(k) * 64 < ncv) v[q][k] = ld_nt(xr + lane + k * 64);
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < RPW; q++)
-        if (r0 + q < rows)
-            softmax_row_f32<LOG, VPL, FULL>(v[q], reinterpret_cast<V *>(y + (r0 + q) * cols), ncv, lane);
-}
-
-template <bool LOG, int VPL>
-__global__ __launch_bounds__(kSmBlock) void k_softmax_wave_f64(const double *__restrict__ x, double *__restrict__ y,
-                                                               int64_t rows, int64_t cols, int64_t r_base)
-{
-    using V = f64x2;
-    const int lane = threadIdx.x & 63;
-    const int64_t r = r_base + int64_t(blockIdx.x) * (kSmBlock / 64) + (threadIdx.x >> 6);
-    if (r >= rows) return;  // uniform per wave
-    const V *xr = reinterpret_cast<const V *>(x + r * cols);
-    V *yr = reinterpret_cast<V *>(y + r * cols);
-    const int64_t ncv = cols / 2;
-
-    V v[VPL];
-#pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int64_t c = lane + int64_t(k) * 64;
-        if (c < ncv) v[k] = ld_nt(xr + c);
-    }
-    double m = -__builtin_inf();
-#pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int64_t c = lane + int64_t(k) * 64;
-        if (c < ncv) {
-#pragma unroll
-            for (int j = 0; j < 2; j++) m = v[k][j] > m ? v[k][j] : m;
-        }
-    }
-    m = wave_max_ignore_nan(m);
-    double s = 0.0;
-#pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int64_t c = lane + int64_t(k) * 64;
-        if (c < ncv) {
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const double e = exp(v[k][j] - m);
-                if (!LOG) v[k][j] = e;
-                s += e;
-            }
-        }
-    }
-    s = wave_sum(s);
-    const double lse = LOG ? log_ge1(s) : 0.0;  // s >= 1 (the maximum contributes 1)
-#pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int64_t c = lane + int64_t(k) * 64;
-        if (c < ncv) {
-            V o;
-#pragma unroll
-            for (int j = 0; j < 2; j++) o[j] = LOG ? (v[k][j] - m) - lse : v[k][j] / s;
-            st_nt(yr + c, o);
-        }
-    }
-}
-
-// General rows: one block per row, three passes over the row.
-template <typename T>
-NH_DEV T block_max_ignore_nan(T v)
-{
-    __shared__ T lds[kSmBlock / 64];
-    v = wave_max_ignore_nan(v);
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
-    __syncthreads();
-    T r = lds[0];
-    for (int i = 1; i < kSmBlock / 64; i++) r = (lds[i] > r) ? lds[i] : r;
-    __syncthreads();
-    return r;
-}
-
-NH_DEV double block_sum(double v)
-{
-    __shared__ double lds[kSmBlock / 64];
-    v = wave_sum(v);
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
-    __syncthreads();
-    double r = lds[0];
-    for (int i = 1; i < kSmBlock / 64; i++) r += lds[i];
-    __syncthreads();
-    return r;
-}
-
-NH_DEV float row_exp(float x, float m) { return exp_diff_f32(x, double(m)); }
+NH_DEV float row_exp(float x, double m) { return exp_diff_f32(x, m); }
 NH_DEV double row_exp(double x, double m) { return exp(x - m); }
 
+// One output value.  f32 takes its last step in double and rounds once; the
+// softmax multiplies by the reciprocal of the sum there (a double division
+// per value made the instruction count, not HBM, the bound).
 template <typename T, bool LOG>
-__global__ __launch_bounds__(kSmBlock) void k_softmax_block(const T *__restrict__ x, T *__restrict__ y, int64_t cols,
-                                                            int64_t r_base)
+NH_DEV T row_out(T v, double md, double lse, double s, double rs)
 {
+    // hides the value's origin: the compiler would keep double(v) from the sum
+    // (two more registers per value) instead of converting again here
+    if constexpr (sizeof(T) == 4) asm("" : "+v"(v));
+    if constexpr (LOG) return T((double(v) - md) - lse);
+    else if constexpr (sizeof(T) == 4) return T(double(v) * rs);
+    else return v / s;
+}
+
+// One row per group of NT lanes, held in VPT vectors per lane (and the last
+// cols % VN values in one scalar of lanes 0 .. rem - 1, whose other lanes hold
+// -inf: it adds 0 to the sum, or NaN where the row is NaN anyway).  FULL: the
+// row is exactly NT * VPT vectors, so no element needs a bounds check.
+//
+// What bounds it: HBM, one read and one write, while the rows in flight per
+// CU cover the latency; hence VPT <= 25 (two 512-lane blocks per CU at 51200
+// f32 values; __launch_bounds__ asks for them) and 1024 lanes only past that.
+// f32, before (three passes of 4-byte accesses per row for odd or long rows)
+// and after: see launch_softmax.
+template <typename T, bool LOG, int NT, int VPT, bool FULL>
+__global__ __launch_bounds__(NT < kSmBlock ? kSmBlock : NT, NT == 512 ? 4 : 1) void k_softmax_rows(
+    const T *__restrict__ x, T *__restrict__ y, int64_t rows, int64_t cols, int64_t r_base)
+{
+    using V = typename Vec16<T>::type;
+    using U = typename VecU<T>::type;
+    using G = RowGrp<NT>;
+    constexpr int VN = Vec16<T>::n;
+    constexpr int RPB = NT < kSmBlock ? kSmBlock / NT : 1;
+    __shared__ T lds_m[G::kWaves];
+    __shared__ double lds_s[G::kWaves];
+    const int lane = threadIdx.x % NT;
+    const int64_t r = r_base + int64_t(blockIdx.x) * RPB + threadIdx.x / NT;
+    if (RPB > 1 && r >= rows) return;  // uniform per group; a block of one row has one
+    const T *xr = x + r * cols;
+    T *yr = y + r * cols;
+    const int ncv = int(cols / VN), rem = FULL ? 0 : int(cols % VN);
+    const auto in_row = [&](int k) { return FULL || lane + k * NT < ncv; };
+    V v[VPT];
+    T vt = neg_inf<T>();
+#pragma unroll
+    for (int k = 0; k < VPT; k++)
+        if (in_row(k)) v[k] = __builtin_nontemporal_load(reinterpret_cast<const U *>(xr) + lane + k * NT);
+    if (rem && lane < rem) vt = xr[int64_t(ncv) * VN + lane];
+
+    T m = vt == vt ? vt : neg_inf<T>();
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        if (in_row(k)) {
+#pragma unroll
+            for (int j = 0; j < VN; j++) {
+                if constexpr (sizeof(T) == 4) m = __builtin_fmaxf(m, v[k][j]);
+                else m = v[k][j] > m ? v[k][j] : m;
+            }
+        }
+    }
+    const double md = double(G::max(m, lds_m));
+    double s = 0.0;
+    // softmax: e_j kept in the input registers, rounded to T as the reference does
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        if (in_row(k)) {
+#pragma unroll
+            for (int j = 0; j < VN; j++) {
+                const T e = row_exp(v[k][j], md);
+                if (!LOG) v[k][j] = e;
+                s += double(e);
+            }
+        }
+    }
+    if (rem) {  // uniform
+        const T e = row_exp(vt, md);
+        if (!LOG) vt = e;
+        s += double(e);
+    }
+    s = G::sum(s, lds_s);
+    double lse = 0.0;  // s >= 1: the maximum contributes 1
+    if constexpr (LOG && sizeof(T) == 4) lse = log_ge1(s);
+    else if constexpr (LOG) lse = NT <= 64 && rem == 0 ? log_ge1(s) : log(s);
+    const double rs = LOG ? 0.0 : 1.0 / s;
+#pragma unroll
+    for (int k = 0; k < VPT; k++) {
+        if (in_row(k)) {
+            V o;
+#pragma unroll
+            for (int j = 0; j < VN; j++) o[j] = row_out<T, LOG>(v[k][j], md, lse, s, rs);
+            __builtin_nontemporal_store(o, reinterpret_cast<U *>(yr) + lane + k * NT);
+        }
+    }
+    if (rem && lane < rem) yr[int64_t(ncv) * VN + lane] = row_out<T, LOG>(vt, md, lse, s, rs);
+}
+
+// Rows wider than the registers of a block: one 1024-lane block per row, two
+// reads.  Each lane keeps a running maximum and the sum of exp(x - maximum),
+// rescaled (in double) when a batch of four vectors raises the maximum; the
+// block's sum is the rescaled total, and the second pass writes the outputs.
+constexpr int kSmWide = 1024;
+template <typename T, bool LOG>
+__global__ __launch_bounds__(kSmWide) void k_softmax_stream(const T *__restrict__ x, T *__restrict__ y, int64_t cols,
+                                                           int64_t r_base)
+{
+    using V = typename Vec16<T>::type;
+    using U = typename VecU<T>::type;
+    using G = RowGrp<kSmWide>;
+    constexpr int VN = Vec16<T>::n, UN = 4;
+    __shared__ T lds_m[G::kWaves];
+    __shared__ double lds_s[G::kWaves];
     const int64_t r = r_base + blockIdx.x;
     const T *xr = x + r * cols;
     T *yr = y + r * cols;
+    const U *xv = reinterpret_cast<const U *>(xr);
+    U *yv = reinterpret_cast<U *>(yr);
+    const int64_t ncv = cols / VN;
     T m = neg_inf<T>();
-    for (int64_t j = threadIdx.x; j < cols; j += kSmBlock) m = xr[j] > m ? xr[j] : m;
-    m = block_max_ignore_nan(m);
-    const double md = double(m);
     double s = 0.0;
-    for (int64_t j = threadIdx.x; j < cols; j += kSmBlock) s += double(row_exp(xr[j], m));
-    s = block_sum(s);
-    if (LOG) {
-        const double lse = log(s);
-        for (int64_t j = threadIdx.x; j < cols; j += kSmBlock) yr[j] = T((double(xr[j]) - md) - lse);
-    } else {
-        for (int64_t j = threadIdx.x; j < cols; j += kSmBlock) yr[j] = T(double(row_exp(xr[j], m)) / s);
-    }
-}
-
-template <typename K, typename... Args>
-static void launch_timed(K kernel, unsigned g, Args... args)
-{
-    NH_LAUNCH(kernel, dim3(g), dim3(kSmBlock), 0, stream(), args...);
-}
-
-template <typename T, bool LOG, int VPL>
-static void launch_wave(const T *x, T *y, int64_t rows, int64_t cols)
-{
-    for_row_launches(rows, kSmBlock / 64, [&](unsigned g, int64_t base) {
-        if constexpr (sizeof(T) == 4) {
-            // (two rows per wave measured slower on MI355X: 89.7 vs 86.2 us at [65536,1024])
-            if (cols == int64_t(VPL) * 256)
-                launch_timed(k_softmax_wave_f32<LOG, VPL, true, 1>, g, x, y, rows, cols, base);
-            else
-                launch_timed(k_softmax_wave_f32<LOG, VPL, false, 1>, g, x, y, rows, cols, base);
-        } else {
-            launch_timed(k_softmax_wave_f64<LOG, VPL>, g, x, y, rows, cols, base);
+    double mr = 0.0;  // what the sum's exponents are relative to: m, or 0 while the lane has seen only -inf
+    const auto rise = [&](T bm) {
+        if (bm > m) {
+            if (s != 0.0) s *= exp(mr - double(bm));
+            m = bm;
+            mr = double(bm);
         }
+    };
+    for (int64_t c = threadIdx.x; c < ncv; c += UN * kSmWide) {
+        V v[UN];
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if (c + u * kSmWide < ncv) v[u] = xv[c + u * kSmWide];
+        T bm = neg_inf<T>();
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if (c + u * kSmWide < ncv) {
+#pragma unroll
+                for (int j = 0; j < VN; j++) bm = v[u][j] > bm ? v[u][j] : bm;
+            }
+        rise(bm);
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if (c + u * kSmWide < ncv) {
+#pragma unroll
+                for (int j = 0; j < VN; j++) s += double(row_exp(v[u][j], mr));
+            }
+    }
+    const int64_t jt = ncv * VN + threadIdx.x;  // at most VN - 1 values past the vectors
+    if (jt < cols) {
+        rise(xr[jt]);
+        s += double(row_exp(xr[jt], mr));
+    }
+    const double md = double(G::max(m, lds_m));
+    // (s = 0: the lane saw only -inf; the outputs of a row of -inf are NaN below)
+    s = G::sum(s == 0.0 ? 0.0 : s * exp(mr - md), lds_s);
+    const double lse = LOG ? log(s) : 0.0;
+    const double rs = LOG ? 0.0 : 1.0 / s;
+    for (int64_t c = threadIdx.x; c < ncv; c += UN * kSmWide) {
+        V v[UN];
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if (c + u * kSmWide < ncv) v[u] = xv[c + u * kSmWide];
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if (c + u * kSmWide < ncv) {
+                V o;
+#pragma unroll
+                for (int j = 0; j < VN; j++)
+                    o[j] = row_out<T, LOG>(LOG ? v[u][j] : T(row_exp(v[u][j], md)), md, lse, s, rs);
+                __builtin_nontemporal_store(o, yv + c + u * kSmWide);
+            }
+    }
+    if (jt < cols) yr[jt] = row_out<T, LOG>(LOG ? xr[jt] : T(row_exp(xr[jt], md)), md, lse, s, rs);
+}
+
+template <typename T, bool LOG, int NT, int VPT>
+static void launch_rows(const T *x, T *y, int64_t rows, int64_t cols)
+{
+    for_row_launches(rows, NT < kSmBlock ? kSmBlock / NT : 1, [&](unsigned g, int64_t base) {
+        constexpr int block = NT < kSmBlock ? kSmBlock : NT;
+        if constexpr (NT <= 64 && sizeof(T) == 4) {
+            if (cols == int64_t(NT) * VPT * Vec16<T>::n) {
+                NH_LAUNCH((k_softmax_rows<T, LOG, NT, VPT, true>), dim3(g), dim3(block), 0, stream(), x, y, rows,
+                          cols, base);
+                return;
+            }
+        }
+        NH_LAUNCH((k_softmax_rows<T, LOG, NT, VPT, false>), dim3(g), dim3(block), 0, stream(), x, y, rows, cols, base);
     });
 }
 
+// The smallest group whose registers hold the row: its lanes stay busy and
+// most rows are in flight.  Narrow rows share a wave, 16 rows of up to 4
+// vectors, 4 of up to 64, 2 of up to 128; where the rows' ends are not vector
+// ends the last take a whole wave (its longer stores: [100000, 511] 73 against
+// 84 us).  Before (a wave per aligned row of up to 4096 values, else three
+// passes of 4-byte accesses) -> now, us:
+//   f32 [55392, 577] softmax / log-softmax  159 -> 45 / 160 -> 47 (256 MB, 5.7 TB/s)
+//       [200000, 16] 42.2 -> 6.0, [200000, 64] 47.4 -> 18.1, [200000, 63] 203 -> 23.7
+//       [100000, 197] 148 -> 37.4, [100000, 260] 43.2 -> 38.8, [100000, 400] 54.0 -> 53.4 (log 52.8 -> 54.5)
+//       [65536, 1024] 87.8 -> 85.3, [8192, 4096] 52.0 -> 46.3, [8192, 4097] 129 -> 52, [4096, 8192] 116 -> 45.5
+//   f64 [100000, 33] 118 -> 12.4, [32768, 1024] the same, [4096, 8191] log-softmax 179 -> 100
+//   log-softmax and argmax, f32: [64, 32000] 77 -> 17.8, [100, 98000] 332 -> 41, [128, 131072] 429 -> 60
 template <typename T, bool LOG>
 static int launch_softmax(const T *x, T *y, int64_t rows, int64_t cols)
 {
-    constexpr int VN = Vec16<T>::n;
-    const bool vec = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15u) == 0 && cols % VN == 0;
-    const int64_t ncv = cols / VN;
-    if (vec && ncv <= 64 * 16) {
-        if (ncv <= 64) launch_wave<T, LOG, 1>(x, y, rows, cols);
-        else if (ncv <= 128) launch_wave<T, LOG, 2>(x, y, rows, cols);
-        else if (ncv <= 256) launch_wave<T, LOG, 4>(x, y, rows, cols);
-        else if (ncv <= 512) launch_wave<T, LOG, 8>(x, y, rows, cols);
-        else launch_wave<T, LOG, 16>(x, y, rows, cols);
-    } else {
+    const int64_t ncv = cols / Vec16<T>::n;
+    if (ncv <= 4) launch_rows<T, LOG, 4, 1>(x, y, rows, cols);
+    else if (ncv <= 16) launch_rows<T, LOG, 16, 1>(x, y, rows, cols);
+    else if (ncv <= 16 * 2) launch_rows<T, LOG, 16, 2>(x, y, rows, cols);
+    else if (ncv <= 16 * 4) launch_rows<T, LOG, 16, 4>(x, y, rows, cols);
+    else if (ncv <= 32 * 4 && cols % Vec16<T>::n == 0) launch_rows<T, LOG, 32, 4>(x, y, rows, cols);
+    else if (ncv <= 64 * 2) launch_rows<T, LOG, 64, 2>(x, y, rows, cols);
+    else if (ncv <= 64 * 4) launch_rows<T, LOG, 64, 4>(x, y, rows, cols);
+    else if (ncv <= 64 * 8) launch_rows<T, LOG, 64, 8>(x, y, rows, cols);
+    else if (ncv <= 64 * 16) launch_rows<T, LOG, 64, 16>(x, y, rows, cols);
+    else if (ncv <= 256 * 8) launch_rows<T, LOG, 256, 8>(x, y, rows, cols);
+    else if (ncv <= 256 * 16) launch_rows<T, LOG, 256, 16>(x, y, rows, cols);
+    else if (ncv <= 512 * 16) launch_rows<T, LOG, 512, 16>(x, y, rows, cols);
+    else if (ncv <= 512 * 25) launch_rows<T, LOG, 512, 25>(x, y, rows, cols);
+    else if (ncv <= 1024 * 16) launch_rows<T, LOG, 1024, 16>(x, y, rows, cols);
+    else if (ncv <= 1024 * 24) launch_rows<T, LOG, 1024, 24>(x, y, rows, cols);
+    else
         for_row_launches(rows, 1, [&](unsigned g, int64_t base) {
-            NH_LAUNCH((k_softmax_block<T, LOG>), dim3(g), dim3(kSmBlock), 0, stream(), x, y, cols, base);
+            NH_LAUNCH((k_softmax_stream<T, LOG>), dim3(g), dim3(kSmWide), 0, stream(), x, y, cols, base);
         });
-    }
     return check_launch();
 }
 

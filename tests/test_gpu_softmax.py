@@ -74,6 +74,59 @@ def test_softmax_errors(pn):
     assert pn.core._lib.neural_softmax(c._ptr, a._ptr) == pn.NeuralError.SHAPE_MISMATCH
 
 
+# Widths at the edges of the row kernels (4 or 16 lanes per row up to 256
+# values; vectors held per lane: 2 .. 16 in a wave, 8 / 16 / 25 in blocks of 256 / 512, 16 / 24 in 1024, two reads beyond),
+# for f32; the f64 edges lie at half of each.
+_EDGES = [1, 2, 3, 5, 15, 16, 19, 20, 63, 64, 67, 68, 127, 129, 255, 256, 257, 511, 513, 1023, 1025, 2047, 2049, 4093, 4096, 4099, 8191, 8197, 16383, 16385,
+          32767, 32769, 51197, 51201, 65535, 65537, 98301, 98304, 98305, 98311, 140003]
+
+
+@pytest.mark.parametrize("cols", _EDGES)
+@pytest.mark.parametrize("dt", ["float32", "float64"])
+def test_row_kernel_edges(pn, dt, cols):
+    """Softmax and log-softmax at each kernel's edges, rows starting at any
+    element offset, against the float64 formula (REL32 / REL64); -inf entries,
+    a NaN row and an all -inf row among them, and in place."""
+    import torch
+    T = getattr(torch, dt)
+    cols = cols if dt == "float32" else max(1, (cols + 1) // 2)
+    rows = 7 if cols > 1024 else 71
+    g = torch.Generator().manual_seed(cols)
+    x = (torch.randn((rows, cols), generator=g, dtype=torch.float64) * 3).to(T)
+    x[1, : cols // 2] = -float("inf")
+    x[3, cols - 1] = float("nan")
+    x[4] = -float("inf")
+    x[5, cols - 1] = 40.0  # the maximum in the last (scalar) value
+    x64 = x.double()
+    e = torch.exp(x64 - x64.max(1, keepdim=True)[0])
+    s = e.sum(1, keepdim=True)
+    rel, floor = (1e-5, 1e-6) if dt == "float32" else (1e-12, 1e-15)
+    pn.set_stream(torch.cuda.current_stream().cuda_stream)
+    try:
+        for off_in, off_out, log in ((0, 0, False), (1, 0, True), (0, 3, False), (1, 1, True), (None, None, False)):
+            buf = torch.zeros(rows * cols + 8, dtype=T, device="cuda")
+            out = torch.full((rows * cols + 8,), 7.0, dtype=T, device="cuda")
+            if off_in is None:  # in place
+                off_in = off_out = 1
+                out = buf
+                buf[0] = buf[1 + rows * cols:] = 7.0
+            xi, yo = (b[o:o + rows * cols].view(rows, cols) for b, o in ((buf, off_in), (out, off_out)))
+            xi.copy_(x)
+            tx, ty = pn.Tensor.from_torch(xi), pn.Tensor.from_torch(yo)
+            f = pn.core._lib.neural_log_softmax if log else pn.core._lib.neural_softmax
+            assert f(ty._ptr, tx._ptr) == 0
+            got = yo.cpu().double()
+            want = (x64 - x64.max(1, keepdim=True)[0]) - torch.log(s) if log else e / s
+            assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+            fin = torch.isfinite(want)
+            bound = rel * want[fin].abs() + (floor if log or dt == "float64" else 0.0)
+            assert bool(((got[fin] - want[fin]).abs() <= bound).all()), (off_in, off_out, log)
+            edge = torch.cat([out[:off_out], out[off_out + rows * cols:]])
+            assert bool((edge == 7.0).all())  # nothing written outside the rows
+    finally:
+        pn.set_stream(None)
+
+
 def test_timed_launch(pn):
     """neural_hip_time_next_launch: the events ride on the chosen launch of the
     calling thread (elapsed time > 0, outputs unchanged), are used once, can
