@@ -12,9 +12,9 @@
 // target tensor's value, loss = mean_rows(-log(p_target + 1e-7)); f32 rows
 // keep the float roundings of e_j, of p_t and of each row's loss.
 //
-// One wave per row with the row in VGPRs (one HBM read; the gradient written
-// once), rows wider than the register budget take a block per row with three
-// passes.  Per-row losses land in a double buffer and are summed by the
+// A row sits in the VGPRs of 4 to 1024 lanes (one HBM read; the gradient
+// written once), at any width and alignment up to 98304 f32 / 49152 f64
+// classes; wider rows are read twice by a block of 1024.  Per-row losses land in a double buffer and are summed by the
 // segmented reduction (fixed order, deterministic); the row sums of exp use a
 // fixed wave tree instead of the reference's sequential order, so losses
 // agree to a few ulps of the row terms, not bit for bit.  An invalid target
@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "reduce_impl.hpp"
+#include "row_group.hpp"
 
 namespace nh {
 
@@ -92,41 +93,53 @@ struct CeArgs {
     int *bad;              // set to 1 when a target is out of range
 };
 
-// Per-element work once m and s are known.  Returns the element's part of the
-// row loss without the log term and without its weight (label-smoothed:
-// x - m) and writes the gradient element.  The row loss is
-// -sum_c st_c ((x_c - m) - lse) = lse * sum_c st_c - A with
+// The row loss is -sum_c st_c ((x_c - m) - lse) = lse * sum_c st_c - A with
 // A = sum_c st_c (x_c - m) = st0 * sum_c (x_c - m) + (st1 - st0) (x_t - m)
 // (st_c = st0 off the target, st1 on it): every term of the reference's sum
 // has one sign (x_c - m <= 0, lse >= 0), and so have the two parts of A, so
 // the regrouping changes only the last bits; the log moves out of the row
 // kernel into the summing pass and the weights out of the element loop.
-template <typename T, int MODE>
-NH_DEV double ce_elem(T xv, int64_t c, int64_t t, double m, double rs, const CeArgs &a, T &g)
-{
-    const double x = double(xv);
-    const double st = a.alpha / double(a.cols) + (c == t ? 1.0 - a.alpha : 0.0);
-    double term = 0.0;
-    if (MODE == CE_LS_FWD || MODE == CE_LS_FUSED) term = x - m;
-    if (MODE == CE_LS_BWD || MODE == CE_LS_FUSED) {
-        const double e = sizeof(T) == 8 ? row_exp_d(x, m) : row_exp_f(float(xv), m);
-        g = T(a.inv_n * (e * rs - st));
+
+// Gradient element from e = exp(x_c - m): (1/B) (e / sum - st_c).  WIDE f32
+// rows take it in double and round once; rows held by at most a wave in float.
+template <typename T, bool WIDE>
+struct CeGrad {
+    double rs, st0, st1, inv_n;
+    NH_DEV T operator()(T e, bool at_t) const
+    {
+        if constexpr (sizeof(T) == 4 && WIDE) {
+            asm("" : "+v"(e));  // or the compiler keeps double(e) of the sum: two more registers per value
+            return T(inv_n * (double(e) * rs - (at_t ? st1 : st0)));
+        } else if constexpr (sizeof(T) == 4) {
+            return float(inv_n) * (e * float(rs) - (at_t ? float(st1) : float(st0)));
+        } else {
+            return T(inv_n * (double(e) * rs - (at_t ? st1 : st0)));
+        }
     }
-    return term;
-}
+};
 
-template <typename T>
-NH_DEV double wave_fmax_t(T v);
-template <> NH_DEV double wave_fmax_t<float>(float v) { return double(wave_fmax(v)); }
-template <> NH_DEV double wave_fmax_t<double>(double v)
+// x_c - m as the row loss sums it.
+template <typename T, bool WIDE>
+NH_DEV double ce_diff(T x, double m)
 {
-    return Grp<64>::reduce(v, [](double a, double b) { return __builtin_fmax(a, b); });
+    if constexpr (sizeof(T) == 4 && !WIDE) return double(x - float(m));
+    else return double(x) - m;
 }
 
-// One wave per row, VPL 16-byte vectors per lane (<= 64 * VPL * VN values).
-// FULL: the row is exactly 64 * VPL * VN values and 16-byte aligned, so no
+// One row per group of NT lanes, VPT 16-byte vectors per lane and the values
+// before and after the vectors in one scalar of the first lanes (RowCut; the
+// other lanes' scalar is -inf and adds nothing).  FULL: the row is exactly NT * VPT vectors, so no
 // element needs a bounds check (per-element checks around the exp turn into
-// exec-mask branches).
+// exec-mask branches).  The lane that
+// holds the target picks x_t or e_t up as it passes; e_c replaces x_c.
+//
+// What bounds it: HBM where enough rows are in flight, so that one block loads
+// or stores while another computes.  A 201 KB row of 50257 f32 classes is 25
+// vectors for each of 512 lanes: 16 in registers and LV = 9 in LDS (72 KB; a
+// lane reads and writes its own slots only), two blocks per CU.  With all 25
+// in registers the compiler spilled 35-84 of them to scratch memory
+// ([4096, 50257] fused f32 373 us against 318; three passes of 4-byte
+// accesses took 861).
 //
 // WAVES: the minimum waves per SIMD the compiler must fit (1: its own
 // choice).  The f64 forward with rows of up to 1024 values takes 5 (83-84
@@ -134,173 +147,233 @@ template <> NH_DEV double wave_fmax_t<double>(double v)
 // [65536,1024] (A/B in one run).  The fused and backward forms keep every
 // exp for the gradient and spill under that bound (fused f64 180 -> 331 us),
 // as do rows of 2048 doubles.
-template <typename T, int VPL, int MODE, bool FULL, int WAVES = 1>
-__global__ __launch_bounds__(256, WAVES) void k_ce_wave(const T *__restrict__ x, CeArgs a, bool vec, int64_t r_base)
+template <typename T, int NT, int VPT, int LV, int MODE, bool FULL, int WAVES>
+__global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T *__restrict__ x, CeArgs a,
+                                                                       int64_t r_base)
 {
     using V = typename Vec16<T>::type;
+    using U = typename VecU<T>::type;
+    using G = RowGrp<NT>;
     constexpr int VN = Vec16<T>::n;
-    const int lane = threadIdx.x & 63;
+    constexpr int RPB = NT < 256 ? 256 / NT : 1;
+    constexpr bool WIDE = NT > 64;
+    constexpr bool LOSS = MODE == CE_LS_FWD || MODE == CE_LS_FUSED;
+    constexpr bool GRAD = MODE == CE_LS_BWD || MODE == CE_LS_FUSED;
     // The f64 forward takes exp_tab (2^(j/64) by the device library's exp2,
     // in LDS): 85-90 -> 84-87 us at [65536,1024] (A/B in one run).  The modes
     // that keep every e for the gradient keep the library's exp: with the
     // table their longer-lived registers made the fused pass 177 -> 182 us.
-    constexpr bool kTab = sizeof(T) == 8 && MODE == CE_LS_FWD;
+    constexpr bool kTab = sizeof(T) == 8 && MODE == CE_LS_FWD && !WIDE;
     __shared__ double etab[kTab ? 64 : 1];
+    __shared__ T lds_m[G::kWaves];
+    __shared__ double lds_s[G::kWaves], lds_a[G::kWaves];
+    __shared__ V more[LV > 0 ? LV : 1][LV > 0 ? NT : 1];
     if constexpr (kTab) {
         if (threadIdx.x < 64) etab[threadIdx.x] = exp2(double(threadIdx.x) * (1.0 / 64.0));
         __syncthreads();
     }
-    const int64_t r = r_base + int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (r >= a.rows) return;  // uniform per wave
+    const int lane = threadIdx.x % NT;
+    const int64_t r = r_base + int64_t(blockIdx.x) * RPB + threadIdx.x / NT;
+    if (RPB > 1 && r >= a.rows) return;  // uniform per group; a block of one row has one
     const int64_t cols = a.cols;
     const T *xr = x + r * cols;
+    T *gr = GRAD ? static_cast<T *>(a.grad) + r * cols : nullptr;
+    const RowCut<T, (NT >= 64)> cut(gr, cols);
+    const int nsc = FULL ? 0 : cut.nsc(), head = FULL ? 0 : cut.head;
+    const auto in_row = [&](int k) { return FULL || lane + k * NT < cut.ncv; };
     // the target first: its load overlaps the row's instead of following the reductions
     int64_t t = 0;
     const bool ok = loss_target(a.tidx, static_cast<const T *>(a.tval), r, cols, t);
-    V v[VPL];
+    V v[VPT], w[LV > 0 ? LV : 1];
+    T vt = -inf_t<T>();
+    const U *xv = reinterpret_cast<const U *>(xr + head);
 #pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int64_t c0 = (int64_t(k) * 64 + lane) * VN;
-        if (FULL || vec) {
-            if (FULL || c0 < cols) v[k] = ld_nt(reinterpret_cast<const V *>(xr + c0));
-        } else {
+    for (int k = 0; k < VPT; k++)
+        if (in_row(k)) v[k] = __builtin_nontemporal_load(xv + lane + k * NT);
 #pragma unroll
-            for (int j = 0; j < VN; j++)
-                if (FULL || c0 + j < cols) v[k][j] = xr[c0 + j];
+    for (int k = 0; k < LV; k++)
+        if (in_row(VPT + k)) w[k] = __builtin_nontemporal_load(xv + lane + (VPT + k) * NT);
+    if (lane < nsc) vt = xr[cut.sc(lane)];
+    // the target's vector and slot, or the scalar that holds it (-1: neither)
+    const bool t_vec = ok && t >= head && t - head < int64_t(FULL ? NT * VPT : cut.ncv) * VN;
+    const int tv = t_vec ? int((t - head) / VN) : -1, tj = int((t - head) % VN);
+    const bool t_mine = ok && !t_vec && lane < nsc && cut.sc(lane) == t;  // in this lane's scalar
+    const auto at = [&](const V &q) {  // q[tj]
+        T x = q[0];
+#pragma unroll
+        for (int j = 1; j < VN; j++) x = j == tj ? q[j] : x;
+        return x;
+    };
+    T mx = vt == vt ? vt : -inf_t<T>();
+#pragma unroll
+    for (int k = 0; k < VPT; k++)
+        if (in_row(k)) {
+#pragma unroll
+            for (int j = 0; j < VN; j++) mx = fmax_nn(mx, v[k][j]);
         }
-    }
-    T mx = -inf_t<T>();
 #pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int64_t c0 = (int64_t(k) * 64 + lane) * VN;
+    for (int k = 0; k < LV; k++)
+        if (in_row(VPT + k)) {
 #pragma unroll
-        for (int j = 0; j < VN; j++)
-            if (FULL || c0 + j < cols) mx = fmax_nn(mx, v[k][j]);
-    }
-    const double m = wave_fmax_t<T>(mx);
-    // e_c = exp(x_c - m), kept for the gradient (the backward modes)
-    constexpr bool KEEP = MODE == CE_LS_BWD || MODE == CE_LS_FUSED;
-    V ev[KEEP ? VPL : 1];
-    // Per-lane sums: double, except the f32 tensor loss, whose reference sums
-    // its float e_c in float (a lane's 16 float partial sums stay far inside
-    // that sum's own rounding); the wave sum is double either way.
-    using Acc = typename std::conditional<MODE == CE_ASM && sizeof(T) == 4, float, double>::type;
+            for (int j = 0; j < VN; j++) mx = fmax_nn(mx, w[k][j]);
+            more[k][lane] = w[k];
+        }
+    const double m = double(G::max(mx, lds_m));
+    const auto row_exp = [&](T xv) {
+        if constexpr (kTab) return exp_tab(double(xv) - m, etab);
+        else if constexpr (sizeof(T) == 8) return row_exp_d(double(xv), m);
+        else return row_exp_f(float(xv), m);
+    };
+    // Per-lane sums: double, except the f32 tensor loss of rows held by a
+    // wave, whose reference sums its float e_c in float (a lane's 64 float
+    // partial sums stay far inside that sum's own rounding); the group sum is
+    // double either way.
+    using Acc = typename std::conditional<MODE == CE_ASM && sizeof(T) == 4 && !WIDE, float, double>::type;
     Acc sl = Acc(0);
-    Acc et = Acc(0);  // CE_ASM: e at the target column, in the lane that holds it
+    double acc = 0.0;
+    double pick = 0.0;  // the lane that holds the target: x_t - m (the losses' A) or e_t (tensor CE)
+    bool mine = t_mine;
+    const auto sum_vec = [&](V &q, int k) {  // vector lane + k NT of the row
+        if (MODE != CE_LS_BWD && lane + k * NT == tv) {
+            const T x1 = at(q);
+            pick = MODE == CE_ASM ? row_exp(x1) : ce_diff<T, WIDE>(x1, m);
+            mine = true;
+        }
 #pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int64_t c0 = (int64_t(k) * 64 + lane) * VN;
+        for (int j = 0; j < VN; j++) {
+            const double e = row_exp(q[j]);
+            if constexpr (LOSS) acc += ce_diff<T, WIDE>(q[j], m);
+            if constexpr (GRAD) q[j] = T(e);
+            sl += Acc(e);
+        }
+    };
 #pragma unroll
-        for (int j = 0; j < VN; j++)
-            if (FULL || c0 + j < cols) {
-                const double e = kTab ? exp_tab(double(v[k][j]) - m, etab)
-                                      : (sizeof(T) == 8 ? row_exp_d(double(v[k][j]), m) : row_exp_f(float(v[k][j]), m));
-                if constexpr (KEEP) ev[k][j] = T(e);
-                if constexpr (MODE == CE_ASM) et = c0 + j == t ? Acc(e) : et;
-                sl += Acc(e);
-            }
+    for (int k = 0; k < VPT; k++)
+        if (in_row(k)) sum_vec(v[k], k);
+#pragma unroll 1
+    for (int k = 0; k < LV; k++)
+        if (in_row(VPT + k)) {
+            V q = more[k][lane];
+            sum_vec(q, VPT + k);
+            if constexpr (GRAD) more[k][lane] = q;
+        }
+    if (nsc) {  // uniform
+        const double e = row_exp(vt);
+        if (LOSS && lane < nsc) acc += ce_diff<T, WIDE>(vt, m);
+        if (t_mine) pick = MODE == CE_ASM ? e : ce_diff<T, WIDE>(vt, m);
+        if constexpr (GRAD) vt = T(e);
+        sl += Acc(e);
     }
-    double s = wave_dsum(double(sl));
+    const double s = G::sum(double(sl), lds_s);
     if (!ok) {
         if (lane == 0) {
             __hip_atomic_store(a.bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (a.row_loss) a.row_loss[r] = __builtin_nan("");
         }
-        return;
+        return;  // uniform per group
     }
-    if (MODE == CE_ASM) {
+    if constexpr (MODE == CE_ASM) {
         // p_t = e_t / sum (f32: e_t, sum and p_t rounded to float); the row's
         // loss -log(p_t + 1e-7) is taken in the summing pass (RedCeLoss), where
         // the double log runs on all lanes instead of on lane 0 of every row.
-        // e_t comes from the lane that computed it (the same value the
-        // reference's exp(x_t - m) gives), not from a second read of the row.
-        const int owner = int((t / VN) % 64);
-        const long long eb = __double_as_longlong(double(et));
-        const int lo = __builtin_amdgcn_readlane(int(eb), owner);
-        const int hi = __builtin_amdgcn_readlane(int(eb >> 32), owner);
-        const double e_t = __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-        if (lane == 0) a.row_loss[r] = sizeof(T) == 4 ? double(float(e_t) / float(s)) : e_t / s;
+        if (mine) a.row_loss[r] = sizeof(T) == 4 ? double(float(pick) / float(s)) : pick / s;
         return;
     }
-    const double rs = 1.0 / s;
     const double st0 = a.alpha / double(cols), st1 = st0 + (1.0 - a.alpha);
-    // f32 rows: the per-element terms in float (the gradient is a float and
-    // each loss term needs ~1e-7 of itself); the loss still sums in double
-    const float mf = float(m), rsf = float(rs), st0f = float(st0), st1f = float(st1), inf_ = float(a.inv_n);
-    double acc = 0.0;
-    T *gr = static_cast<T *>(a.grad) + r * cols;
+    if constexpr (GRAD) {
+        const CeGrad<T, WIDE> grad{1.0 / s, st0, st1, a.inv_n};
+        const auto store_vec = [&](const V &q, int k) {
+            V g;
 #pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int64_t c0 = (int64_t(k) * 64 + lane) * VN;
-        V g;
-#pragma unroll
-        for (int j = 0; j < VN; j++)
-            if (FULL || c0 + j < cols) {
-                const bool at_t = c0 + j == t;
-                if constexpr (sizeof(T) == 4) {
-                    if (MODE == CE_LS_FWD || MODE == CE_LS_FUSED) acc += double(v[k][j] - mf);
-                    if constexpr (KEEP) g[j] = inf_ * (ev[k][j] * rsf - (at_t ? st1f : st0f));
-                } else {
-                    if (MODE == CE_LS_FWD || MODE == CE_LS_FUSED) acc += double(v[k][j]) - m;
-                    if constexpr (KEEP) g[j] = T(a.inv_n * (double(ev[k][j]) * rs - (at_t ? st1 : st0)));
-                }
-            }
-        if (MODE == CE_LS_BWD || MODE == CE_LS_FUSED) {
-            if (FULL || vec) {
-                if (FULL || c0 < cols) st_nt(reinterpret_cast<V *>(gr + c0), g);
-            } else {
+            for (int j = 0; j < VN; j++) g[j] = grad(q[j], false);
+            if (lane + k * NT == tv) {
 #pragma unroll
                 for (int j = 0; j < VN; j++)
-                    if (FULL || c0 + j < cols) gr[c0 + j] = g[j];
+                    if (j == tj) g[j] = grad(q[j], true);
             }
-        }
+            __builtin_nontemporal_store(g, reinterpret_cast<U *>(gr + head) + lane + k * NT);
+        };
+#pragma unroll
+        for (int k = 0; k < VPT; k++)
+            if (in_row(k)) store_vec(v[k], k);
+#pragma unroll 3
+        for (int k = 0; k < LV; k++)
+            if (in_row(VPT + k)) store_vec(more[k][lane], VPT + k);
+        if (lane < nsc) gr[cut.sc(lane)] = grad(vt, t_mine);
     }
-    if (MODE == CE_LS_FWD || MODE == CE_LS_FUSED) {
-        acc = wave_dsum(acc);
-        // x_t from the registers of the lane that holds it: its vector k and
-        // slot j are the same for every lane, so the pick is a uniform select
-        const int kt = int(t / (64 * VN)), jt = int(t % VN), owner = int((t / VN) % 64);
-        T xl = T(0);
-#pragma unroll
-        for (int k = 0; k < VPL; k++)
-#pragma unroll
-            for (int j = 0; j < VN; j++)
-                if (k == kt && j == jt) xl = v[k][j];
-        double xv;
-        if constexpr (sizeof(T) == 4) {
-            xv = double(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(xl), owner)));
-        } else {
-            const long long xb = __double_as_longlong(double(xl));
-            const int lo = __builtin_amdgcn_readlane(int(xb), owner);
-            const int hi = __builtin_amdgcn_readlane(int(xb >> 32), owner);
-            xv = __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned int>(lo));
-        }
+    if constexpr (LOSS) {
+        acc = G::sum(st0 * acc + (mine ? (st1 - st0) * pick : 0.0), lds_a);
         if (lane == 0) {
-            const double xt = sizeof(T) == 4 ? double(float(xv) - mf) : xv - m;
-            a.row_loss[r] = st0 * acc + (st1 - st0) * xt;
+            a.row_loss[r] = acc;
             a.row_s[r] = s;
         }
     }
 }
 
-// Block per row (any width): max, sum of exp, then the outputs, each a pass
-// over the row.
+// Rows wider than a block's registers: 1024 lanes per row and two reads, the
+// first for the maximum and the sum of exp (a running maximum per lane, the
+// lane's sum rescaled in double when a batch of vectors raises it), the second
+// for the outputs.
+constexpr int kCeWide = 1024;
 template <typename T, int MODE>
-__global__ __launch_bounds__(256) void k_ce_block(const T *__restrict__ x, CeArgs a, int64_t r_base)
+__global__ __launch_bounds__(kCeWide) void k_ce_stream(const T *__restrict__ x, CeArgs a, int64_t r_base)
 {
-    using G = Grp<256>;
+    using V = typename Vec16<T>::type;
+    using U = typename VecU<T>::type;
+    using G = RowGrp<kCeWide>;
+    constexpr int VN = Vec16<T>::n, UN = 4;
+    constexpr bool LOSS = MODE == CE_LS_FWD || MODE == CE_LS_FUSED;
+    constexpr bool GRAD = MODE == CE_LS_BWD || MODE == CE_LS_FUSED;
+    __shared__ T lds_m[G::kWaves];
+    __shared__ double lds_s[G::kWaves], lds_a[G::kWaves];
     const int64_t r = r_base + blockIdx.x;
-    const int64_t cols = a.cols;
+    const int64_t cols = a.cols, ncv = cols / VN;
     const T *xr = x + r * cols;
-    T mx = -inf_t<T>();
-    for (int64_t c = threadIdx.x; c < cols; c += 256) mx = fmax_nn(mx, xr[c]);
-    const double m = double(G::reduce(mx, [](T p, T q) { return fmax_nn(p, q); }));
-    double s = 0.0;
-    for (int64_t c = threadIdx.x; c < cols; c += 256)
-        s += sizeof(T) == 8 ? row_exp_d(double(xr[c]), m) : row_exp_f(float(xr[c]), m);
-    s = G::reduce(s, [](double p, double q) { return p + q; });
+    const U *xv = reinterpret_cast<const U *>(xr);
     int64_t t = 0;
     const bool ok = loss_target(a.tidx, static_cast<const T *>(a.tval), r, cols, t);
+    const T xt = ok ? xr[t] : T(0);
+    const auto row_exp = [](T xv, double m) {
+        return sizeof(T) == 8 ? row_exp_d(double(xv), m) : row_exp_f(float(xv), m);
+    };
+    T mx = -inf_t<T>();
+    double s = 0.0, mr = 0.0;  // mr: what the sum's exponents are relative to (0 while only -inf was seen)
+    const auto rise = [&](T bm) {
+        if (bm > mx) {
+            if (s != 0.0) s *= exp(mr - double(bm));
+            mx = bm;
+            mr = double(bm);
+        }
+    };
+    for (int64_t c = threadIdx.x; c < ncv; c += UN * kCeWide) {
+        V v[UN];
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if (c + u * kCeWide < ncv) v[u] = xv[c + u * kCeWide];
+        T bm = -inf_t<T>();
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if (c + u * kCeWide < ncv) {
+#pragma unroll
+                for (int j = 0; j < VN; j++) bm = fmax_nn(bm, v[u][j]);
+            }
+        rise(bm);
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if (c + u * kCeWide < ncv) {
+#pragma unroll
+                for (int j = 0; j < VN; j++) s += row_exp(v[u][j], mr);
+            }
+    }
+    const int64_t jt = ncv * VN + threadIdx.x;  // at most VN - 1 values past the vectors
+    if (jt < cols) {
+        rise(xr[jt]);
+        s += row_exp(xr[jt], mr);
+    }
+    const double m = double(G::max(mx, lds_m));
+    // a row of only -inf is NaN, as exp(-inf - -inf) makes it
+    s = G::sum(s == 0.0 ? s : s * exp(mr - m), lds_s);
+    if (m == -__builtin_inf()) s = __builtin_nan("");
     if (!ok) {
         if (threadIdx.x == 0) {
             __hip_atomic_store(a.bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -308,59 +381,94 @@ __global__ __launch_bounds__(256) void k_ce_block(const T *__restrict__ x, CeArg
         }
         return;
     }
-    if (MODE == CE_ASM) {
-        if (threadIdx.x == 0) {
-            if (sizeof(T) == 4) a.row_loss[r] = double(float(row_exp_f(float(xr[t]), m)) / float(s));
-            else a.row_loss[r] = row_exp_d(double(xr[t]), m) / s;
-        }
+    if constexpr (MODE == CE_ASM) {
+        const double e_t = row_exp(xt, m);
+        if (threadIdx.x == 0) a.row_loss[r] = sizeof(T) == 4 ? double(float(e_t) / float(s)) : e_t / s;
         return;
     }
-    const double rs = 1.0 / s;
-    double acc = 0.0;
+    const double st0 = a.alpha / double(cols), st1 = st0 + (1.0 - a.alpha);
+    const CeGrad<T, true> grad{1.0 / s, st0, st1, a.inv_n};
     T *gr = static_cast<T *>(a.grad) + r * cols;
-    for (int64_t c = threadIdx.x; c < cols; c += 256) {
-        T g = T(0);
-        acc += ce_elem<T, MODE>(xr[c], c, t, m, rs, a, g);
-        if (MODE == CE_LS_BWD || MODE == CE_LS_FUSED) gr[c] = g;
+    double acc = 0.0;
+    const int64_t tv = t / VN;
+    const int tj = int(t % VN);
+    for (int64_t c = threadIdx.x; c < ncv; c += UN * kCeWide) {
+        V v[UN];
+#pragma unroll
+        for (int u = 0; u < UN; u++)
+            if (c + u * kCeWide < ncv) v[u] = xv[c + u * kCeWide];
+#pragma unroll
+        for (int u = 0; u < UN; u++) {
+            const int64_t i = c + u * kCeWide;
+            if (i < ncv) {
+                V g;
+#pragma unroll
+                for (int j = 0; j < VN; j++) {
+                    if constexpr (LOSS) acc += ce_diff<T, true>(v[u][j], m);
+                    if constexpr (GRAD) g[j] = grad(T(row_exp(v[u][j], m)), i == tv && j == tj);
+                }
+                if constexpr (GRAD) __builtin_nontemporal_store(g, reinterpret_cast<U *>(gr) + i);
+            }
+        }
     }
-    if (MODE == CE_LS_FWD || MODE == CE_LS_FUSED) {
-        acc = G::reduce(acc, [](double p, double q) { return p + q; });
+    if (jt < cols) {
+        const T xj = xr[jt];
+        if constexpr (LOSS) acc += ce_diff<T, true>(xj, m);
+        if constexpr (GRAD) gr[jt] = grad(T(row_exp(xj, m)), jt == t);
+    }
+    if constexpr (LOSS) {
+        acc = G::sum(acc, lds_a);
         if (threadIdx.x == 0) {
-            const double st0 = a.alpha / double(cols), st1 = st0 + (1.0 - a.alpha);
-            const double xt = double(xr[t]) - m;  // as ce_elem forms the other terms
-            a.row_loss[r] = st0 * acc + (st1 - st0) * xt;
+            a.row_loss[r] = st0 * acc + (st1 - st0) * ce_diff<T, true>(xt, m);
             a.row_s[r] = s;
         }
     }
 }
 
-template <typename T, int MODE, int VPL>
-static void launch_ce_wave(const T *x, const CeArgs &a, bool vec)
+template <typename T, int MODE, int NT, int VPT, int LV = 0>
+static void launch_ce_rows(const T *x, const CeArgs &a)
 {
-    constexpr int W = sizeof(T) == 8 && MODE == CE_LS_FWD && VPL <= 8 ? 5 : 1;
-    for_row_launches(a.rows, 4, [&](unsigned g, int64_t base) {
-        if (vec && a.cols == int64_t(64) * VPL * Vec16<T>::n)
-            NH_LAUNCH((k_ce_wave<T, VPL, MODE, true, W>), dim3(g), dim3(256), 0, stream(), x, a, vec, base);
-        else
-            NH_LAUNCH((k_ce_wave<T, VPL, MODE, false, W>), dim3(g), dim3(256), 0, stream(), x, a, vec, base);
+    constexpr int W = NT == 512 ? 4 : (NT <= 64 && sizeof(T) == 8 && MODE == CE_LS_FWD && VPT <= 8 ? 5 : 1);
+    constexpr int block = NT < 256 ? 256 : NT;
+    for_row_launches(a.rows, block / NT, [&](unsigned g, int64_t base) {
+        if constexpr (NT <= 64) {
+            if (a.cols == int64_t(NT) * VPT * Vec16<T>::n) {
+                constexpr unsigned lds = sizeof(T) == 4 && VPT >= 4 ? kFullRowsLds : 0;
+                NH_LAUNCH((k_ce_rows<T, NT, VPT, LV, MODE, true, W>), dim3(g), dim3(block), lds, stream(), x, a, base);
+                return;
+            }
+        }
+        NH_LAUNCH((k_ce_rows<T, NT, VPT, LV, MODE, false, W>), dim3(g), dim3(block), 0, stream(), x, a, base);
     });
 }
 
+// The smallest group whose registers hold the row (as launch_softmax).  Before
+// (a wave per row up to 4096 f32 / 2048 f64 values, element by element where
+// the width was no multiple of the vector, then three passes) -> now, us,
+// smoothed fused form with its summing launches:
+//   f32 [65536, 10] 32.1 -> 10.7, [32768, 256] 24.3 -> 19.2, [30000, 1001] 84.3 -> 49.0, [65536, 1024] 93.2 -> 89.9
+//       [8192, 3000] 107 -> 43.5, [4096, 8192] 115 -> 52.4, [2048, 32000] 267 -> 104, [4096, 50257] 861 -> 317
+//       [600, 98000] 517 -> 110, [500, 131072] 682 -> 134 (two reads)
+//   f64 [65536, 10] 33.7 -> 14.3, [30000, 1001] 104 -> 92, [4096, 8553] 203 -> 110, [2000, 24001] 332 -> 167
 template <typename T, int MODE>
 static int launch_ce(const T *x, const CeArgs &a)
 {
-    constexpr int VN = Vec16<T>::n;
-    const bool vec = (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && a.cols % VN == 0 &&
-                     (!a.grad || (reinterpret_cast<uintptr_t>(a.grad) & 15u) == 0);
-    const int64_t per = ceil_div(a.cols, int64_t(64) * VN);  // vectors per lane
-    if (per <= 1) launch_ce_wave<T, MODE, 1>(x, a, vec);
-    else if (per <= 2) launch_ce_wave<T, MODE, 2>(x, a, vec);
-    else if (per <= 4) launch_ce_wave<T, MODE, 4>(x, a, vec);
-    else if (per <= 8) launch_ce_wave<T, MODE, 8>(x, a, vec);
-    else if (per <= 16) launch_ce_wave<T, MODE, 16>(x, a, vec);
+    const int64_t ncv = a.cols / Vec16<T>::n;
+    if (ncv <= 4) launch_ce_rows<T, MODE, 4, 1>(x, a);
+    else if (ncv <= 16) launch_ce_rows<T, MODE, 16, 1>(x, a);
+    else if (ncv <= 16 * 4) launch_ce_rows<T, MODE, 16, 4>(x, a);
+    else if (ncv <= 64 * 2) launch_ce_rows<T, MODE, 64, 2>(x, a);
+    else if (ncv <= 64 * 4) launch_ce_rows<T, MODE, 64, 4>(x, a);
+    else if (ncv <= 64 * 8) launch_ce_rows<T, MODE, 64, 8>(x, a);
+    else if (ncv <= 64 * 16) launch_ce_rows<T, MODE, 64, 16>(x, a);
+    else if (ncv <= 256 * 8) launch_ce_rows<T, MODE, 256, 8>(x, a);
+    else if (ncv <= 256 * 16) launch_ce_rows<T, MODE, 256, 16>(x, a);
+    else if (ncv <= 512 * 16) launch_ce_rows<T, MODE, 512, 16>(x, a);
+    else if (ncv <= 512 * 25) launch_ce_rows<T, MODE, 512, 16, 9>(x, a);
+    else if (ncv <= 1024 * 24) launch_ce_rows<T, MODE, 1024, 24>(x, a);
     else
         for_row_launches(a.rows, 1, [&](unsigned g, int64_t base) {
-            NH_LAUNCH((k_ce_block<T, MODE>), dim3(g), dim3(256), 0, stream(), x, a, base);
+            NH_LAUNCH((k_ce_stream<T, MODE>), dim3(g), dim3(kCeWide), 0, stream(), x, a, base);
         });
     return check_launch();
 }

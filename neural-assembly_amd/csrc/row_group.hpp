@@ -1,0 +1,93 @@
+// row_group.hpp -- reductions over the lanes that share one row, for the kernels
+// that hold a row in registers (softmax, cross-entropy).
+#pragma once
+
+#include "common.hpp"
+
+namespace nh {
+
+// Group-wide max (NaN-ignoring) and sum over the NT lanes that share a row:
+// 4, 16 or 32 lanes of a wave (DPP moves, and one swizzle across 16), one wave,
+// or a block of NT lanes through LDS.
+template <int NT>
+struct RowGrp {
+    static constexpr int kWaves = NT < 64 ? 1 : NT / 64;
+    template <typename T> NH_DEV static T dpp(T v, int step)
+    {
+        if constexpr (sizeof(T) == 4)
+            return step == 0 ? dpp_f<kDppXor1>(v) : step == 1 ? dpp_f<kDppXor2>(v)
+                 : step == 2 ? dpp_f<kDppHalfMirror>(v) : dpp_f<kDppMirror>(v);
+        else
+            return step == 0 ? dpp_d<kDppXor1>(v) : step == 1 ? dpp_d<kDppXor2>(v)
+                 : step == 2 ? dpp_d<kDppHalfMirror>(v) : dpp_d<kDppMirror>(v);
+    }
+    template <typename T, typename C>
+    NH_DEV static T part(T v, C comb)
+    {
+#pragma unroll
+        for (int i = 0; i < (NT == 4 ? 2 : 4); i++) v = comb(v, dpp(v, i));
+        return NT == 32 ? comb(v, __shfl_xor(v, 16, 64)) : v;
+    }
+    template <typename T, typename C>
+    NH_DEV static T across(T w, T *lds, C comb)
+    {
+        if constexpr (kWaves == 1) {
+            return w;
+        } else {
+            if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = w;
+            __syncthreads();
+            T r = lds[0];
+#pragma unroll
+            for (int i = 1; i < kWaves; i++) r = comb(r, lds[i]);
+            return r;
+        }
+    }
+    NH_DEV static float max(float v, float *lds)
+    {
+        if constexpr (NT < 64) return part(v, [](float a, float b) { return __builtin_fmaxf(a, b); });
+        else return across(wave_fmax(v), lds, [](float a, float b) { return __builtin_fmaxf(a, b); });
+    }
+    NH_DEV static double max(double v, double *lds)
+    {
+        if constexpr (NT < 64) return part(v, [](double a, double b) { return __builtin_fmax(a, b); });
+        else return across(wave_max_ignore_nan(v), lds, [](double a, double b) { return __builtin_fmax(a, b); });
+    }
+    NH_DEV static double sum(double v, double *lds)
+    {
+        if constexpr (NT < 64) return part(v, [](double a, double b) { return a + b; });
+        else return across(wave_dsum(v), lds, [](double a, double b) { return a + b; });
+    }
+};
+
+// Unused dynamic LDS that the check-free f32 wave kernels (4 or more vectors
+// per lane) are launched with: it holds residency to 4 blocks of 4 rows per CU.
+// Fewer rows in flight suit the memory here: [65536, 1024] softmax 85.6 us
+// with 8 blocks, 84.2 with 6, 81.9 with 4, 83.8 with 3; fused cross-entropy
+// 95.0 / 93.9 / 89.9 / 91.6 us.
+constexpr unsigned kFullRowsLds = 40000;
+
+// How a row of `cols` values is cut for a group of NT lanes: `head` values up to
+// the first 64-byte boundary of the row that is written, ncv vectors, `rem`
+// values past them; lane l < nsc() holds value sc(l) as a scalar.  Vector
+// stores that start inside a 64-byte block ran 12% slower (64 M f32 copy, 99.7
+// against 88 us whatever the offset inside the block; loads do not mind).
+// HEAD = false (groups without lanes or work to spare): head = 0.
+template <typename T, bool HEAD>
+struct RowCut {
+    static constexpr int VN = Vec16<T>::n;
+    int head, ncv, rem;
+    NH_DEV RowCut(const void *written, int64_t cols)
+    {
+        head = 0;
+        if constexpr (HEAD) {
+            const int h = int((64 - (reinterpret_cast<uintptr_t>(written) & 63)) & 63) / int(sizeof(T));
+            head = h < cols ? h : int(cols);
+        }
+        ncv = int((cols - head) / VN);
+        rem = int((cols - head) % VN);
+    }
+    NH_DEV int nsc() const { return head + rem; }
+    NH_DEV int64_t sc(int lane) const { return lane < head ? lane : int64_t(ncv) * VN + lane; }
+};
+
+}  // namespace nh

@@ -21,12 +21,12 @@
 // 2048 f64 values, a block of 256 to 1024 lanes beyond, up to 98304 / 49152
 // values -- so it is read once and written once at any width and alignment:
 // 16-byte accesses at the element's own alignment and one scalar per lane for
-// the last cols % VN values.  Wider rows are read twice.
+// the values at the row's ends.  Wider rows are read twice.
 #include <cmath>
 
 #include <hip/hip_ext.h>
 
-#include "common.hpp"
+#include "row_group.hpp"
 
 namespace nh {
 
@@ -42,59 +42,6 @@ template <> NH_DEV double neg_inf<double>() { return -__builtin_inf(); }
 // against (float)exp((double)x - (double)m) for any spread of the row.  A NaN
 // passes through and makes the row's sum NaN, as in the reference.
 NH_DEV float exp_diff_f32(float x, double md) { return exp_d2f(double(x) - md); }
-
-// Group-wide max (NaN-ignoring) and sum over the NT lanes that share a row:
-// 4, 16 or 32 lanes of a wave (DPP moves, and one swizzle across 16), one wave,
-// or a block of NT lanes through LDS.
-template <int NT>
-struct RowGrp {
-    static constexpr int kWaves = NT < 64 ? 1 : NT / 64;
-    template <typename T> NH_DEV static T dpp(T v, int step)
-    {
-        if constexpr (sizeof(T) == 4)
-            return step == 0 ? dpp_f<kDppXor1>(v) : step == 1 ? dpp_f<kDppXor2>(v)
-                 : step == 2 ? dpp_f<kDppHalfMirror>(v) : dpp_f<kDppMirror>(v);
-        else
-            return step == 0 ? dpp_d<kDppXor1>(v) : step == 1 ? dpp_d<kDppXor2>(v)
-                 : step == 2 ? dpp_d<kDppHalfMirror>(v) : dpp_d<kDppMirror>(v);
-    }
-    template <typename T, typename C>
-    NH_DEV static T part(T v, C comb)
-    {
-#pragma unroll
-        for (int i = 0; i < (NT == 4 ? 2 : 4); i++) v = comb(v, dpp(v, i));
-        return NT == 32 ? comb(v, __shfl_xor(v, 16, 64)) : v;
-    }
-    template <typename T, typename C>
-    NH_DEV static T across(T w, T *lds, C comb)
-    {
-        if constexpr (kWaves == 1) {
-            return w;
-        } else {
-            if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = w;
-            __syncthreads();
-            T r = lds[0];
-#pragma unroll
-            for (int i = 1; i < kWaves; i++) r = comb(r, lds[i]);
-            return r;
-        }
-    }
-    NH_DEV static float max(float v, float *lds)
-    {
-        if constexpr (NT < 64) return part(v, [](float a, float b) { return __builtin_fmaxf(a, b); });
-        else return across(wave_fmax(v), lds, [](float a, float b) { return __builtin_fmaxf(a, b); });
-    }
-    NH_DEV static double max(double v, double *lds)
-    {
-        if constexpr (NT < 64) return part(v, [](double a, double b) { return __builtin_fmax(a, b); });
-        else return across(wave_max_ignore_nan(v), lds, [](double a, double b) { return __builtin_fmax(a, b); });
-    }
-    NH_DEV static double sum(double v, double *lds)
-    {
-        if constexpr (NT < 64) return part(v, [](double a, double b) { return a + b; });
-        else return across(wave_dsum(v), lds, [](double a, double b) { return a + b; });
-    }
-};
 
 NH_DEV float row_exp(float x, double m) { return exp_diff_f32(x, m); }
 NH_DEV double row_exp(double x, double m) { return exp(x - m); }
@@ -113,9 +60,10 @@ NH_DEV T row_out(T v, double md, double lse, double s, double rs)
     else return v / s;
 }
 
-// One row per group of NT lanes, held in VPT vectors per lane (and the last
-// cols % VN values in one scalar of lanes 0 .. rem - 1, whose other lanes hold
-// -inf: it adds 0 to the sum, or NaN where the row is NaN anyway).  FULL: the
+// One row per group of NT lanes, held in VPT vectors per lane (and the values
+// before and after the vectors in one scalar of the first lanes, see RowCut;
+// the other lanes' scalar is -inf, which adds 0 to the sum, or NaN where the
+// row is NaN anyway).  FULL: the
 // row is exactly NT * VPT vectors, so no element needs a bounds check.
 //
 // What bounds it: HBM, one read and one write, while the rows in flight per
@@ -139,14 +87,15 @@ __global__ __launch_bounds__(NT < kSmBlock ? kSmBlock : NT, NT == 512 ? 4 : 1) v
     if (RPB > 1 && r >= rows) return;  // uniform per group; a block of one row has one
     const T *xr = x + r * cols;
     T *yr = y + r * cols;
-    const int ncv = int(cols / VN), rem = FULL ? 0 : int(cols % VN);
-    const auto in_row = [&](int k) { return FULL || lane + k * NT < ncv; };
+    const RowCut<T, (NT >= 256)> cut(yr, cols);  // in a wave the head costs what it saves: [55392, 577] 45.0 -> 46.7 us
+    const int nsc = FULL ? 0 : cut.nsc(), head = FULL ? 0 : cut.head;
+    const auto in_row = [&](int k) { return FULL || lane + k * NT < cut.ncv; };
     V v[VPT];
     T vt = neg_inf<T>();
 #pragma unroll
     for (int k = 0; k < VPT; k++)
-        if (in_row(k)) v[k] = __builtin_nontemporal_load(reinterpret_cast<const U *>(xr) + lane + k * NT);
-    if (rem && lane < rem) vt = xr[int64_t(ncv) * VN + lane];
+        if (in_row(k)) v[k] = __builtin_nontemporal_load(reinterpret_cast<const U *>(xr + head) + lane + k * NT);
+    if (lane < nsc) vt = xr[cut.sc(lane)];
 
     T m = vt == vt ? vt : neg_inf<T>();
 #pragma unroll
@@ -173,7 +122,7 @@ __global__ __launch_bounds__(NT < kSmBlock ? kSmBlock : NT, NT == 512 ? 4 : 1) v
             }
         }
     }
-    if (rem) {  // uniform
+    if (nsc) {  // uniform
         const T e = row_exp(vt, md);
         if (!LOG) vt = e;
         s += double(e);
@@ -181,7 +130,7 @@ __global__ __launch_bounds__(NT < kSmBlock ? kSmBlock : NT, NT == 512 ? 4 : 1) v
     s = G::sum(s, lds_s);
     double lse = 0.0;  // s >= 1: the maximum contributes 1
     if constexpr (LOG && sizeof(T) == 4) lse = log_ge1(s);
-    else if constexpr (LOG) lse = NT <= 64 && rem == 0 ? log_ge1(s) : log(s);
+    else if constexpr (LOG) lse = NT <= 64 && cols % VN == 0 ? log_ge1(s) : log(s);
     const double rs = LOG ? 0.0 : 1.0 / s;
 #pragma unroll
     for (int k = 0; k < VPT; k++) {
@@ -189,10 +138,10 @@ __global__ __launch_bounds__(NT < kSmBlock ? kSmBlock : NT, NT == 512 ? 4 : 1) v
             V o;
 #pragma unroll
             for (int j = 0; j < VN; j++) o[j] = row_out<T, LOG>(v[k][j], md, lse, s, rs);
-            __builtin_nontemporal_store(o, reinterpret_cast<U *>(yr) + lane + k * NT);
+            __builtin_nontemporal_store(o, reinterpret_cast<U *>(yr + head) + lane + k * NT);
         }
     }
-    if (rem && lane < rem) yr[int64_t(ncv) * VN + lane] = row_out<T, LOG>(vt, md, lse, s, rs);
+    if (lane < nsc) yr[cut.sc(lane)] = row_out<T, LOG>(vt, md, lse, s, rs);
 }
 
 // Rows wider than the registers of a block: one 1024-lane block per row, two
@@ -281,8 +230,8 @@ static void launch_rows(const T *x, T *y, int64_t rows, int64_t cols)
         constexpr int block = NT < kSmBlock ? kSmBlock : NT;
         if constexpr (NT <= 64 && sizeof(T) == 4) {
             if (cols == int64_t(NT) * VPT * Vec16<T>::n) {
-                NH_LAUNCH((k_softmax_rows<T, LOG, NT, VPT, true>), dim3(g), dim3(block), 0, stream(), x, y, rows,
-                          cols, base);
+                NH_LAUNCH((k_softmax_rows<T, LOG, NT, VPT, true>), dim3(g), dim3(block), VPT >= 4 ? kFullRowsLds : 0,
+                          stream(), x, y, rows, cols, base);
                 return;
             }
         }

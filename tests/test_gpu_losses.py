@@ -288,3 +288,93 @@ def test_ls_ce_loss_left_in_device_memory(pn, k):
     assert lib.label_smoothing_ce_forward_dev(xt.data_ptr(), tt.data_ptr(), b, k, 1.5, p) == -1
     pn.synchronize()
     assert math.isnan(losses[0].item()) and losses[3].item() == 7.0  # untouched by the refused calls
+
+
+# Class counts at the edges of the row kernels (4 or 16 lanes per row up to 259
+# f32 values; 2 .. 16 vectors per lane in a wave, 8 / 16 in a block of 256, 16
+# and 16 + 9 (the 9 in LDS) in 512, 24 in 1024, two reads beyond); f64 at half.
+_EDGES = [1, 2, 3, 15, 16, 19, 20, 64, 67, 68, 256, 259, 260, 511, 513, 1023, 1025, 2049, 4096, 4099, 4101, 8193, 16385,
+          32768, 32785, 49153, 51200, 51217, 98304, 98321, 120001]
+
+
+@pytest.mark.parametrize("k", _EDGES)
+@pytest.mark.parametrize("dt", ["float32", "float64"])
+def test_row_kernel_edges(pn, dt, k):
+    """Fused, backward and forward smoothed CE and the tensor CE at each row
+    kernel's edges against the float64 formula, at several element offsets of
+    logits and gradient, the target in the first, last and inner values, -inf
+    logits, a NaN row and a row of only -inf.  Bounds: those of the module."""
+    import torch
+    lib = pn.core._lib
+    T = getattr(torch, dt)
+    k = k if dt == "float32" else max(1, (k + 1) // 2)
+    b = 9
+    rng = np.random.default_rng(k)
+    x = rng.normal(0, 3, (b, k)).astype(dt)
+    t = rng.integers(0, k, b)
+    t[:4] = [0, k - 1, max(0, k - 2), min(k - 1, 17)]
+    if k > 4:
+        x[5, : k // 2] = -np.inf
+        t[5] = k - 1
+    special = [5, 6, 7]  # the loss of these rows is not finite
+    x[6, k // 2] = np.nan
+    x[7] = -np.inf
+    fine = [r for r in range(b) if r not in special]
+    x64, a = x.astype(np.float64), 0.1
+    f64 = dt == "float64"
+    pn.set_stream(torch.cuda.current_stream().cuda_stream)
+    try:
+        for rows, oi, og in ((fine, 0, 0), (fine, 1, 3), (fine, 3, 0), (list(range(b)), 1, 1)):
+            n = len(rows)
+            bx, bg = (torch.full((n * k + 8,), 7.0, dtype=T, device="cuda") for _ in range(2))
+            X, G = bx[oi:oi + n * k].view(n, k), bg[og:og + n * k].view(n, k)
+            X.copy_(torch.from_numpy(x[rows]))
+            tt = torch.from_numpy(t[rows]).cuda()
+            loss = torch.zeros((), dtype=torch.float64, device="cuda")
+            args = (X.data_ptr(), tt.data_ptr(), n, k, a)
+            fn = lib.label_smoothing_ce_fused_dev if f64 else lib.label_smoothing_ce_fused_f32_dev
+            assert fn(*args, loss.data_ptr(), G.data_ptr()) == 0
+            xr = x64[rows]
+            with np.errstate(all="ignore"):
+                d = xr - np.max(np.where(np.isnan(xr), -np.inf, xr), axis=1, keepdims=True)
+                e = np.exp(d)
+                s = e.sum(axis=1, keepdims=True)
+                st = np.full((n, k), a / k)
+                st[np.arange(n), t[rows]] += 1 - a
+                want = (e / s - st) / n
+                want_loss = -(st * (d - np.log(s))).sum() / n
+            got = G.cpu().numpy().astype(np.float64)
+            assert np.array_equal(np.isnan(got), np.isnan(want))
+            ok = ~np.isnan(want)
+            bound = 1e-12 * np.abs(want[ok]) + 2e-15 / n if f64 else 1e-5 * np.abs(want[ok]) + 2e-7 / n
+            assert np.all(np.abs(got[ok] - want[ok]) <= bound), (oi, og)
+            if np.isfinite(want_loss):
+                scale = _bound(xr, t[rows], a)
+                assert abs(loss.item() - want_loss) <= (1e-12 if f64 else 2e-6) * scale
+            else:
+                assert not np.isfinite(loss.item())
+            edge = torch.cat([bg[:og], bg[og + n * k:]])
+            assert bool((edge == 7.0).all())  # nothing written outside the rows
+            if f64:
+                fused = G.clone()
+                G.fill_(0.0)
+                assert lib.label_smoothing_ce_backward(*args, G.data_ptr()) == 0
+                assert torch.equal(fused.view(torch.int64), G.view(torch.int64))
+                fwd = torch.zeros((), dtype=torch.float64, device="cuda")
+                assert lib.label_smoothing_ce_forward_dev(*args, fwd.data_ptr()) == 0
+                if np.isfinite(want_loss):
+                    assert abs(fwd.item() - want_loss) <= 1e-12 * scale
+            if rows is fine:
+                got_ce = ctypes.c_double()
+                tx, tv = pn.Tensor.from_torch(X), pn.Tensor.from_torch(tt.to(T))
+                assert lib.neural_cross_entropy_loss(tx._ptr, tv._ptr, ctypes.byref(got_ce)) == 0
+                want_ce = np.mean(-np.log((e / s)[np.arange(n), t[rows]] + 1e-7))
+                assert abs(got_ce.value - want_ce) <= (1e-12 * abs(want_ce) + 1e-15 if f64
+                                                       else 2e-6 * abs(want_ce) + 2e-7)
+        # a target outside [0, k): NaN loss, the other rows' gradients written
+        tt[1] = k
+        G.fill_(7.0)
+        assert fn(*args, loss.data_ptr(), G.data_ptr()) == 0
+        assert np.isnan(loss.item()) and bool((G[1] == 7.0).all()) and not bool((G[0] == 7.0).any())
+    finally:
+        pn.set_stream(None)
