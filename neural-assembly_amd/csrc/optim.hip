@@ -3,8 +3,9 @@
 // Reference: optimizers_c.c:64-562.  The handle keeps the hyper-parameters,
 // the step count and per-parameter float64 moment buffers that are allocated
 // (zeroed) on the first step and sized by numel(param).  Here the buffers
-// live in HBM and each step is one fused kernel per parameter tensor that
-// reads param, grad, m, v once and writes param, m, v once.
+// live in HBM and each step is one fused launch for up to kStepTab parameter
+// tensors of a dtype, which reads param, grad, m, v once and writes param, m, v
+// once.
 //
 // Per-element arithmetic is the reference's, in double, in the same order,
 // without FMA contraction; the bias corrections bc1 = 1 - pow(beta1, t),
@@ -14,8 +15,9 @@
 //
 // OPTS state blob (optimizers_c.c:84-100,391-562): 80-byte header, then
 // int64 sizes, then f64 velocities (SGD) or all m followed by all v.
-#include <cmath>
+#include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdlib>
 #include <new>
 #include <vector>
@@ -127,114 +129,188 @@ NH_DEV double adam_f64(double pd, double gd, double &m, double &v, const AdamArg
 
 constexpr int kOBlock = 256;
 
-// One element per lane and one 256-lane tile per block (the grid covers the
-// whole tensor; the loop only runs for tensors beyond 2^32 elements).
-// Measured on 100 M f32 params with f64 moments: 698 us (79 % of HBM) here,
-// against 825 us for a grid of 16 blocks per CU striding over tiles of
-// 2-element vectors, and 710-725 us for 2 or 4 elements in flight per lane.
-template <bool W>
-__global__ __launch_bounds__(kOBlock) void k_adam_f32(float *__restrict__ p, const float *__restrict__ g,
-                                                      double *__restrict__ m, double *__restrict__ v, int64_t n,
-                                                      AdamArgs a)
+// The tensors of one launch, in its kernel arguments (no upload, nothing kept
+// between calls): 44 bytes per tensor within the 4 KiB of arguments.
+struct StepEntry {
+    void *p;
+    const void *g;
+    double *m, *v;  // SGD: m holds the velocity
+    int64_t n;
+};
+constexpr int kStepTab = 88;
+struct StepTab {
+    StepEntry e[kStepTab];
+    int32_t first[kStepTab];  // first block of each tensor
+    int32_t count;
+    int32_t tiles;            // 256-element tiles per block
+};
+static_assert(sizeof(StepTab) + sizeof(AdamArgs) + 64 <= 4096, "kernel arguments");
+
+// One element per lane, `tiles` 256-lane tiles per block (1 unless the grid
+// would pass kMaxGridBlocks); a block finds its tensor with one compare of its
+// index per lane and two ballots.
+// Bound by HBM, 44 B per element (f32 Adam).  A launch per tensor let the chip
+// drain and refill between tensors: norm pass and step over 85 M values in 144
+// tensors 1072 -> 718 us (70 of them the norm), 1.2 M values in 288 tensors
+// 1033 -> 90 us, 50 M in 12 413 -> 389 us; large tensors gain little.
+// Measured at 100 M f32 params with f64 moments, one tensor: 698 us with one
+// element per lane, 710-725 us for 2 or 4 in flight per lane, 825 us for a grid
+// of 16 blocks per CU striding over the tensor.
+template <typename T, int TYPE>
+__global__ __launch_bounds__(kOBlock) void k_opt_step(const StepTab tab, AdamArgs a)
 {
-    const int64_t stride = int64_t(gridDim.x) * kOBlock;
-    for (int64_t j = int64_t(blockIdx.x) * kOBlock + threadIdx.x; j < n; j += stride) {
-        const float pd = ld_nt(p + j), gd = ld_nt(g + j);
-        double mm = ld_nt(m + j), vq = ld_nt(v + j);
-        const float r = W ? adamw_f32(pd, gd, mm, vq, a) : adam_f32(pd, gd, mm, vq, a);
-        st_nt(p + j, r);
-        st_nt(m + j, mm);
-        st_nt(v + j, vq);
+    const int b = int(blockIdx.x);
+    int i = 0;
+    if (tab.count > 1) {
+        const int lane = int(threadIdx.x & 63);
+        static_assert(kStepTab <= 128, "two ballots");
+        const bool c0 = lane < tab.count && tab.first[lane] <= b;
+        const bool c1 = lane + 64 < tab.count && tab.first[lane + 64 < kStepTab ? lane + 64 : 0] <= b;
+        i = __builtin_amdgcn_readfirstlane(int(__popcll(__ballot(c0)) + __popcll(__ballot(c1))) - 1);
+    }
+    const StepEntry &e = tab.e[i];
+    T *__restrict__ p = static_cast<T *>(e.p);
+    const T *__restrict__ g = static_cast<const T *>(e.g);
+    const int64_t j0 = int64_t(b - tab.first[i]) * tab.tiles * kOBlock + threadIdx.x;
+    for (int k = 0; k < tab.tiles; k++) {
+        const int64_t j = j0 + int64_t(k) * kOBlock;
+        if (j >= e.n) return;
+        if constexpr (TYPE == OPT_SGD) {  // sgd_step_impl (optimizers_c.c:218-249)
+            const double nv = a.b1 * ld_nt(e.m + j) + double(ld_nt(g + j));
+            st_nt(e.m + j, nv);
+            st_nt(p + j, ld_nt(p + j) - T(a.lr * nv));
+        } else {
+            const T pd = ld_nt(p + j), gd = ld_nt(g + j);
+            double mm = ld_nt(e.m + j), vq = ld_nt(e.v + j);
+            T r;
+            if constexpr (sizeof(T) == 4) r = TYPE == OPT_ADAMW ? adamw_f32(pd, gd, mm, vq, a) : adam_f32(pd, gd, mm, vq, a);
+            else r = TYPE == OPT_ADAMW ? adamw_f64(pd, gd, mm, vq, a) : adam_f64(pd, gd, mm, vq, a);
+            st_nt(p + j, r);
+            st_nt(e.m + j, mm);
+            st_nt(e.v + j, vq);
+        }
     }
 }
 
-template <bool W>
-__global__ __launch_bounds__(kOBlock) void k_adam_f64(double *__restrict__ p, const double *__restrict__ g,
-                                                      double *__restrict__ m, double *__restrict__ v, int64_t n,
-                                                      AdamArgs a)
+template <typename T>
+static int launch_step(int type, const StepTab &tab, unsigned blocks, const AdamArgs &a)
 {
-    const int64_t stride = int64_t(gridDim.x) * kOBlock;
-    for (int64_t j = int64_t(blockIdx.x) * kOBlock + threadIdx.x; j < n; j += stride) {
-        const double pd = ld_nt(p + j), gd = ld_nt(g + j);
-        double mm = ld_nt(m + j), vq = ld_nt(v + j);
-        const double r = W ? adamw_f64(pd, gd, mm, vq, a) : adam_f64(pd, gd, mm, vq, a);
-        st_nt(p + j, r);
-        st_nt(m + j, mm);
-        st_nt(v + j, vq);
+    if (type == OPT_SGD) NH_LAUNCH((k_opt_step<T, OPT_SGD>), dim3(blocks), dim3(kOBlock), 0, stream(), tab, a);
+    else if (type == OPT_ADAM) NH_LAUNCH((k_opt_step<T, OPT_ADAM>), dim3(blocks), dim3(kOBlock), 0, stream(), tab, a);
+    else NH_LAUNCH((k_opt_step<T, OPT_ADAMW>), dim3(blocks), dim3(kOBlock), 0, stream(), tab, a);
+    return check_launch();
+}
+
+// The tensors e[0..n) of one dtype, as few launches as the argument table and
+// the grid allow.
+static int launch_steps(int type, int dtype, const StepEntry *e, size_t n, const AdamArgs &a)
+{
+    for (size_t i = 0; i < n;) {
+        StepTab tab;
+        tab.count = 0;
+        tab.tiles = 1;
+        while (ceil_div(e[i].n, int64_t(tab.tiles) * kOBlock) > kMaxGridBlocks) tab.tiles *= 2;
+        int64_t blocks = 0;
+        for (; i < n && tab.count < kStepTab; i++) {
+            const int64_t nb = ceil_div(e[i].n, int64_t(tab.tiles) * kOBlock);
+            if (blocks + nb > kMaxGridBlocks) break;
+            tab.e[tab.count] = e[i];
+            tab.first[tab.count++] = int32_t(blocks);
+            blocks += nb;
+        }
+        NH_TRY(dtype == NEURAL_DTYPE_FLOAT32 ? launch_step<float>(type, tab, unsigned(blocks), a)
+                                             : launch_step<double>(type, tab, unsigned(blocks), a));
     }
+    return NEURAL_OK;
 }
 
-// sgd_step_impl (optimizers_c.c:218-249).
-__global__ __launch_bounds__(kOBlock) void k_sgd_f32(float *__restrict__ p, const float *__restrict__ g,
-                                                     double *__restrict__ vel, int64_t n, double lr, double mom)
-{
-    const int64_t stride = int64_t(gridDim.x) * kOBlock;
-    for (int64_t j = int64_t(blockIdx.x) * kOBlock + threadIdx.x; j < n; j += stride) {
-        const double grad = double(ld_nt(g + j));
-        const double nv = mom * ld_nt(vel + j) + grad;
-        st_nt(vel + j, nv);
-        st_nt(p + j, ld_nt(p + j) - float(lr * nv));
-    }
-}
-
-__global__ __launch_bounds__(kOBlock) void k_sgd_f64(double *__restrict__ p, const double *__restrict__ g,
-                                                     double *__restrict__ vel, int64_t n, double lr, double mom)
-{
-    const int64_t stride = int64_t(gridDim.x) * kOBlock;
-    for (int64_t j = int64_t(blockIdx.x) * kOBlock + threadIdx.x; j < n; j += stride) {
-        const double nv = mom * ld_nt(vel + j) + ld_nt(g + j);
-        st_nt(vel + j, nv);
-        st_nt(p + j, ld_nt(p + j) - lr * nv);
-    }
-}
-
-inline unsigned o_grid(int64_t n)
-{
-    int64_t g = ceil_div(n, kOBlock);
-    const int64_t cap = kMaxGridBlocks;
-    if (g > cap) g = cap;
-    return unsigned(g < 1 ? 1 : g);
-}
-
-static int step_param(OptHandle *o, size_t i, NeuralTensor *p, const NeuralTensor *g, const AdamArgs &a)
+// One parameter of the step, made ready on the device (nothing launched).
+static int step_prepare(OptHandle *o, size_t i, NeuralTensor *p, const NeuralTensor *g, StepEntry &e)
 {
     const int64_t sz = o->sizes[i];
+    e.n = 0;
     if (!p || !g) return set_error(NEURAL_ERR_NULL_POINTER);
     NH_TRY(check_tensor(p));
     if (g->dtype != p->dtype) return set_error(NEURAL_ERR_DTYPE_MISMATCH);
     if (numel(p) != sz || numel(g) != sz) return set_error(NEURAL_ERR_SHAPE_MISMATCH);
     if (!is_contiguous(p) || !is_contiguous(g)) return set_error(NEURAL_ERR_INVALID_ARGUMENT);
     if (sz == 0) return NEURAL_OK;
-    const void *gp = nullptr;
     const void *pr = nullptr;
-    void *pw = nullptr;
-    NH_TRY(dev_read(g, &gp));
+    NH_TRY(dev_read(g, &e.g));
     NH_TRY(dev_read(p, &pr));
-    NH_TRY(dev_write(p, &pw, false));
-    if (o->type == OPT_SGD) {
-        if (p->dtype == NEURAL_DTYPE_FLOAT32)
-            NH_LAUNCH(k_sgd_f32, dim3(o_grid(sz)), dim3(kOBlock), 0, stream(), static_cast<float *>(pw),
-                               static_cast<const float *>(gp), o->vel[i], sz, o->lr, o->momentum);
-        else
-            NH_LAUNCH(k_sgd_f64, dim3(o_grid(sz)), dim3(kOBlock), 0, stream(), static_cast<double *>(pw),
-                               static_cast<const double *>(gp), o->vel[i], sz, o->lr, o->momentum);
-    } else {
-        const bool w = o->type == OPT_ADAMW;
-        if (p->dtype == NEURAL_DTYPE_FLOAT32) {
-            float *P = static_cast<float *>(pw);
-            const float *G = static_cast<const float *>(gp);
-            if (w) NH_LAUNCH(k_adam_f32<true>, dim3(o_grid(sz)), dim3(kOBlock), 0, stream(), P, G, o->m[i], o->v[i], sz, a);
-            else NH_LAUNCH(k_adam_f32<false>, dim3(o_grid(sz)), dim3(kOBlock), 0, stream(), P, G, o->m[i], o->v[i], sz, a);
-        } else {
-            double *P = static_cast<double *>(pw);
-            const double *G = static_cast<const double *>(gp);
-            if (w) NH_LAUNCH(k_adam_f64<true>, dim3(o_grid(sz)), dim3(kOBlock), 0, stream(), P, G, o->m[i], o->v[i], sz, a);
-            else NH_LAUNCH(k_adam_f64<false>, dim3(o_grid(sz)), dim3(kOBlock), 0, stream(), P, G, o->m[i], o->v[i], sz, a);
+    NH_TRY(dev_write(p, &e.p, false));
+    e.m = o->type == OPT_SGD ? o->vel[i] : o->m[i];
+    e.v = o->type == OPT_SGD ? nullptr : o->v[i];
+    e.n = sz;
+    return NEURAL_OK;
+}
+
+// True when the order of the parameters' updates could show: a parameter
+// tensor that shares bytes with another parameter or with a gradient (tied
+// weights passed twice), or a tensor whose bytes are the caller's host memory.
+static bool step_order_matters(void **params, void **grads, int64_t n)
+{
+    struct Span {
+        uintptr_t lo, hi;
+        bool write;
+    };
+    std::vector<Span> s;
+    s.reserve(size_t(2 * n));
+    for (int64_t i = 0; i < n; i++) {
+        const NeuralTensor *t[2] = {static_cast<const NeuralTensor *>(params[i]),
+                                    static_cast<const NeuralTensor *>(grads[i])};
+        for (int k = 0; k < 2; k++) {
+            if (!t[k]) continue;
+            if (t[k]->st->kind == KIND_EXT_HOST) return true;
+            const uintptr_t lo = reinterpret_cast<uintptr_t>(t[k]->dev);
+            s.push_back({lo, lo + uintptr_t(numel(t[k])) * elem_size(t[k]->dtype), k == 0});
         }
     }
-    NH_TRY(check_launch());
-    NH_TRY(dev_written(p));
-    return NEURAL_OK;
+    std::sort(s.begin(), s.end(), [](const Span &a, const Span &b) { return a.lo < b.lo; });
+    uintptr_t end_any = 0, end_write = 0;
+    for (const Span &x : s) {
+        if (x.lo < x.hi && (x.lo < end_write || (x.write && x.lo < end_any))) return true;
+        end_any = x.hi > end_any ? x.hi : end_any;
+        if (x.write) end_write = x.hi > end_write ? x.hi : end_write;
+    }
+    return false;
+}
+
+// Every parameter's update.  The first parameter that cannot be updated ends
+// the step with its error, after the ones before it have been updated (the
+// reference's loop, optimizers_c.c:218-348).
+static int step_all(OptHandle *o, void **params, void **grads, int64_t n, const AdamArgs &a)
+{
+    const bool ordered = n > 1 && step_order_matters(params, grads, n);
+    std::vector<StepEntry> list[2];  // by dtype
+    std::vector<NeuralTensor *> written;
+    if (!ordered)
+        for (auto &l : list) l.reserve(size_t(n));
+    written.reserve(size_t(n));
+    int rc = NEURAL_OK;
+    for (int64_t i = 0; i < n && rc == NEURAL_OK; i++) {
+        NeuralTensor *p = static_cast<NeuralTensor *>(params[i]);
+        StepEntry e;
+        rc = step_prepare(o, size_t(i), p, static_cast<const NeuralTensor *>(grads[i]), e);
+        if (rc != NEURAL_OK || e.n == 0) continue;
+        if (ordered) {
+            rc = launch_steps(o->type, p->dtype, &e, 1, a);
+            if (rc == NEURAL_OK) rc = dev_written(p);
+        } else {
+            list[p->dtype == NEURAL_DTYPE_FLOAT32 ? 0 : 1].push_back(e);
+            written.push_back(p);
+        }
+    }
+    for (int d = 0; d < 2; d++) {
+        const int lrc = launch_steps(o->type, d == 0 ? NEURAL_DTYPE_FLOAT32 : NEURAL_DTYPE_FLOAT64, list[d].data(),
+                                     list[d].size(), a);
+        rc = rc == NEURAL_OK ? lrc : rc;
+    }
+    for (NeuralTensor *p : written) {
+        const int wrc = dev_written(p);
+        rc = rc == NEURAL_OK ? wrc : rc;
+    }
+    return rc == NEURAL_OK ? NEURAL_OK : set_error(rc);
 }
 
 static OptHandle *make(int type)
@@ -322,9 +398,8 @@ static int opt_step_impl(void *opt, void **params, void **grads, int64_t n)
         a.bc1 = 1.0 - std::pow(o->beta1, double(o->t));
         a.bc2 = 1.0 - std::pow(o->beta2, double(o->t));
     }
-    for (int64_t i = 0; i < n; i++)
-        NH_TRY(step_param(o, size_t(i), static_cast<NeuralTensor *>(params[i]),
-                          static_cast<const NeuralTensor *>(grads[i]), a));
+    if (o->type == OPT_SGD) a.b1 = o->momentum;
+    NH_TRY(step_all(o, params, grads, n, a));
     return set_error(NEURAL_OK);
 }
 

@@ -4,7 +4,7 @@ interface of the reference's ``pyneural/optim.py:16-237`` over the C
 optimizer handle of ``optimizers_c.c:135-562``.
 
 One handle owns the float64 moments (on the GPU here) and the step counter;
-``opt_step`` updates every parameter with one fused kernel each.  The state
+``opt_step`` updates every parameter, up to 88 tensors to a launch.  The state
 blob is the OPTS format of ``opt_state_export`` (checkpoints embed it).
 
 Each concrete optimizer only names its C constructor and the order of the

@@ -83,6 +83,93 @@ def test_steps_bit_exact(pn, ora, kind, dt, n):
         same_bits(gv2, v2)
 
 
+@pytest.mark.parametrize("kind", ["adamw", "adam", "sgd"])
+@pytest.mark.parametrize("count", [2, 64, 65, 88, 89, 200])
+def test_step_many_tensors(pn, ora, kind, count):
+    """Lists around what one launch holds (88 tensors, 64 per ballot), mixed
+    dtypes, sizes around the 256-element tile and empty ones, parameters that
+    are slices of one buffer at odd offsets: bit-exact against the oracle."""
+    import torch
+    rng = np.random.default_rng(count)
+    sizes = [int(rng.choice([0, 1, 255, 256, 257, 511, 513, 1000, 5000])) for _ in range(count)]
+    dts = [np.float32 if rng.random() < 0.7 else np.float64 for _ in range(count)]
+    flat = {d: torch.zeros(sum(sizes) + 8, dtype=torch.float32 if d == np.float32 else torch.float64, device="cuda")
+            for d in (np.float32, np.float64)}
+    at = {np.float32: 1, np.float64: 1}
+    ps, gs, ref = [], [], []
+    for n, d in zip(sizes, dts):
+        p, g = _data(n, d, seed=n + len(ps))
+        view = flat[d][at[d]:at[d] + n]
+        at[d] += n
+        view.copy_(torch.from_numpy(p))
+        ps.append((pn.Tensor.from_torch(view) if n else pn.Tensor.from_numpy(p), view))
+        gs.append(pn.Tensor.from_numpy(g))
+        ref.append([p, g, np.zeros(n), np.zeros(n)])
+    torch.cuda.synchronize()
+    opt = {"adamw": lambda: pn.AdamW(LR, B1, B2, EPS, WD), "adam": lambda: pn.Adam(LR, B1, B2, EPS),
+           "sgd": lambda: pn.SGD(0.01, 0.9)}[kind]()
+    for step in range(1, 4):
+        opt.step([p for p, _ in ps], gs)
+        for p, g, m, v in ref:
+            if not p.size:
+                continue
+            if kind == "adamw":
+                ora.adamw_step(p, g, m, v, LR, B1, B2, EPS, WD, step)
+            elif kind == "adam":
+                ora.adam_step(p, g, m, v, LR, B1, B2, EPS, step)
+            else:
+                ora.sgd_step(p, g, m, 0.01, 0.9)
+    torch.cuda.synchronize()
+    for (_, view), (p, _, _, _) in zip(ps, ref):
+        same_bits(view.cpu().numpy(), p)
+    blob = opt.state_bytes()
+    got = _blob_moments(blob, sizes, 1 if kind == "sgd" else 2)
+    for k, (_, _, m, v) in enumerate(ref):
+        same_bits(got[k], m)
+        if kind != "sgd":
+            same_bits(got[count + k], v)
+
+
+def test_step_order_and_errors_in_lists(pn, ora):
+    """A tensor passed twice (tied weights) is stepped twice, in order, each
+    with its own moments; host-buffer tensors sharing one buffer likewise; a
+    list that fails at its third tensor has updated the first two."""
+    n = 1000
+    p, g = _data(n, np.float32, 3)
+    g2 = (g * 2).astype(np.float32)
+
+    def twice(r):
+        m, v, m2, v2 = (np.zeros(n) for _ in range(4))
+        for t in (1, 2):
+            ora.adamw_step(r, g, m, v, LR, B1, B2, EPS, WD, t)
+            ora.adamw_step(r, g2, m2, v2, LR, B1, B2, EPS, WD, t)
+        return r
+
+    tp, tg, tg2 = pn.Tensor.from_numpy(p), pn.Tensor.from_numpy(g), pn.Tensor.from_numpy(g2)
+    opt = pn.AdamW(LR, B1, B2, EPS, WD)
+    for _ in range(2):
+        opt.step([tp, tp], [tg, tg2])
+    same_bits(tp.numpy(), twice(p.copy()))
+
+    host = p.copy()
+    h1, h2 = pn.Tensor.from_numpy_zero_copy(host), pn.Tensor.from_numpy_zero_copy(host)
+    opt = pn.AdamW(LR, B1, B2, EPS, WD)
+    for _ in range(2):
+        opt.step([h1, h2], [tg, tg2])
+    same_bits(host, twice(p.copy()))
+
+    opt = pn.AdamW(LR, B1, B2, EPS, WD)
+    a, b, c = (pn.Tensor.from_numpy(p) for _ in range(3))
+    with pytest.raises(pn.NeuralException) as e:
+        opt.step([a, b, c, a], [tg, tg2, pn.Tensor.from_numpy(g[:5]), tg])
+    assert e.value.error_code == pn.NeuralError.SHAPE_MISMATCH
+    for t, gr in ((a, g), (b, g2)):
+        r = p.copy()
+        ora.adamw_step(r, gr, np.zeros(n), np.zeros(n), LR, B1, B2, EPS, WD, 1)
+        same_bits(t.numpy(), r)
+    same_bits(c.numpy(), p)
+
+
 def test_adamw_cfg5_ten_steps(pn, ora):
     """cfg5's AdamW as BASELINE specifies it (params N(0, 0.02), grads
     N(0, 1e-3) with 32 NaN, 32 +Inf and 32 -Inf injected, lr 1e-3, wd 0.01),
