@@ -253,6 +253,28 @@ int build_nd(const NeuralTensor *out, const NeuralTensor *a, const NeuralTensor 
     return NEURAL_OK;
 }
 
+bool nd32_of(const ND4 &d, int64_t n, ND32 &o)
+{
+    constexpr int64_t kMax = INT32_MAX;
+    if (n > kMax) return false;
+    const int64_t *from[3] = {d.so, d.sa, d.sb};
+    int32_t *to[3] = {o.so, o.sa, o.sb};
+    for (int k = 0; k < 3; k++) {
+        int64_t reach = 0;  // largest offset in either direction, all dims together
+        for (int i = 0; i < 4; i++) {
+            const int64_t st = from[k][i] < 0 ? -from[k][i] : from[k][i];
+            if (d.shape[i] > 1 && st > kMax / (d.shape[i] - 1)) return false;
+            reach += (d.shape[i] - 1) * st;
+            to[k][i] = d.shape[i] > 1 ? int32_t(from[k][i]) : 0;
+        }
+        if (reach > kMax) return false;
+    }
+    o.d3 = fast_div(uint32_t(d.shape[3]));
+    o.d2 = fast_div(uint32_t(d.shape[2]));
+    o.d1 = fast_div(uint32_t(d.shape[1]));
+    return true;
+}
+
 // ---- raw-pointer f32 (simd.asm) --------------------------------------------------------
 
 struct OpFma {

@@ -327,16 +327,117 @@ __global__ __launch_bounds__(kBlock) void k_map2_nd(const T *a, const T *b, T *o
     }
 }
 
-template <typename T, typename F>
-__global__ __launch_bounds__(kBlock) void k_map1_nd(const T *a, T *o, int64_t n, ND4 d, F f)
+// The same with 32-bit indices: up to 2^31 - 1 output elements, every operand's
+// offsets below 2^31.  Division by an extent is a multiply-high and a shift
+// (exact for n < 2^31: m = floor(2^(31 + s) / d) + 1, s = ceil(log2 d)).
+struct FastDiv {
+    uint32_t d, m, sh;
+    NH_DEV uint32_t div(uint32_t n) const { return d == 1 ? n : __umulhi(n, m) >> sh; }
+};
+inline FastDiv fast_div(uint32_t d)
 {
-    const int64_t stride = int64_t(gridDim.x) * kBlock;
-    for (int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x; i < n; i += stride) {
-        int64_t oo, oa, ob;
-        nd_offsets(d, i, oo, oa, ob);
-        o[oo] = f(a[oa]);
+    const uint32_t s = d > 1 ? 32 - uint32_t(__builtin_clz(d - 1)) : 0;
+    return {d, uint32_t((uint64_t(1) << (31 + s)) / d + 1), s ? s - 1 : 0};
+}
+struct ND32 {
+    FastDiv d3, d2, d1;  // extents of dims 3 (innermost), 2, 1
+    int32_t so[4], sa[4], sb[4];
+};
+// ND32 of d when the indices and offsets of n elements fit 32 bits.
+bool nd32_of(const ND4 &d, int64_t n, ND32 &o);
+
+struct Off3 {
+    int32_t o, a, b;
+    uint32_t i3;
+};
+NH_DEV Off3 nd32_offsets(const ND32 &d, uint32_t idx)
+{
+    const uint32_t r = d.d3.div(idx), i3 = idx - r * d.d3.d;
+    const uint32_t q = d.d2.div(r), i2 = r - q * d.d2.d;
+    const uint32_t i0 = d.d1.div(q), i1 = q - i0 * d.d1.d;
+    const auto off = [&](const int32_t (&s)[4]) {
+        return int32_t(i0) * s[0] + int32_t(i1) * s[1] + int32_t(i2) * s[2] + int32_t(i3) * s[3];
+    };
+    return {off(d.so), off(d.sa), off(d.sb), i3};
+}
+
+// VEC: the output is contiguous and each input's innermost stride is 0 or 1;
+// a lane then makes kFlatU 16-byte vectors of the output, reading VN values of
+// a dense operand at its own alignment and one value of a broadcast one, and
+// finds its place once per vector.  A vector that runs past the end of an
+// innermost row is made element by element.  Else: one element per lane.
+// Bound by HBM like the flat kernels; the 64-bit form spends three 64-bit
+// divisions per element and 4-byte accesses.  Before -> now, us: f32
+// [32, 256, 56, 56] times, then plus [1, 256, 1, 1] 192 -> 67 (411 MB), [32, 256,
+// 57, 57] 199 -> 69, f64 [16, 64, 112, 112] 104 -> 68; bias + leaky ReLU and
+// column sums f32 [41280, 126] 199 -> 33; calls of a few microseconds alike.
+template <typename T, typename Op, bool VEC>
+__global__ __launch_bounds__(kBlock) void k_map2_nd32(const T *a, const T *b, T *o, uint32_t n, ND32 d, Op op)
+{
+    if constexpr (VEC) {
+        using V = typename Vec16<T>::type;
+        using U = typename VecU<T>::type;
+        constexpr uint32_t VN = Vec16<T>::n;
+        const uint32_t nv = n / VN;
+        const uint32_t base = uint32_t(flat_lane0(int64_t(blockIdx.x) * (kBlock * kFlatU)));
+        const auto read = [](const T *p, bool dense) {
+            if (dense) return V(*reinterpret_cast<const U *>(p));
+            V v;
+            const T x = *p;
+#pragma unroll
+            for (uint32_t k = 0; k < VN; k++) v[k] = x;
+            return v;
+        };
+        V ra[kFlatU], rb[kFlatU];
+        Off3 at[kFlatU];
+#pragma unroll
+        for (int u = 0; u < kFlatU; u++) {
+            const uint32_t i = base + u * 64;
+            if (i < nv) {
+                at[u] = nd32_offsets(d, i * VN);
+                if (at[u].i3 + VN <= d.d3.d) {
+                    ra[u] = read(a + at[u].a, d.sa[3] != 0);
+                    rb[u] = read(b + at[u].b, d.sb[3] != 0);
+                } else {
+#pragma unroll
+                    for (uint32_t k = 0; k < VN; k++) {
+                        const Off3 f = nd32_offsets(d, i * VN + k);
+                        ra[u][k] = a[f.a];
+                        rb[u][k] = b[f.b];
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kFlatU; u++) {
+            const uint32_t i = base + u * 64;
+            if (i < nv) {
+                V r;
+#pragma unroll
+                for (uint32_t k = 0; k < VN; k++) r[k] = op(ra[u][k], rb[u][k]);
+                reinterpret_cast<U *>(o)[i] = r;
+            }
+        }
+        if (blockIdx.x == 0 && nv * VN + threadIdx.x < n) {
+            const uint32_t j = nv * VN + threadIdx.x;
+            const Off3 f = nd32_offsets(d, j);
+            o[j] = op(a[f.a], b[f.b]);
+        }
+    } else {
+        const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+        if (i >= n) return;
+        const Off3 f = nd32_offsets(d, i);
+        o[f.o] = op(a[f.a], b[f.b]);
     }
 }
+
+// Unary f over the same layouts: a binary op that ignores its second operand
+// (strides 0, the first operand's own address).
+template <typename F>
+struct OpFirst {
+    F f;
+    template <class T> NH_DEV T operator()(T x, T) const { return f(x); }
+};
 
 // ---- host-side launch helpers ---------------------------------------------------
 
@@ -357,6 +458,24 @@ inline unsigned strided_grid(int64_t n)
     const int64_t cap = kMaxGridBlocks;
     if (g > cap) g = cap;
     return unsigned(g < 1 ? 1 : g);
+}
+
+// o = op(a, b) over the layout d of n output elements (out_dense: the output
+// is contiguous).
+template <typename T, typename Op>
+int launch_map2_nd(const T *a, const T *b, T *o, int64_t n, const ND4 &d, bool out_dense, Op op)
+{
+    ND32 e;
+    if (!nd32_of(d, n, e)) {
+        NH_LAUNCH((k_map2_nd<T, Op>), dim3(strided_grid(n)), dim3(kBlock), 0, stream(), a, b, o, n, d, op);
+    } else if (out_dense && (e.sa[3] | e.sb[3] | 1) == 1) {
+        NH_LAUNCH((k_map2_nd32<T, Op, true>), dim3(flat_grid(n, Vec16<T>::n)), dim3(kBlock), 0, stream(), a, b, o,
+                  uint32_t(n), e, op);
+    } else {
+        NH_LAUNCH((k_map2_nd32<T, Op, false>), dim3(strided_grid(n)), dim3(kBlock), 0, stream(), a, b, o, uint32_t(n),
+                  e, op);
+    }
+    return check_launch();
 }
 
 template <typename T, typename Op>
@@ -472,13 +591,14 @@ int run_unary(NeuralTensor *out, const NeuralTensor *in, F32 f32, F64 f64)
     } else {
         ND4 d;
         NH_TRY(build_nd(out, in, nullptr, d));
-        if (in->dtype == NEURAL_DTYPE_FLOAT32)
-            NH_LAUNCH((k_map1_nd<float, F32>), dim3(strided_grid(n)), dim3(kBlock), 0, stream(),
-                               static_cast<const float *>(src), static_cast<float *>(dst), n, d, f32);
-        else
-            NH_LAUNCH((k_map1_nd<double, F64>), dim3(strided_grid(n)), dim3(kBlock), 0, stream(),
-                               static_cast<const double *>(src), static_cast<double *>(dst), n, d, f64);
-        NH_TRY(check_launch());
+        const bool dense = is_contiguous(out);
+        if (in->dtype == NEURAL_DTYPE_FLOAT32) {
+            const float *A = static_cast<const float *>(src);
+            NH_TRY(launch_map2_nd(A, A, static_cast<float *>(dst), n, d, dense, OpFirst<F32>{f32}));
+        } else {
+            const double *A = static_cast<const double *>(src);
+            NH_TRY(launch_map2_nd(A, A, static_cast<double *>(dst), n, d, dense, OpFirst<F64>{f64}));
+        }
     }
     NH_TRY(dev_written(out));
     return set_error(NEURAL_OK);
@@ -524,8 +644,7 @@ int launch_binary(NeuralTensor *out, const NeuralTensor *a, const NeuralTensor *
     }
     ND4 d;
     NH_TRY(build_nd(out, a, b, d));
-    NH_LAUNCH((k_map2_nd<T, Op>), dim3(strided_grid(n)), dim3(kBlock), 0, stream(), A, B, O, n, d, op);
-    return check_launch();
+    return launch_map2_nd(A, B, O, n, d, is_contiguous(out), op);
 }
 
 // Binary op on tensors: flat when all three are contiguous and equal in size,

@@ -101,3 +101,59 @@ def test_random_broadcast_and_views(pn, dt):
             same_bits(got, want.astype(dt))
             if okind == 2 and to.dim() >= 1:
                 assert bool((base[..., 1::2] == 0).all()), (case, op, "stepped output wrote between its elements")
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("inner", [1, 2, 3, 4, 5, 7, 49, 63, 64, 65, 3001])
+def test_broadcast_vector_edges(pn, dt, inner):
+    """The 4-D broadcasts whose output is made in 16-byte vectors: innermost
+    extents around the vector (vectors that run past a row's end), broadcast
+    along any dimension on either side, operands that start inside a vector,
+    in place, and strided or reversed operands and outputs, which take the
+    element-wise form.  Bit-exact against numpy, as is a unary op on views."""
+    import torch
+    lib = pn.core._lib
+    rng = np.random.default_rng(inner)
+    shape = (3, 5, 2, inner)
+    T = torch.float32 if dt == np.float32 else torch.float64
+    n = int(np.prod(shape))
+
+    def wrap(arr, off=0, strides=None):
+        """arr in a device buffer at an element offset (contiguous)."""
+        buf = torch.zeros(arr.size + 4, dtype=T, device="cuda")
+        v = buf[off:off + arr.size].view(arr.shape)
+        v.copy_(torch.from_numpy(np.ascontiguousarray(arr)))
+        return v
+
+    pn.set_stream(torch.cuda.current_stream().cuda_stream)
+    try:
+        x = rng.normal(0, 1, shape).astype(dt)
+        for bs in [(1, 5, 1, 1), (5, 1, 1), (3, 1, 2, 1), (inner,), (1, 1, 1, inner), (3, 1, 1, inner), (1,), (2, 1),
+                   shape]:
+            b = rng.normal(0, 1, bs).astype(dt)
+            for oa, ob, oo in ((0, 0, 0), (1, 3, 2)):
+                va, vb, vo = wrap(x, oa), wrap(b, ob), wrap(np.zeros(shape, dt), oo)
+                ta, tb, to = (pn.Tensor.from_torch(v) for v in (va, vb, vo))
+                for f, op in ((lib.neural_add, np.add), (lib.neural_sub, np.subtract)):
+                    assert f(to._ptr, ta._ptr, tb._ptr) == 0
+                    same_bits(vo.cpu().numpy(), op(x, b))
+                assert lib.neural_sub(to._ptr, tb._ptr, ta._ptr) == 0  # the broadcast operand first
+                same_bits(vo.cpu().numpy(), np.subtract(b, x))
+                assert lib.neural_mul(ta._ptr, ta._ptr, tb._ptr) == 0  # in place
+                same_bits(va.cpu().numpy(), x * b)
+        # views: permuted, stepped, strided output
+        big = rng.normal(0, 1, (2, 5, 3, 2 * inner)).astype(dt)
+        vb = wrap(big)
+        views = [(vb.permute(2, 1, 0, 3)[..., ::2], big.transpose(2, 1, 0, 3)[..., ::2]),
+                 (vb.permute(2, 1, 0, 3)[..., :inner], big.transpose(2, 1, 0, 3)[..., :inner])]
+        for tv, nv in views:
+            out = torch.zeros((3, 5, 2, 2 * inner), dtype=T, device="cuda")
+            for vo in (torch.zeros(shape, dtype=T, device="cuda"), out[..., ::2]):
+                ta, tb, to = pn.Tensor.from_torch(wrap(x)), pn.Tensor.from_torch(tv), pn.Tensor.from_torch(vo)
+                assert lib.neural_add(to._ptr, ta._ptr, tb._ptr) == 0
+                same_bits(vo.cpu().numpy().copy(), x + nv)
+                assert lib.neural_neg(to._ptr, tb._ptr) == 0
+                same_bits(vo.cpu().numpy().copy(), -np.ascontiguousarray(nv))
+            assert bool((out[..., 1::2] == 0).all())
+    finally:
+        pn.set_stream(None)
