@@ -239,3 +239,32 @@ def test_reduce_deterministic_large(pn, ora):
     assert outs[0] == outs[1] == outs[2]
     e = ora.rowsum_exact(x)
     assert np.all(np.abs(np.frombuffer(outs[0], np.float32) - e) <= 1e-5 * np.sum(np.abs(x), axis=1) + np.abs(e) * 6e-8)
+
+
+@pytest.mark.parametrize("cols", [1, 2, 3, 4, 5, 17, 63, 126, 128, 129, 255, 256, 257, 259, 515, 4097])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_colsum_edges(pn, dt, cols):
+    """Column sums and means where the lanes' column vectors, the rows per wave
+    and the row chunks end unevenly, from buffers that start inside a vector:
+    within 1e-5 (f32) / 1e-13 (f64) of sum|x| of the float64 sum."""
+    import torch
+    rng = np.random.default_rng(cols)
+    tol = 1e-5 if dt == np.float32 else 1e-13
+    pn.set_stream(torch.cuda.current_stream().cuda_stream)
+    try:
+        for rows in (1, 2, 31, 64, 65, 513, 4100):
+            x = rng.normal(0, 3, (rows, cols)).astype(dt)
+            buf = torch.zeros(rows * cols + 3, dtype=torch.float32 if dt == np.float32 else torch.float64,
+                              device="cuda")
+            for off in (0, 1):
+                v = buf[off:off + rows * cols].view(rows, cols)
+                v.copy_(torch.from_numpy(x))
+                t, out = pn.Tensor.from_torch(v), pn.Tensor.create([cols], pn.float32 if dt == np.float32 else pn.float64)
+                e = x.astype(np.float64).sum(axis=0)
+                bound = tol * np.abs(x.astype(np.float64)).sum(axis=0)
+                assert pn.core._lib.neural_reduce_sum(t._ptr, 0, out._ptr) == 0
+                assert np.all(np.abs(out.numpy() - e) <= bound), (rows, off)
+                assert pn.core._lib.neural_reduce_mean(t._ptr, 0, out._ptr) == 0
+                assert np.all(np.abs(out.numpy() - e / rows) <= bound / rows), (rows, off)
+    finally:
+        pn.set_stream(None)
