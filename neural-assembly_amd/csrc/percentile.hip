@@ -6,8 +6,16 @@
 // (clamped to [0, n - 1]; p outside [0, 0.5] taken as 0.01) and calibrates on
 // that range with the same expressions as calibrate_minmax.
 //
-// Here the two order statistics are found by a radix select on the device,
-// never sorting: each element maps to a 64-bit key that orders as the
+// Here the two order statistics are found on the device without sorting the
+// data.  First a sampled select (select_sampled): 2048 sampled values, sorted
+// by one block, bracket each rank; one pass over the data counts what lies
+// below each bracket and copies the keys strictly inside it; a histogram over
+// the copied keys narrows them to one bucket, which one block sorts.  The
+// result is exact: the counts say where each rank lies, and a rank that its
+// bracket missed, or copies that do not fit, send the call to the radix
+// select below.  Data of up to 2048 values are sorted as they are.
+//
+// The radix select (select_ranks): each element maps to a 64-bit key that orders as the
 // comparator does (-0 and +0 compare equal, so they share one key), and eight
 // histogram passes -- 12 bits (sign and exponent), six of 8 bits, 4 bits; one
 // histogram for each rank, counting only the elements that match the rank's
@@ -36,6 +44,7 @@
 
 #include "common.hpp"
 #include "quant_common.hpp"
+#include "reduce_impl.hpp"
 
 namespace nh {
 
@@ -382,6 +391,668 @@ __global__ __launch_bounds__(64) void k_pct_zero_pick(const double *__restrict__
 
 }  // namespace
 
+// ---- the sampled select --------------------------------------------------------------
+
+namespace {
+
+constexpr int kFB = 1024;        // lanes of the one-block steps
+constexpr int kSample = 2 * kFB; // sampled values
+constexpr int kList = 4096;      // the most keys the last step looks at per rank
+constexpr int kFineBins = 8192;  // buckets of the histogram over the copied keys
+
+constexpr int64_t kMaxCopies = int64_t(1) << 22;
+
+// How far the bracket of the rank at fraction f reaches to either side, in
+// sampled values.
+__host__ __device__ inline double sample_margin(double f) { return 4.0 * sqrt(kSample * f * (1.0 - f)) + 3.0; }
+
+struct PctFast {
+    double l[2], u[2];  // bracket of each rank
+    // elements below l, equal to l, strictly inside, equal to u
+    unsigned long long lt[2], eql[2], in[2], equ[2];
+    unsigned long long kmin[2], kmax[2];  // keys of the elements strictly inside
+    int bucket[2];      // the rank's bucket, -1: none to search
+    int64_t rem[2];     // the rank's place in its bucket
+    int64_t count[2];   // elements in its bucket
+    unsigned long long bmin[2], bmax[2];  // smallest and largest key of a bucket too full to list
+    unsigned listed[2];
+    int bad;            // give up: the radix select answers
+};
+
+// What each block of the pass over the data saw, per rank, one array per value:
+// the counts, the range of the keys strictly inside (as doubles), and the keys
+// it copied.  (8192 waves adding into one record by atomics took 500 us.)
+struct PctSeen {
+    double *mn[2], *mx[2];
+    unsigned *n[8];  // lt, eql, in, equ: rank 0, rank 1 each
+    unsigned *copied;
+};
+
+// Ascending bitonic sort of kSample keys by kFB lanes, lane t holding keys 2 t
+// and 2 t + 1: neighbours meet in registers, partners up to 64 apart by lane
+// shuffles, beyond in LDS (10 of the 66 steps).  4096 keys with every step in
+// LDS took 42 us with the sampling, 18 now.
+__device__ void block_sort(uint64_t (&k)[2], uint64_t *lds)
+{
+    static_assert(kSample == 2 * kFB, "two keys per lane");
+    const int i0 = 2 * int(threadIdx.x);
+    for (int w = 2; w <= kSample; w <<= 1) {
+        const bool up = (i0 & w) == 0;
+        for (int j = w >> 1; j >= 2; j >>= 1) {
+            const bool keep_min = ((i0 & j) == 0) == up;
+            uint64_t o[2];
+            if (j >= 128) {
+                __syncthreads();
+                lds[i0] = k[0];
+                lds[i0 + 1] = k[1];
+                __syncthreads();
+                o[0] = lds[i0 ^ j];
+                o[1] = lds[(i0 ^ j) + 1];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 2; e++) o[e] = __shfl_xor(static_cast<unsigned long long>(k[e]), j >> 1, 64);
+            }
+#pragma unroll
+            for (int e = 0; e < 2; e++) k[e] = (k[e] < o[e]) == keep_min ? k[e] : o[e];
+        }
+        const bool swap = (k[0] > k[1]) == up;
+        const uint64_t x = swap ? k[1] : k[0];
+        k[1] = swap ? k[0] : k[1];
+        k[0] = x;
+    }
+    __syncthreads();
+    lds[i0] = k[0];
+    lds[i0 + 1] = k[1];
+    __syncthreads();
+}
+
+__device__ __forceinline__ double key_double(uint64_t k)
+{
+    return __longlong_as_double(static_cast<long long>((k >> 63) ? (k & ~(uint64_t(1) << 63)) : ~k));
+}
+
+// One block: sample, sort, bracket.  Sample i is element h(i) of the i-th of
+// kSample equal slices (h a hash, so that no period of the data meets the
+// slices).  The bracket of rank r reaches 4 standard deviations of the sample
+// rank and 3 more to either side; past the sample's ends it is unbounded.
+// n <= kSample: the sample is the data, and the block answers (res).
+__global__ __launch_bounds__(kFB) void k_pct_sample(const double *__restrict__ x, int64_t n, int64_t r0, int64_t r1,
+                                                    PctFast *st, unsigned *hist, PctResult *res, Ticket tk)
+{
+    __shared__ uint64_t k[kSample];
+    const bool all = n <= kSample;
+    uint64_t mine[2];
+#pragma unroll
+    for (int e = 0; e < 2; e++) {
+        const int i = 2 * int(threadIdx.x) + e;
+        int64_t at = i;
+        if (!all) {
+            const int64_t a = int64_t(double(n) * i / kSample), b = int64_t(double(n) * (i + 1) / kSample);
+            uint32_t h = uint32_t(i) * 2654435761u;
+            h ^= h >> 15;
+            h *= 2246822519u;
+            h ^= h >> 13;
+            at = a + int64_t((double(h) * 0x1p-32) * double(b - a));
+        }
+        const double v = x[at < n ? at : n - 1];
+        // past the end of short data: above everything
+        mine[e] = i < n ? pct_key_bits(static_cast<uint64_t>(__double_as_longlong(v))) : ~uint64_t(0);
+    }
+    block_sort(mine, k);
+    if (all) {
+        if (threadIdx.x == 0) {
+            PctResult r;
+            r.err = 0;
+            for (int q = 0; q < 2; q++) {
+                const int at = int(q ? r1 : r0);
+                int lo = 0, hi = at;  // first place of the key
+                while (lo < hi) {
+                    const int mid = (lo + hi) / 2;
+                    if (k[mid] < k[at]) lo = mid + 1;
+                    else hi = mid;
+                }
+                r.key[q] = k[at];
+                r.within[q] = at - lo;
+            }
+            *res = r;
+            publish(tk);
+        }
+        return;
+    }
+    for (int i = threadIdx.x; i < 2 * kFineBins; i += kFB) hist[i] = 0u;
+    if (threadIdx.x < 2) {  // a lane per rank
+        const int q = int(threadIdx.x);
+        const double f = (double(q ? r1 : r0) + 0.5) / double(n);
+        const double dev = sample_margin(f);
+        const double lo = floor(kSample * f - dev), hi = ceil(kSample * f + dev);
+        const uint64_t kl = lo < 0.0 ? 0 : k[int(lo)], ku = hi > kSample - 1 ? 0 : k[int(hi)];
+        st->l[q] = lo < 0.0 ? -__builtin_inf() : key_double(kl);
+        st->u[q] = hi > kSample - 1 ? __builtin_inf() : key_double(ku);
+        st->bmin[q] = ~0ull;
+        st->bmax[q] = 0ull;
+        st->bucket[q] = -1;
+        st->rem[q] = st->count[q] = 0;
+        st->listed[q] = 0u;
+        // NaN data around a rank: give up
+        const uint64_t nan = __ballot(kl == ~uint64_t(0) || ku == ~uint64_t(0));
+        if (q == 0) st->bad = nan ? 1 : 0;
+    }
+}
+
+__device__ __forceinline__ uint64_t wave_min_u64(uint64_t v)
+{
+    for (int off = 32; off >= 1; off >>= 1) {
+        const uint64_t o = __shfl_xor(static_cast<unsigned long long>(v), off, 64);
+        v = o < v ? o : v;
+    }
+    return v;
+}
+__device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) { return ~wave_min_u64(~v); }
+
+// The one pass over the data, tiles dealt round-robin.  Most elements lie
+// between the two brackets: two compares and a ballot count them.  The others
+// (a few percent) are packed into the wave's LDS queue and looked at 64 at a
+// time: counted per rank with ballots, and the keys strictly inside either
+// bracket copied to the block's region.  A NaN compares false and counts as
+// above every bracket, where the comparator's order puts it.
+// Bound by HBM: 50 M values (400 MB) in 66 us at p = 0.001; looking at the
+// others in place took 87 (half the waves have one).
+__global__ __launch_bounds__(kPB) void k_pct_scan(const double *__restrict__ x, int64_t n, int64_t R,
+                                                  const PctFast *__restrict__ st, uint64_t *__restrict__ keys,
+                                                  PctSeen seen)
+{
+    constexpr int W = kPB / 64;
+    __shared__ unsigned nout;
+    __shared__ double queue[W][64 * (kPU + 1)];
+    __shared__ unsigned sn[W][8];
+    __shared__ double sr[W][4];
+    if (st->bad) return;  // set by an earlier launch: uniform
+    if (threadIdx.x == 0) nout = 0u;
+    __syncthreads();
+    const int lane = int(threadIdx.x & 63), w = int(threadIdx.x >> 6);
+    double *wq = queue[w];
+    const double l0 = st->l[0], u0 = st->u[0], l1 = st->l[1], u1 = st->u[1];
+    // brackets that meet leave nothing between them: um = inf
+    const double um = u0 < l1 ? u0 : __builtin_inf();
+    unsigned c[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // lt, eql, in, equ per rank; uniform over the wave
+    double mn[2] = {__builtin_inf(), __builtin_inf()}, mx[2] = {-__builtin_inf(), -__builtin_inf()};
+    const auto look = [&](double v) {  // one element per lane, NaN: none
+        uint64_t inside = 0;
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const double l = q ? l1 : l0, h = q ? u1 : u0;
+            const bool iq = v > l && v < h;
+            const uint64_t bq = __ballot(iq), el = __ballot(v == l);
+            c[q] += __popcll(__ballot(v < l));
+            c[2 + q] += __popcll(el);
+            c[4 + q] += __popcll(bq);
+            c[6 + q] += __popcll(__ballot(v == h) & ~el);  // l == u: one atom, counted once
+            inside |= bq;
+            mn[q] = __builtin_fmin(mn[q], iq ? v : __builtin_inf());
+            mx[q] = __builtin_fmax(mx[q], iq ? v : -__builtin_inf());
+        }
+        if (inside) {
+            unsigned base = 0u;
+            if (lane == 0) base = atomicAdd(&nout, unsigned(__popcll(inside)));
+            base = __builtin_amdgcn_readfirstlane(base);
+            const int64_t slot = int64_t(base) + __popcll(inside & ((uint64_t(1) << lane) - 1));
+            if (((inside >> lane) & 1) && slot < R)
+                keys[int64_t(blockIdx.x) * R + slot] =
+                    pct_key_bits(static_cast<uint64_t>(__double_as_longlong(v)));
+        }
+    };
+    const auto settle = [] {  // the wave's queue writes before its reads, and back
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    int qn = 0;  // queued, uniform; below 64 between tiles
+    for (int64_t t0 = int64_t(blockIdx.x) * kTile; t0 < n; t0 += int64_t(gridDim.x) * kTile) {
+        double v[kPU];
+        const bool full = t0 + kTile <= n;
+#pragma unroll
+        for (int u = 0; u < kPU; u++) {
+            const int64_t i = t0 + u * kPB + int64_t(threadIdx.x);
+            if (full || i < n) v[u] = __builtin_nontemporal_load(x + i);
+            else v[u] = __builtin_nan("");  // counts nowhere
+        }
+#pragma unroll
+        for (int u = 0; u < kPU; u++) {
+            const bool mid = v[u] > um && v[u] < l1;
+            const uint64_t other = __ballot(!mid);
+            c[1] += 64 - unsigned(__popcll(other));
+            if (other) {
+                if (!mid)
+                    wq[qn + int(__builtin_amdgcn_mbcnt_hi(uint32_t(other >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo(uint32_t(other), 0u)))] = v[u];
+                qn += __popcll(other);
+            }
+        }
+        if (qn >= 64) {
+            settle();
+            while (qn >= 64) {
+                qn -= 64;
+                look(wq[qn + lane]);
+            }
+            settle();
+        }
+    }
+    settle();
+    look(lane < qn ? wq[lane] : __builtin_nan(""));
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        for (int off = 32; off >= 1; off >>= 1) {
+            mn[q] = __builtin_fmin(mn[q], __shfl_xor(mn[q], off, 64));
+            mx[q] = __builtin_fmax(mx[q], __shfl_xor(mx[q], off, 64));
+        }
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) sn[w][i] = c[i];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            sr[w][q] = mn[q];
+            sr[w][2 + q] = mx[q];
+        }
+    }
+    __syncthreads();
+    const int t = int(threadIdx.x), q = t & 1;
+    if (t < 8) {
+        unsigned sum = 0;
+        for (int k = 0; k < W; k++) sum += sn[k][t];
+        seen.n[t][blockIdx.x] = sum;
+    } else if (t < 10) {
+        double m = sr[0][q];
+        for (int k = 1; k < W; k++) m = __builtin_fmin(m, sr[k][q]);
+        seen.mn[q][blockIdx.x] = m;
+    } else if (t < 12) {
+        double m = sr[0][2 + q];
+        for (int k = 1; k < W; k++) m = __builtin_fmax(m, sr[k][2 + q]);
+        seen.mx[q][blockIdx.x] = m;
+    } else if (t == 12) {
+        seen.copied[blockIdx.x] = nout;  // above R: the copies did not fit
+    }
+}
+
+// One block: the blocks' records into the state, a wave per value.
+__global__ __launch_bounds__(kFB) void k_pct_fold(PctFast *st, PctSeen seen, int g, int64_t R)
+{
+    if (st->bad) return;  // uniform: this launch writes it after the barrier below, when every wave has read it
+    const int lane = int(threadIdx.x & 63), w = int(threadIdx.x >> 6), q = w & 1;
+    __syncthreads();
+    constexpr int U = 16;  // loads in flight per lane
+    if (w < 8) {
+        unsigned long long sum = 0;
+        for (int b = lane; b < g; b += 64 * U) {
+            unsigned v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) v[u] = b + 64 * u < g ? seen.n[w][b + 64 * u] : 0u;
+#pragma unroll
+            for (int u = 0; u < U; u++) sum += v[u];
+        }
+        for (int off = 32; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        if (lane == 0) (w < 2 ? st->lt : w < 4 ? st->eql : w < 6 ? st->in : st->equ)[q] = sum;
+    } else if (w < 12) {
+        // the smallest, or minus the largest; nothing inside: kmin > kmax (+inf, -inf)
+        const bool low = w < 10;
+        const double *from = low ? seen.mn[q] : seen.mx[q];
+        double m = __builtin_inf();
+        for (int b = lane; b < g; b += 64 * U) {
+            double v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                v[u] = b + 64 * u < g ? from[b + 64 * u] : (low ? __builtin_inf() : -__builtin_inf());
+#pragma unroll
+            for (int u = 0; u < U; u++) m = __builtin_fmin(m, low ? v[u] : -v[u]);
+        }
+        for (int off = 32; off >= 1; off >>= 1) m = __builtin_fmin(m, __shfl_xor(m, off, 64));
+        if (lane == 0)
+            (low ? st->kmin : st->kmax)[q] = pct_key_bits(static_cast<uint64_t>(__double_as_longlong(low ? m : -m)));
+    } else if (w == 12) {
+        bool over = false;
+        for (int b = lane; b < g; b += 64 * U) {
+            unsigned v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) v[u] = b + 64 * u < g ? seen.copied[b + 64 * u] : 0u;
+#pragma unroll
+            for (int u = 0; u < U; u++) over = over || int64_t(v[u]) > R;
+        }
+        const uint64_t any = __ballot(over);
+        if (lane == 0) st->bad = any ? 1 : 0;
+    }
+}
+
+// Where rank r lies: 0 at l, 1 strictly inside, 2 at u, -1 outside the
+// bracket; rel: its place there.
+__device__ __forceinline__ int pct_place(const PctFast &s, int q, int64_t r, int64_t &rel)
+{
+    rel = r - int64_t(s.lt[q]);
+    if (rel < 0) return -1;
+    if (rel < int64_t(s.eql[q])) return 0;
+    rel -= int64_t(s.eql[q]);
+    if (rel < int64_t(s.in[q])) return 1;
+    rel -= int64_t(s.in[q]);
+    return rel < int64_t(s.equ[q]) ? 2 : -1;
+}
+
+// Buckets: (key - kmin) >> shift, below kFineBins.
+__device__ __forceinline__ int pct_shift(uint64_t kmin, uint64_t kmax)
+{
+    const uint64_t range = kmax - kmin;
+    const int bits = range ? 64 - __builtin_clzll(range) : 0;
+    return bits > 13 ? bits - 13 : 0;
+}
+static_assert(kFineBins == 1 << 13, "pct_shift");
+
+// Histogram of the copied keys strictly inside each rank's bracket: LDS
+// counters (64 KiB a block), so that a value that recurs does not queue at one
+// address (25000 equal outliers among 0.8% of 50 M values: 309 us with one
+// global atomic per key, 10 so).  A wave per region.
+__global__ __launch_bounds__(kFB) void k_pct_fine(const PctFast *__restrict__ st, int64_t R, int g,
+                                                  const uint64_t *__restrict__ keys, const unsigned *__restrict__ cnt,
+                                                  unsigned *hist)
+{
+    __shared__ unsigned h[2 * kFineBins];
+    if (st->bad) return;
+    for (int i = threadIdx.x; i < 2 * kFineBins; i += kFB) h[i] = 0u;
+    __syncthreads();
+    const uint64_t k0 = st->kmin[0], e0 = st->kmax[0], k1 = st->kmin[1], e1 = st->kmax[1];
+    const int s0 = pct_shift(k0, e0), s1 = pct_shift(k1, e1);
+    const int lane = int(threadIdx.x & 63);
+    for (int b = int(blockIdx.x) * (kFB / 64) + int(threadIdx.x >> 6); b < g; b += int(gridDim.x) * (kFB / 64)) {
+        const uint64_t *from = keys + int64_t(b) * R;
+        const int n = int(cnt[b]);
+#pragma unroll 4
+        for (int i = lane; i < n; i += 64) {
+            const uint64_t k = from[i];
+            if (k >= k0 && k <= e0) atomicAdd(&h[(k - k0) >> s0], 1u);
+            if (k >= k1 && k <= e1) atomicAdd(&h[kFineBins + ((k - k1) >> s1)], 1u);
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 2 * kFineBins; i += kFB)
+        if (h[i]) atomicAdd(&hist[i], h[i]);
+}
+
+// One block: the bucket of each rank that lies strictly inside its bracket.
+__global__ __launch_bounds__(kFB) void k_pct_bucket(PctFast *st, const unsigned *__restrict__ hist, int64_t r0,
+                                                    int64_t r1)
+{
+    __shared__ int64_t sums[kFB / 64];
+    if (st->bad) return;
+    constexpr int PER = kFineBins / kFB;
+    const int lane = int(threadIdx.x & 63), w = int(threadIdx.x >> 6);
+    for (int q = 0; q < 2; q++) {
+        int64_t rel;
+        if (pct_place(*st, q, q ? r1 : r0, rel) != 1) continue;  // uniform
+        unsigned h[PER];
+        int64_t mine = 0;
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            h[j] = hist[q * kFineBins + int(threadIdx.x) * PER + j];
+            mine += h[j];
+        }
+        int64_t inc = mine;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int64_t o = __shfl_up(static_cast<long long>(inc), off, 64);
+            if (lane >= off) inc += o;
+        }
+        if (lane == 63) sums[w] = inc;
+        __syncthreads();
+        for (int i = 0; i < w; i++) inc += sums[i];
+        int64_t before = inc - mine;
+        if (rel >= before && rel < inc) {
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                if (rel >= before && rel < before + int64_t(h[j])) {
+                    st->bucket[q] = int(threadIdx.x) * PER + j;
+                    st->rem[q] = rel - before;
+                    st->count[q] = int64_t(h[j]);
+                }
+                before += int64_t(h[j]);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// The keys of each rank's bucket, listed where they fit (kList per rank), else
+// their smallest and largest.  A wave per region, and few blocks: an atomic on
+// one address of device memory takes about 35 ns, so each block gathers in LDS
+// and makes one per rank (one per block of 2048 took 280 us).
+constexpr int kListBlocks = 64;
+__global__ __launch_bounds__(kFB) void k_pct_list(PctFast *st, int64_t R, int g, const uint64_t *__restrict__ keys,
+                                                  const unsigned *__restrict__ cnt, uint64_t *list)
+{
+    constexpr int W = kFB / 64;
+    __shared__ uint64_t buf[2][kList], smn[2][W], smx[2][W];
+    __shared__ int have[2], base[2];
+    if (st->bad) return;
+    const int lane = int(threadIdx.x & 63), w = int(threadIdx.x >> 6);
+    if (threadIdx.x < 2) have[threadIdx.x] = 0;
+    __syncthreads();
+    uint64_t k0[2], k1[2], mn[2] = {~uint64_t(0), ~uint64_t(0)}, mx[2] = {0, 0};
+    int want[2], sh[2];
+    bool fits[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        k0[q] = st->kmin[q];
+        k1[q] = st->kmax[q];
+        want[q] = st->bucket[q];  // -1: matches nothing
+        sh[q] = pct_shift(k0[q], k1[q]);
+        fits[q] = st->count[q] <= kList;
+    }
+    for (int b = int(blockIdx.x) * W + w; b < g; b += int(gridDim.x) * W) {
+        const uint64_t *from = keys + int64_t(b) * R;
+        const int n = int(cnt[b]);
+#pragma unroll 4
+        for (int i = lane; i < n; i += 64) {
+            const uint64_t k = from[i];
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                if (k < k0[q] || k > k1[q] || int((k - k0[q]) >> sh[q]) != want[q]) continue;
+                if (fits[q]) {
+                    buf[q][atomicAdd(&have[q], 1)] = k;  // the whole bucket fits
+                } else {
+                    mn[q] = k < mn[q] ? k : mn[q];
+                    mx[q] = k > mx[q] ? k : mx[q];
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const uint64_t lo = wave_min_u64(mn[q]), hi = wave_max_u64(mx[q]);
+        if (lane == 0) {
+            smn[q][w] = lo;
+            smx[q][w] = hi;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        const int q = int(threadIdx.x);
+        uint64_t lo = ~uint64_t(0), hi = 0;
+        for (int i = 0; i < W; i++) {
+            lo = smn[q][i] < lo ? smn[q][i] : lo;
+            hi = smx[q][i] > hi ? smx[q][i] : hi;
+        }
+        if (lo <= hi) {
+            atomicMin(&st->bmin[q], static_cast<unsigned long long>(lo));
+            atomicMax(&st->bmax[q], static_cast<unsigned long long>(hi));
+        }
+        base[q] = have[q] ? int(atomicAdd(&st->listed[q], unsigned(have[q]))) : 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+        for (int i = threadIdx.x; i < have[q]; i += kFB) list[q * kList + base[q] + i] = buf[q][i];
+}
+
+// One block: each rank's key and its place among the equal keys.  A listed
+// key is the answer when as many keys below it and equal to it surround the
+// rank's place; each lane counts for its own keys, after a histogram over the
+// bucket's width has left the keys of one of its kSub parts.
+__global__ __launch_bounds__(kFB) void k_pct_answer(const PctFast *st, const uint64_t *__restrict__ list, int64_t r0,
+                                                    int64_t r1, PctResult *res, Ticket tk)
+{
+    constexpr int kSubBits = 12, kSub = 1 << kSubBits;
+    __shared__ uint64_t k[kList];
+    __shared__ unsigned sub[kSub], wsum[kFB / 64];
+    __shared__ int left, part, part_before;
+    __shared__ PctResult r;
+    const bool bad = st->bad;
+    if (threadIdx.x == 0) r.err = bad ? 2 : 0;
+    for (int q = 0; q < 2 && !bad; q++) {
+        int64_t rel;
+        const int place = pct_place(*st, q, q ? r1 : r0, rel);
+        if (place == 1 && st->count[q] <= kList) {  // uniform
+            const int all = int(st->count[q]);
+            rel = st->rem[q];
+            const int sh = pct_shift(st->kmin[q], st->kmax[q]), ss = sh > kSubBits ? sh - kSubBits : 0;
+            const uint64_t lo = st->kmin[q] + (uint64_t(st->bucket[q]) << sh);
+            __syncthreads();  // the first rank's LDS has been read
+            for (int i = threadIdx.x; i < kSub; i += kFB) sub[i] = 0u;
+            if (threadIdx.x == 0) left = 0;
+            __syncthreads();
+            for (int i = threadIdx.x; i < all; i += kFB) atomicAdd(&sub[(list[q * kList + i] - lo) >> ss], 1u);
+            __syncthreads();
+            // exclusive prefix over the parts: kSub / kFB per lane
+            unsigned h[kSub / kFB], mine_n = 0u;
+#pragma unroll
+            for (int j = 0; j < kSub / kFB; j++) {
+                h[j] = sub[int(threadIdx.x) * (kSub / kFB) + j];
+                mine_n += h[j];
+            }
+            unsigned inc = mine_n;
+            for (int off = 1; off < 64; off <<= 1) {
+                const unsigned o = __shfl_up(inc, off, 64);
+                if (int(threadIdx.x & 63) >= off) inc += o;
+            }
+            if ((threadIdx.x & 63) == 63) wsum[threadIdx.x >> 6] = inc;
+            __syncthreads();
+            for (int i = 0; i < int(threadIdx.x >> 6); i++) inc += wsum[i];
+            int64_t before = int64_t(inc) - int64_t(mine_n);
+#pragma unroll
+            for (int j = 0; j < kSub / kFB; j++) {
+                if (rel >= before && rel < before + int64_t(h[j])) {  // one lane
+                    part = int(threadIdx.x) * (kSub / kFB) + j;
+                    part_before = int(before);
+                }
+                before += int64_t(h[j]);
+            }
+            __syncthreads();
+            rel -= part_before;
+            for (int i = threadIdx.x; i < all; i += kFB) {
+                const uint64_t key = list[q * kList + i];
+                if (int((key - lo) >> ss) == part) k[atomicAdd(&left, 1)] = key;
+            }
+            __syncthreads();
+            const int m = left;
+            for (int i = threadIdx.x; i < m; i += kFB) {
+                const uint64_t mine = k[i];
+                int less = 0, eq = 0;
+                for (int o = 0; o < m; o++) {
+                    less += k[o] < mine ? 1 : 0;
+                    eq += k[o] == mine ? 1 : 0;
+                }
+                if (rel >= less && rel < less + eq) {  // equal keys write the same
+                    r.key[q] = mine;
+                    r.within[q] = rel - less;
+                }
+            }
+        } else if (threadIdx.x == 0) {
+            if (place == 1) {
+                r.key[q] = st->bmin[q];
+                r.within[q] = st->rem[q];
+                if (st->bmin[q] != st->bmax[q]) r.err = 2;
+            } else if (place >= 0) {
+                r.key[q] = pct_key_bits(static_cast<uint64_t>(__double_as_longlong(place ? st->u[q] : st->l[q])));
+                r.within[q] = rel;
+            } else {
+                r.err = 2;
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        *res = r;
+        publish(tk);
+    }
+}
+
+}  // namespace
+
+// The sampled select (seven launches, one for n <= kSample): 50 M Laplace values
+// with outliers 318 -> 124 us per call at p = 0.001, 451 -> 151 at 0.01, 5 M 181 ->
+// 68, 100 K 94 -> 52, 4096 91 -> 51, against the radix select alone (two full
+// passes of 110 us and 15 short launches).  *done = false: the
+// radix select has to answer.
+static int select_sampled(const double *x, int64_t n, const int64_t r[2], uint64_t key[2], int64_t within[2],
+                          bool *done)
+{
+    *done = false;
+    const bool all = n <= kSample;
+    const int64_t tiles = ceil_div(n, int64_t(kTile));
+    int64_t g = int64_t(num_cus()) * 8;
+    if (g > tiles) g = tiles;
+    // The share of the data that the brackets are expected to hold: 0.5% at p =
+    // 0.0001, 1% at 0.001, 4% at 0.01, 17% at 0.3.  Past kMaxCopies copied keys
+    // a bucket outgrows the list and the call would be made twice (268 M values
+    // at p = 0.01, some of them: 1210 us on average against 1966 for the radix
+    // select; at p = 0.3 2718 against 2102), so the radix select takes it.
+    double held = 0.0;
+    for (int q = 0; q < 2; q++) held += 2.0 * sample_margin((double(r[q]) + 0.5) / double(n)) / kSample;
+    if (!all && held * double(n) > double(kMaxCopies)) return NEURAL_OK;
+    // A block's region: twice its expected copies and two tiles (a run of
+    // matches in sorted data is dealt over the blocks tile by tile).
+    const int64_t share = ceil_div(tiles, g);
+    const int64_t reg = int64_t(double(share) * held * 2.0) + 2;
+    const int64_t R = (reg < share ? reg : share) * kTile;
+    // [state][hist 2 x kFineBins x u32][list 2 x kList x u64][records, counts: g each][keys g x R x u64]
+    const size_t st_b = 512, hist_b = 2 * kFineBins * sizeof(unsigned), list_b = 2 * kList * sizeof(uint64_t);
+    static_assert(sizeof(PctFast) <= 512, "state record");
+    const size_t seen_off = st_b + hist_b + list_b;
+    const size_t keys_off = (seen_off + size_t(g) * (4 * sizeof(double) + 9 * sizeof(unsigned)) + 255) / 256 * 256;
+    char *ws = static_cast<char *>(dev_alloc(all ? st_b : keys_off + size_t(g * R) * sizeof(uint64_t)));
+    if (!ws) return set_error(NEURAL_ERR_OUT_OF_MEMORY);
+    auto *st = reinterpret_cast<PctFast *>(ws);
+    auto *hist = reinterpret_cast<unsigned *>(ws + st_b);
+    auto *list = reinterpret_cast<uint64_t *>(ws + st_b + hist_b);
+    PctSeen seen;
+    auto *sd = reinterpret_cast<double *>(ws + seen_off);
+    auto *su = reinterpret_cast<unsigned *>(sd + 4 * g);
+    for (int q = 0; q < 2; q++) {
+        seen.mn[q] = sd + q * g;
+        seen.mx[q] = sd + (2 + q) * g;
+    }
+    for (int i = 0; i < 8; i++) seen.n[i] = su + i * g;
+    unsigned *cnt = seen.copied = su + 8 * g;
+    auto *keys = reinterpret_cast<uint64_t *>(ws + keys_off);
+    WsGuard wg;
+    auto *res = static_cast<PctResult *>(workspace().host_result_dev);
+    const Ticket tk = next_ticket();
+    NH_LAUNCH(k_pct_sample, dim3(1), dim3(kFB), 0, stream(), x, n, r[0], r[1], st, hist, res, tk);
+    if (!all) {
+        NH_LAUNCH(k_pct_scan, dim3(unsigned(g)), dim3(kPB), 0, stream(), x, n, R, st, keys, seen);
+        NH_LAUNCH(k_pct_fold, dim3(1), dim3(kFB), 0, stream(), st, seen, int(g), R);
+        NH_LAUNCH(k_pct_fine, dim3(unsigned(ceil_div(g, int64_t(kFB / 64)))), dim3(kFB), 0, stream(), st, R, int(g), keys,
+                  cnt, hist);
+        NH_LAUNCH(k_pct_bucket, dim3(1), dim3(kFB), 0, stream(), st, hist, r[0], r[1]);
+        NH_LAUNCH(k_pct_list, dim3(kListBlocks), dim3(kFB), 0, stream(), st, R, int(g), keys, cnt, list);
+        NH_LAUNCH(k_pct_answer, dim3(1), dim3(kFB), 0, stream(), st, list, r[0], r[1], res, tk);
+    }
+    int rc = check_launch();
+    PctResult out{};
+    if (rc == NEURAL_OK) rc = host_result_wait(tk.value, &out, sizeof(out));
+    dev_free(ws);
+    if (rc != NEURAL_OK) return set_error(rc);
+    *done = out.err == 0;
+    for (int q = 0; q < 2; q++) {
+        key[q] = out.key[q];
+        within[q] = out.within[q];
+    }
+    return NEURAL_OK;
+}
+
 // Keys of the elements at ranks r[0], r[1] of the comparator's order, and the
 // rank within its run of equal keys (rank - elements with a smaller key).
 // Eight passes fix the keys a digit at a time, each followed by a one-block
@@ -489,7 +1160,9 @@ static int calibrate_pct(const double *data, int64_t n, double percentile, int s
     const int64_t ranks[2] = {lo_idx, hi_idx};
     uint64_t key[2];
     int64_t within[2];
-    if (select_ranks(x, n, ranks, key, within) != NEURAL_OK) return -1;
+    bool done = false;
+    if (select_sampled(x, n, ranks, key, within, &done) != NEURAL_OK) return -1;
+    if (!done && select_ranks(x, n, ranks, key, within) != NEURAL_OK) return -1;
     double v[2];
     for (int q = 0; q < 2; q++) {
         v[q] = key_value(key[q]);

@@ -426,6 +426,46 @@ def test_calibrate_percentile_full_size_vs_stable_sort(pn):
         assert got.scale == scale
 
 
+@pytest.mark.parametrize("n", [2, 2047, 2048, 2049, 5000, 70_001, 3_000_001])
+def test_calibrate_percentile_sampled_select(pn, n):
+    """Around the size that one block sorts and past it: data whose ranks fall
+    on heavy values (ReLU outputs, few levels: more equal keys in a bucket than
+    are listed), pairs of neighbouring doubles (a full bucket with two keys:
+    the radix select answers), values spanning all exponents, a narrow range,
+    infinities, NaN above everything and around the rank: bit-exact against a
+    stable device sort with the comparator's order."""
+    import torch
+    lib = pn.core._lib
+    rng = np.random.default_rng(n)
+    g = rng.normal(0, 1, n)
+    levels = rng.integers(0, 100, n) / 100.0
+    cases = {"relu": np.maximum(g, 0.0), "levels": levels, "pairs": np.where(rng.random(n) < 0.5, levels,
+                                                                             np.nextafter(levels, 2.0)),
+             "exponents": np.sign(g) * np.exp(rng.uniform(-600, 600, n)), "narrow": 1000.0 + 1e-9 * g,
+             "normal": g, "outliers": np.where(rng.random(n) < 0.001, 1e200 * g, g)}
+    inf = g.copy()
+    inf[rng.random(n) < 0.02] = np.inf
+    inf[rng.random(n) < 0.02] = -np.inf
+    cases["inf"] = inf
+    nan = g.copy()
+    nan[rng.random(n) < 0.0005] = np.nan  # above the upper rank of p = 0.01, around that of p = 0.0005
+    cases["nan"] = nan
+    for name, x in cases.items():
+        xd = torch.from_numpy(x).cuda()
+        srt = torch.sort(xd, stable=True).values.cpu().numpy()  # NaN last
+        torch.cuda.synchronize()
+        for p in (0.0, 0.0005, 0.01, 0.123, 0.4, 0.5):
+            lo, hi = int(n * p), min(n - 1, int(n * (1.0 - p)))
+            if np.isnan(srt[lo]) or np.isnan(srt[hi]) or np.isinf(srt[lo]) or np.isinf(srt[hi]):
+                continue  # the parameters do not hold the two values
+            got = pn.core.QuantParamsC()
+            assert lib.calibrate_percentile(xd.data_ptr(), n, ctypes.c_double(p), 0, ctypes.byref(got)) == 0
+            a, b = srt[lo], srt[hi]
+            if a == b:
+                a, b = a - 0.5, b + 0.5  # the affine epilogue widens a point
+            assert (got.min_val, got.max_val) == (a, b), (name, p, got.min_val, a, got.max_val, b)
+
+
 def test_quantized_matmul_full_size_vs_exact_f64(pn):
     """4096^3 (the size the product is measured at): every inner sum
     sum_k (A - za)(B - zb) is an integer below 2^31 here (|terms| <= 255 * 255,
