@@ -208,13 +208,14 @@ struct BiasPre {
     using V = typename Vec16<T>::type;
     const T *bias;  // [cols]
     T *y;           // this row of the output
-    NH_DEV V load(int64_t i) const { return reinterpret_cast<const V *>(bias)[i]; }
+    using U = typename VecU<T>::type;
+    NH_DEV V load(int64_t i) const { return V(reinterpret_cast<const U *>(bias)[i]); }
     NH_DEV V vec(const V &v, const V &b, int64_t i) const
     {
         V r;
 #pragma unroll
         for (int k = 0; k < Vec16<T>::n; k++) r[k] = v[k] + b[k];
-        st_nt(reinterpret_cast<V *>(y) + i, r);
+        __builtin_nontemporal_store(r, reinterpret_cast<U *>(y) + i);
         return r;
     }
     NH_DEV T one(T x, int64_t j) const
@@ -236,16 +237,16 @@ struct BiasRow {
 // One group of TPR lanes per row, as k_reduce_rows: the row of x is read
 // once, y = x + b written once, and the statistics of y stored.
 template <typename T, int TPR>
-__global__ __launch_bounds__(kRBlock) void k_bias_row_stats(const T *__restrict__ x, const T *__restrict__ bias,
-                                                            T *__restrict__ y, int64_t rows, int64_t cols,
-                                                            RedStats<T> red, bool vec)
+__global__ __launch_bounds__(Grp<TPR>::kBlock) void k_bias_row_stats(const T *__restrict__ x,
+                                                                     const T *__restrict__ bias, T *__restrict__ y,
+                                                                     int64_t rows, int64_t cols, RedStats<T> red)
 {
-    constexpr int RPB = kRBlock / TPR;
+    constexpr int RPB = Grp<TPR>::kBlock / TPR;
     for (int64_t r = int64_t(blockIdx.x) * RPB + threadIdx.x / TPR; r < rows; r += int64_t(gridDim.x) * RPB) {
         const T *xr = x + r * cols;
         const BiasPre<T> pre{bias, y + r * cols};
         T y0 = T(0);  // y[r][0] as lane 0 computed it
-        const typename RedStats<T>::L l = seg_walk<T, RedStats<T>, TPR, true>(red, xr, 0, cols, vec, pre, &y0);
+        const typename RedStats<T>::L l = seg_walk<T, RedStats<T>, TPR, true>(red, xr, 0, cols, pre, &y0);
         const BiasRow<T> row{xr, bias};
         const typename RedStats<T>::B b = red.template finish<TPR>(l, row, 0, cols);
         if (Grp<TPR>::lane() == 0) red.store(nullptr, r, b, FirstOnly<T>{y0}, cols);
@@ -263,14 +264,15 @@ static int row_stats_launch(const T *x, const T *bias, T *y, int64_t rows, int64
     if (!bias) return launch_reduce(x, rows, cols, cols, red, nullptr);
     const ReducePlan plan = reduce_plan<T>(rows, cols);
     if (plan.gx > 1) return NEURAL_ERR_NOT_IMPLEMENTED;  // the caller takes the two-pass route
-    const bool vec = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(bias) |
-                       reinterpret_cast<uintptr_t>(y)) & 15u) == 0 && cols % Vec16<T>::n == 0;
     if (plan.tpr == 64)
         NH_LAUNCH((k_bias_row_stats<T, 64>), dim3(rows_grid(rows, kRBlock / 64)), dim3(kRBlock), 0, stream(), x,
-                  bias, y, rows, cols, red, vec);
+                  bias, y, rows, cols, red);
+    else if (plan.tpr == kRWide)
+        NH_LAUNCH((k_bias_row_stats<T, kRWide>), dim3(rows_grid(rows, 1)), dim3(kRWide), 0, stream(), x, bias, y, rows,
+                  cols, red);
     else
         NH_LAUNCH((k_bias_row_stats<T, kRBlock>), dim3(rows_grid(rows, 1)), dim3(kRBlock), 0, stream(), x, bias,
-                  y, rows, cols, red, vec);
+                  y, rows, cols, red);
     return check_launch();
 }
 

@@ -38,6 +38,7 @@
 namespace nh {
 
 constexpr int kRBlock = 256;
+constexpr int kRWide = 1024;  // lanes of a block that has a whole longer row to itself
 constexpr int kRUnroll = 4;
 
 // ---- generic cross-lane helpers ---------------------------------------------------------
@@ -82,14 +83,15 @@ NH_DEV S dpp_obj(const S &s)
     return r;
 }
 
-// Group of TPR lanes (64 = one wave, 256 = the whole block).  reduce() leaves
+// Group of TPR lanes (64 = one wave, 256 or 1024 = the whole block).  reduce() leaves
 // the same value in every lane of the group: the pairs are fixed and each
 // pair computes comb(a, b) and comb(b, a), equal for commutative comb.  Within
 // a wave: quad swaps (xor 1, xor 2), the half-row and row mirrors as DPP
 // operand moves (no LDS traffic), then lane exchanges across 16 and 32.
 template <int TPR>
 struct Grp {
-    static_assert(TPR == 64 || TPR == kRBlock, "a group is one wave or one block");
+    static_assert(TPR == 64 || TPR == kRBlock || TPR == kRWide, "a group is one wave or one block");
+    static constexpr int kBlock = TPR == 64 ? kRBlock : TPR;  // lanes of a block of such groups
     NH_DEV static int lane() { return int(threadIdx.x) % TPR; }
     template <typename S, typename C>
     NH_DEV static S reduce(S s, C comb)
@@ -103,13 +105,13 @@ struct Grp {
         if constexpr (TPR == 64) {
             return s;
         } else {
-            __shared__ S lds[kRBlock / 64];
+            __shared__ S lds[TPR / 64];
             const int w = threadIdx.x >> 6;
             if ((threadIdx.x & 63) == 0) lds[w] = s;
             __syncthreads();
             S r = lds[0];
 #pragma unroll
-            for (int i = 1; i < kRBlock / 64; i++) r = comb(r, lds[i]);
+            for (int i = 1; i < TPR / 64; i++) r = comb(r, lds[i]);
             __syncthreads();
             return r;
         }
@@ -148,8 +150,11 @@ struct NoPre {
 };
 
 // Walk row elements [lo, hi) with a group of TPR lanes and return the group's
-// combined lane state (the same in every lane of the group).  `vec` promises
-// that row is 16-byte aligned and lo is a multiple of the vector width.  NT:
+// combined lane state (the same in every lane of the group).  lo is a multiple
+// of the vector width; the row may start anywhere (16-byte loads at the
+// element's own alignment: rows of a width that is no multiple of the vector
+// took 4-byte loads, one in flight per lane: bias add and four row reductions
+// [8192, 3001] f32 125 us, now 99; [20000, 1241] 192 -> 99).  NT:
 // the vector loads are non-temporal.  A prologue `pre` (Pre::kActive) maps
 // each loaded vector / element (by its index in the row) before it is reduced;
 // the fused producers use it to compute and store a value and reduce it in the
@@ -158,7 +163,7 @@ struct NoPre {
 // `first` (optional) receives the first value the lane walked: for the
 // group's lane 0 that is element lo (after the prologue).
 template <typename T, class Red, int TPR, bool NT, class Pre = NoPre>
-NH_DEV typename Red::L seg_walk(const Red &red, const T *__restrict__ row, int64_t lo, int64_t hi, bool vec,
+NH_DEV typename Red::L seg_walk(const Red &red, const T *__restrict__ row, int64_t lo, int64_t hi,
                                 const Pre &pre = Pre{}, T *first = nullptr)
 {
     using L = typename Red::L;
@@ -166,48 +171,47 @@ NH_DEV typename Red::L seg_walk(const Red &red, const T *__restrict__ row, int64
     constexpr bool kRel = RelIndex<Red>::value;
     L st = red.linit();
     const int lane = G::lane();
-    int64_t tail = lo;
-    if (vec) {
-        using V = typename Vec16<T>::type;
-        constexpr int VN = Vec16<T>::n;
-        const V *xv = reinterpret_cast<const V *>(row);
-        const int64_t v0 = lo / VN, v1 = hi / VN;
-        for (int64_t c = v0 + lane; c < v1; c += int64_t(TPR) * kRUnroll) {
-            V r[kRUnroll];
-            decltype(pre.load(0)) aux[kRUnroll];
+    using V = typename Vec16<T>::type;
+    constexpr int VN = Vec16<T>::n;
+    using U = typename VecU<T>::type;
+    const U *xv = reinterpret_cast<const U *>(row);
+    // a segment of at most TPR elements: one per lane, one load
+    const int64_t v0 = lo / VN, v1 = hi - lo <= TPR ? v0 : hi / VN;
+    for (int64_t c = v0 + lane; c < v1; c += int64_t(TPR) * kRUnroll) {
+        V r[kRUnroll];
+        decltype(pre.load(0)) aux[kRUnroll];
+#pragma unroll
+        for (int u = 0; u < kRUnroll; u++) {
+            const int64_t i = c + int64_t(u) * TPR;
+            if (i < v1) r[u] = NT ? V(__builtin_nontemporal_load(xv + i)) : V(xv[i]);
+        }
+        if constexpr (Pre::kActive) {
 #pragma unroll
             for (int u = 0; u < kRUnroll; u++) {
                 const int64_t i = c + int64_t(u) * TPR;
-                if (i < v1) r[u] = NT ? ld_nt(xv + i) : xv[i];
+                if (i < v1) aux[u] = pre.load(i);
             }
-            if constexpr (Pre::kActive) {
-#pragma unroll
-                for (int u = 0; u < kRUnroll; u++) {
-                    const int64_t i = c + int64_t(u) * TPR;
-                    if (i < v1) aux[u] = pre.load(i);
-                }
-#pragma unroll
-                for (int u = 0; u < kRUnroll; u++) {
-                    const int64_t i = c + int64_t(u) * TPR;
-                    if (i < v1) r[u] = pre.vec(r[u], aux[u], i);
-                }
-            }
-            if (first && c == v0 + lane) *first = r[0][0];
-            const int32_t rb = kRel ? int32_t(c - v0) * VN : 0;  // lo is a multiple of VN here
 #pragma unroll
             for (int u = 0; u < kRUnroll; u++) {
                 const int64_t i = c + int64_t(u) * TPR;
-                if (i < v1) {
+                if (i < v1) r[u] = pre.vec(r[u], aux[u], i);
+            }
+        }
+        if (first && c == v0 + lane) *first = r[0][0];
+        const int32_t rb = kRel ? int32_t(c - v0) * VN : 0;  // lo is a multiple of VN here
 #pragma unroll
-                    for (int k = 0; k < VN; k++) {
-                        if constexpr (kRel) red.lacc(st, r[u][k], rb + (u * TPR * VN + k));
-                        else red.lacc(st, r[u][k], i * VN + k);
-                    }
+        for (int u = 0; u < kRUnroll; u++) {
+            const int64_t i = c + int64_t(u) * TPR;
+            if (i < v1) {
+#pragma unroll
+                for (int k = 0; k < VN; k++) {
+                    if constexpr (kRel) red.lacc(st, r[u][k], rb + (u * TPR * VN + k));
+                    else red.lacc(st, r[u][k], i * VN + k);
                 }
             }
         }
-        tail = v1 * VN > lo ? v1 * VN : lo;
     }
+    const int64_t tail = v1 * VN > lo ? v1 * VN : lo;
     for (int64_t j = tail + lane; j < hi; j += TPR) {
         const T x = pre.one(row[j], j);
         if (first && j == tail + lane && tail == lo) *first = x;
@@ -218,10 +222,10 @@ NH_DEV typename Red::L seg_walk(const Red &red, const T *__restrict__ row, int64
 
 // Reduce row elements [lo, hi) to the segment summary (`first`: see seg_walk).
 template <typename T, class Red, int TPR, bool NT>
-NH_DEV typename Red::B seg_reduce(const Red &red, const T *__restrict__ row, int64_t lo, int64_t hi, bool vec,
+NH_DEV typename Red::B seg_reduce(const Red &red, const T *__restrict__ row, int64_t lo, int64_t hi,
                                   T *first = nullptr)
 {
-    return red.template finish<TPR>(seg_walk<T, Red, TPR, NT>(red, row, lo, hi, vec, NoPre{}, first), row, lo, hi);
+    return red.template finish<TPR>(seg_walk<T, Red, TPR, NT>(red, row, lo, hi, NoPre{}, first), row, lo, hi);
 }
 
 // Reducers whose store() reads only element 0 of the row (argmax: x0 NaN
@@ -289,12 +293,12 @@ NH_DEV void publish(const Ticket &tk)
     }
 }
 
-// One group (wave or block) per row; RPB = 256 / TPR rows per block.
+// One group (wave or block) per row; a block of waves takes 4 rows.
 template <typename T, class Red, int TPR>
-__global__ __launch_bounds__(kRBlock) void k_reduce_rows(const T *__restrict__ x, int64_t rows, int64_t cols,
-                                                         int64_t ld, Red red, void *out, bool vec, Ticket tk)
+__global__ __launch_bounds__(Grp<TPR>::kBlock) void k_reduce_rows(const T *__restrict__ x, int64_t rows, int64_t cols,
+                                                                  int64_t ld, Red red, void *out, Ticket tk)
 {
-    constexpr int RPB = kRBlock / TPR;
+    constexpr int RPB = Grp<TPR>::kBlock / TPR;
     // rows past the grid (more than kMaxGridBlocks * RPB) are taken in further
     // rounds; r is uniform per group
     for (int64_t r = int64_t(blockIdx.x) * RPB + threadIdx.x / TPR; r < rows; r += int64_t(gridDim.x) * RPB) {
@@ -304,13 +308,13 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_rows(const T *__restrict__ x
         // for the whole sequence than non-temporal ones
         if constexpr (StoreReadsFirst<Red>::value) {
             T x0 = T(0);
-            const typename Red::B b = seg_reduce<T, Red, TPR, false>(red, xr, 0, cols, vec, &x0);
+            const typename Red::B b = seg_reduce<T, Red, TPR, false>(red, xr, 0, cols, &x0);
             if (Grp<TPR>::lane() == 0) {
                 red.store(out, r, b, FirstOnly<T>{x0}, cols);
                 publish(tk);  // tickets are used with a single row only
             }
         } else {
-            const typename Red::B b = seg_reduce<T, Red, TPR, false>(red, xr, 0, cols, vec);
+            const typename Red::B b = seg_reduce<T, Red, TPR, false>(red, xr, 0, cols);
             if (Grp<TPR>::lane() == 0) {
                 red.store(out, r, b, xr, cols);
                 publish(tk);  // tickets are used with a single row only
@@ -324,13 +328,13 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_rows(const T *__restrict__ x
 // kernel boundary before k_reduce_combine publishes the summaries.
 template <typename T, class Red>
 __global__ __launch_bounds__(kRBlock) void k_reduce_seg(const T *__restrict__ x, int64_t cols, int64_t ld,
-                                                        int64_t chunk, Red red, typename Red::B *partials, bool vec)
+                                                        int64_t chunk, Red red, typename Red::B *partials)
 {
     const int64_t r = blockIdx.y;
     const T *xr = x + r * ld;
     const int64_t lo = int64_t(blockIdx.x) * chunk;
     const int64_t hi = lo + chunk < cols ? lo + chunk : cols;
-    const typename Red::B b = seg_reduce<T, Red, kRBlock, true>(red, xr, lo, hi, vec);
+    const typename Red::B b = seg_reduce<T, Red, kRBlock, true>(red, xr, lo, hi);
     if (threadIdx.x == 0) partials[r * int64_t(gridDim.x) + blockIdx.x] = b;
 }
 
@@ -352,8 +356,9 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_combine(const T *__restrict_
 
 // Reduce `rows` rows of `cols` elements (row r at x + r*ld) and store through
 // Red::store into `out` (device memory).  Many rows: one wave (cols <= 2048)
-// or one block per row.  Few long rows: ~4 blocks per CU spread over the rows,
-// each block one contiguous segment of a multiple of 16 KiB, then the
+// or one block per row.  Few rows of up to kWideBytes: a block of 1024 lanes
+// per row, one launch.  Few longer rows: ~4 blocks per CU spread over the
+// rows, each block one contiguous segment of a multiple of 16 KiB, then the
 // one-block-per-row combine.
 //
 // The segment summaries go to the shared workspace (under WsGuard), or to
@@ -376,9 +381,17 @@ ReducePlan reduce_plan(int64_t rows, int64_t cols)
     const int64_t want = int64_t(num_cus()) * 4;  // blocks that keep every CU streaming (measured: 4/CU >= 8/CU here)
     constexpr int64_t kGran = int64_t(kRBlock) * kRUnroll * VN;
     ReducePlan p{1, cols, cols <= 2048 ? 64 : kRBlock};
-    // (a single block per row is slower even for a 512 KiB row: 18.7 us vs
-    // 9.4 us for 32 segments + the combine launch, measured)
-    if (rows < want && cols > 2 * kGran) {
+    // A row of up to kWideBytes keeps a block of 1024 lanes busy for 3-5 us, less
+    // than segments and their second launch take; with more rows than CUs only
+    // where there would be segments ([900, 4096] with the step's four reductions
+    // 21 us with 256 lanes per row, 31 with 1024).  The argmax of a decode step
+    // [64, 32000] 9 -> 5 us; the four of [62, 17600] with the bias add 33.5 ->
+    // 19.5; a whole tensor of 60000 f32,
+    // min and max, 17.0 -> 13.2 us with its quantize and dequantize.
+    constexpr int64_t kWideBytes = 256 << 10;
+    if (rows < want && cols * int64_t(sizeof(T)) <= kWideBytes && cols > (rows <= num_cus() ? 2048 : 2 * kGran)) {
+        p.tpr = kRWide;
+    } else if (rows < want && cols > 2 * kGran) {
         p.gx = ceil_div(want, rows);
         p.chunk = ceil_div(ceil_div(cols, p.gx), kGran) * kGran;
         p.gx = ceil_div(cols, p.chunk);
@@ -406,7 +419,6 @@ int launch_reduce(const T *x, int64_t rows, int64_t cols, int64_t ld, const Red 
     if (tk.slot && rows != 1) return set_error(NEURAL_ERR_INTERNAL);
     static_assert(sizeof(typename Red::B) <= 64, "segment summary must fit a 64-byte partial slot");
     if (rows <= 0 || cols <= 0) return NEURAL_OK;
-    const bool vec = ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) && ((ld * int64_t(sizeof(T))) % 16 == 0);
     const ReducePlan plan = reduce_plan<T>(rows, cols);
     const int64_t gx = plan.gx, chunk = plan.chunk;
     if (RelIndex<Red>::value && chunk >= (int64_t(1) << 31)) return set_error(NEURAL_ERR_TENSOR_TOO_LARGE);
@@ -417,16 +429,18 @@ int launch_reduce(const T *x, int64_t rows, int64_t cols, int64_t ld, const Red 
         if (!scratch) wg.lock();
         auto *part = static_cast<typename Red::B *>(scratch ? scratch : workspace().partials);
         const dim3 grid{unsigned(gx), unsigned(rows), 1u};
-        NH_LAUNCH((k_reduce_seg<T, Red>), grid, dim3(kRBlock), 0, stream(), x, cols, ld, chunk, red, part,
-                           vec);
+        NH_LAUNCH((k_reduce_seg<T, Red>), grid, dim3(kRBlock), 0, stream(), x, cols, ld, chunk, red, part);
         NH_LAUNCH((k_reduce_combine<T, Red>), dim3(unsigned(rows)), dim3(kRBlock), 0, stream(), x, cols, ld,
                            int(gx), red, part, out, tk);
     } else if (plan.tpr == 64) {
         NH_LAUNCH((k_reduce_rows<T, Red, 64>), dim3(rows_grid(rows, kRBlock / 64)), dim3(kRBlock), 0, stream(), x,
-                  rows, cols, ld, red, out, vec, tk);
+                  rows, cols, ld, red, out, tk);
+    } else if (plan.tpr == kRWide) {
+        NH_LAUNCH((k_reduce_rows<T, Red, kRWide>), dim3(rows_grid(rows, 1)), dim3(kRWide), 0, stream(), x, rows, cols,
+                  ld, red, out, tk);
     } else {
         NH_LAUNCH((k_reduce_rows<T, Red, kRBlock>), dim3(rows_grid(rows, 1)), dim3(kRBlock), 0, stream(), x, rows,
-                  cols, ld, red, out, vec, tk);
+                  cols, ld, red, out, tk);
     }
     return check_launch();
 }

@@ -268,3 +268,58 @@ def test_colsum_edges(pn, dt, cols):
                 assert np.all(np.abs(out.numpy() - e / rows) <= bound / rows), (rows, off)
     finally:
         pn.set_stream(None)
+
+
+@pytest.mark.parametrize("cols", [1, 3, 63, 64, 65, 67, 255, 257, 1023, 2047, 2048, 2049, 8193, 32768, 32770, 65536, 65541])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_row_reductions_unaligned_edges(pn, ora, dt, cols):
+    """Row sum, max and argmax at the edges of the row plans (one element per
+    lane, a wave, a block of 256 or 1024 lanes, segments), rows and buffers that
+    start inside a vector; the fused statistics, with and without a bias add,
+    equal bit for bit."""
+    import torch
+    lib = pn.core._lib
+    rng = np.random.default_rng(cols)
+    T = torch.float32 if dt == np.float32 else torch.float64
+    D = pn.float32 if dt == np.float32 else pn.float64
+    tol = 1e-6 if dt == np.float32 else 1e-13
+    pn.set_stream(torch.cuda.current_stream().cuda_stream)
+    try:
+        for rows, off in ((1, 0), (3, 1), (5, 0), (300, 1)):
+            if rows * cols > 4_000_000:
+                continue
+            x = rng.normal(0, 3, (rows, cols)).astype(dt)
+            x[0, cols - 1] = 50.0  # the last element the maximum of one row
+            if cols > 8:
+                x[rows - 1, cols // 2] = np.nan
+            buf = torch.zeros(rows * cols + 3, dtype=T, device="cuda")
+            v = buf[off:off + rows * cols].view(rows, cols)
+            v.copy_(torch.from_numpy(x))
+            t = pn.Tensor.from_torch(v)
+            s, mx, s2, me2, mx2 = (pn.Tensor.create([rows], D) for _ in range(5))
+            at, at2 = np.empty(rows, np.int64), np.empty(rows, np.int64)
+            assert lib.neural_reduce_sum(t._ptr, 1, s._ptr) == 0
+            assert lib.neural_reduce_max(t._ptr, 1, mx._ptr) == 0
+            assert lib.neural_reduce_argmax(t._ptr, 1, at.ctypes.data) == 0
+            e, mag = x.astype(np.float64).sum(axis=1), np.abs(x.astype(np.float64)).sum(axis=1)
+            ok = ~np.isnan(e)
+            assert np.all(np.abs(s.numpy()[ok] - e[ok]) <= tol * mag[ok]) and np.array_equal(np.isnan(s.numpy()), ~ok)
+            same_bits(mx.numpy(), ora.rowmax_chain(x))
+            same_bits(at, ora.rowargmax(x))
+            assert lib.neural_row_stats(t._ptr, s2._ptr, me2._ptr, mx2._ptr, at2.ctypes.data) == 0
+            for a, b in ((s, s2), (mx, mx2)):
+                same_bits(a.numpy(), b.numpy())
+            same_bits(at, at2)
+            bias = rng.normal(0, 1, cols).astype(dt)
+            tb, y = pn.Tensor.from_numpy(bias), pn.Tensor.create([rows, cols], D)
+            assert lib.neural_bias_add_row_stats(y._ptr, t._ptr, tb._ptr, s2._ptr, me2._ptr, mx2._ptr,
+                                                 at2.ctypes.data) == 0
+            same_bits(y.numpy(), x + bias)
+            assert lib.neural_reduce_sum(y._ptr, 1, s._ptr) == 0
+            assert lib.neural_reduce_max(y._ptr, 1, mx._ptr) == 0
+            assert lib.neural_reduce_argmax(y._ptr, 1, at.ctypes.data) == 0
+            for a, b in ((s, s2), (mx, mx2)):
+                same_bits(a.numpy(), b.numpy())
+            same_bits(at, at2)
+    finally:
+        pn.set_stream(None)
