@@ -106,7 +106,10 @@ struct Workspace {
     void         *result;      // 256 bytes of small results
     void         *host_result; // 256 bytes of coherent pinned host memory (host address)
     void         *host_result_dev; // the same bytes as kernels address them
+    void         *host_small;      // kSmallD2H bytes of coherent pinned host memory
+    void         *host_small_dev;  // (device_to_host), and as kernels address them
 };
+constexpr size_t kSmallD2H = size_t(16) << 10;
 constexpr int kMaxPartials = 16384;
 constexpr int kCounters = 1024;
 Workspace   &workspace();
@@ -214,6 +217,12 @@ struct Ticket {
 };
 Ticket       next_ticket();
 int          host_result_wait(unsigned long long ticket, void *dst, size_t bytes);
+// Copy device bytes to the host, done on return.  Up to kSmallD2H bytes one
+// block stores them into pinned host memory with a ticket; more take a copy
+// command and a stream wait, as all sizes did.  Tensor.numpy() whole, copy
+// command -> ticket: 4 B 23.6 -> 12.8 us, 4 KiB 23.2 -> 13.3, 16 KiB 23.7 ->
+// 17.1; at 32 KiB the copy command is the faster one (11.6 against 17.6).
+int          device_to_host(void *dst, const void *src, size_t bytes);
 
 }  // namespace nh
 

@@ -116,6 +116,8 @@ int ensure_init()
                 hipMalloc(&r.ws.result, 256) != hipSuccess ||
                 hipHostMalloc(&r.ws.host_result, 256, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
                 hipHostGetDevicePointer(&r.ws.host_result_dev, r.ws.host_result, 0) != hipSuccess ||
+                hipHostMalloc(&r.ws.host_small, kSmallD2H, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
+                hipHostGetDevicePointer(&r.ws.host_small_dev, r.ws.host_small, 0) != hipSuccess ||
                 std::memset(r.ws.host_result, 0, 256) == nullptr ||
                 hipMemset(r.ws.counter, 0, sizeof(unsigned) * kCounters) != hipSuccess ||
                 hipMemset(r.ws.result, 0, 256) != hipSuccess ||
@@ -245,28 +247,71 @@ Ticket next_ticket()
     return t;
 }
 
-int host_result_wait(unsigned long long ticket, void *dst, size_t bytes)
+// Until the ticket shows in host memory.
+static int wait_ticket(unsigned long long ticket)
 {
-    if (bytes > kTicketOffset) return set_error(NEURAL_ERR_INTERNAL);
-    const char *area = static_cast<const char *>(workspace().host_result);
-    const volatile unsigned long long *word =
-        reinterpret_cast<const volatile unsigned long long *>(area + kTicketOffset);
+    const volatile unsigned long long *word = reinterpret_cast<const volatile unsigned long long *>(
+        static_cast<const char *>(workspace().host_result) + kTicketOffset);
     // Spin on the ticket for a while (a kernel that ends normally stores it
     // within microseconds of finishing), then fall back to the stream wait,
     // which also surfaces a fault.
-    bool seen = false;
     for (long spins = 0; spins < (1L << 26); spins++) {
-        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == ticket) {
-            seen = true;
-            break;
-        }
+        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == ticket) return NEURAL_OK;
         __builtin_ia32_pause();
     }
-    if (!seen) {
-        NH_TRY(sync());
-        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != ticket) return set_error(NEURAL_ERR_INTERNAL);
+    NH_TRY(sync());
+    return __atomic_load_n(word, __ATOMIC_ACQUIRE) == ticket ? NEURAL_OK : set_error(NEURAL_ERR_INTERNAL);
+}
+
+int host_result_wait(unsigned long long ticket, void *dst, size_t bytes)
+{
+    if (bytes > kTicketOffset) return set_error(NEURAL_ERR_INTERNAL);
+    NH_TRY(wait_ticket(ticket));
+    std::memcpy(dst, workspace().host_result, bytes);
+    return NEURAL_OK;
+}
+
+// One block: `bytes` of device memory into mapped host memory, then the
+// ticket.  Bound by the link and the wait; 16 bytes per lane where src allows.
+__global__ __launch_bounds__(1024) void k_to_host(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst,
+                                                  unsigned bytes, Ticket tk)
+{
+    const uintptr_t a = reinterpret_cast<uintptr_t>(src);
+    unsigned done = 0;
+    if ((a & 15) == 0) {
+        for (unsigned i = threadIdx.x; i < bytes / 16; i += 1024)
+            reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+        done = bytes & ~15u;
+    } else if ((a & 3) == 0) {
+        for (unsigned i = threadIdx.x; i < bytes / 4; i += 1024)
+            reinterpret_cast<uint32_t *>(dst)[i] = reinterpret_cast<const uint32_t *>(src)[i];
+        done = bytes & ~3u;
     }
-    std::memcpy(dst, area, bytes);
+    for (unsigned i = done + threadIdx.x; i < bytes; i += 1024) dst[i] = src[i];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence_system();
+        __hip_atomic_store(tk.slot, tk.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+int device_to_host(void *dst, const void *src, size_t bytes)
+{
+    if (bytes == 0) return NEURAL_OK;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    // No result can come back while the stream records: the copy and wait refuse it.
+    if (bytes > kSmallD2H || hipStreamIsCapturing(stream(), &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        NH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream()));
+        return sync();
+    }
+    WsGuard wg;
+    const Ticket tk = next_ticket();
+    NH_LAUNCH(k_to_host, dim3(1), dim3(1024), 0, stream(), static_cast<const uint8_t *>(src),
+              static_cast<uint8_t *>(workspace().host_small_dev), unsigned(bytes), tk);
+    NH_TRY(check_launch());
+    NH_TRY(wait_ticket(tk.value));
+    std::memcpy(dst, workspace().host_small, bytes);
     return NEURAL_OK;
 }
 
@@ -359,16 +404,15 @@ int Staged::finish(bool download)
     // A mirror-backed output was written on the device; the caller may read
     // it through the host pointer, so the written range goes back there too
     // (the storage keeps its state: SYNCED stays in sync, DEVICE stays ahead).
-    if ((owned || mirror) && download && bytes)
-        NH_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream()));
+    const bool back = (owned || mirror) && download && bytes;
+    if (back) NH_TRY(device_to_host(host, dev, bytes));
     if (mirror) {
-        if (download && bytes) NH_TRY(sync());
         mirror = nullptr;
         dev = nullptr;
         return NEURAL_OK;
     }
     if (owned) {
-        NH_TRY(sync());
+        if (!back) NH_TRY(sync());
         dev_free(dev);
         dev = nullptr;
         owned = false;
@@ -430,10 +474,7 @@ static int download_span(Storage *s)
 {
     const int64_t span = s->hi - s->lo;
     if (span <= 0) return NEURAL_OK;
-    char *host0 = static_cast<char *>(s->host) + s->lo;
-    NH_HIP(hipMemcpyAsync(host0, s->dev_block, size_t(span), hipMemcpyDeviceToHost, stream()));
-    NH_TRY(sync());
-    return NEURAL_OK;
+    return device_to_host(static_cast<char *>(s->host) + s->lo, s->dev_block, size_t(span));
 }
 
 int dev_read(const NeuralTensor *t, const void **p)
@@ -976,8 +1017,12 @@ int neural_tensor_download(NeuralTensor *t, void *host_dst, uint64_t bytes)
     if (bytes != neural_tensor_bytes(t) || !nh::is_contiguous(t)) return set_error(NEURAL_ERR_SHAPE_MISMATCH);
     const void *s = nullptr;
     NH_TRY(dev_read(t, &s));
-    NH_HIP(hipMemcpyAsync(host_dst, s, bytes, hipMemcpyDeviceToHost, stream()));
-    NH_TRY(sync());
+    if (is_device_ptr(host_dst)) {
+        NH_HIP(hipMemcpyAsync(host_dst, s, bytes, hipMemcpyDeviceToHost, stream()));
+        NH_TRY(sync());
+    } else {
+        NH_TRY(device_to_host(host_dst, s, bytes));
+    }
     return set_error(NEURAL_OK);
 }
 

@@ -109,6 +109,42 @@ def test_torch_stream_interop(pn):
         pn.set_stream(None)
 
 
+@pytest.mark.parametrize("nbytes", [4, 12, 16, 20, 4092, 16380, 16384, 16388, 65536])
+def test_small_results_to_host(pn, rng, nbytes):
+    """Results of up to 16 KiB come back through pinned host memory, larger
+    ones by a copy command: whole tensors, the host mirror, and ranges at
+    every alignment, with the bytes beside them left alone."""
+    lib = pn.core._lib
+    n = nbytes // 4
+    for step in range(3):  # the pinned buffer is reused: no result is the last one's
+        x = rng.normal(size=n).astype(np.float32)
+        t = pn.Tensor.from_numpy(x)
+        y = t + t
+        same_bits(y.numpy(), x + x)
+        same_bits(np.array(y.numpy_zero_copy()), x + x)
+    for dt in (np.float32, np.float64):
+        z = rng.normal(size=nbytes // np.dtype(dt).itemsize + 1).astype(dt)
+        same_bits(pn.Tensor.from_numpy(z).numpy(), z)
+    # an f32 range that starts 4 bytes into a mirror
+    c = pn.Tensor.from_numpy(np.full(n + 2, 7.0, dtype=np.float32))
+    pc = lib.neural_tensor_data(c._ptr)
+    assert lib.simd_add_f32(pc + 4, x.ctypes.data, x.ctypes.data, n) == 0
+    want = np.concatenate([[np.float32(7)], x + x, [np.float32(7)]])
+    same_bits(np.ctypeslib.as_array(ctypes.cast(pc, ctypes.POINTER(ctypes.c_float)), shape=(n + 2,)).copy(), want)
+    same_bits(c.numpy(), want)
+    # bytes: host memory, and a mirror at an odd byte
+    prm = pn.core.QuantParamsC()
+    if lib.calibrate_minmax_f32(x.ctypes.data, n, 1, ctypes.byref(prm)) == 0:
+        q = np.empty(n, dtype=np.int8)
+        assert lib.quantize_tensor_f32(x.ctypes.data, q.ctypes.data, n, ctypes.byref(prm)) == 0
+        m = pn.Tensor.zeros([n])
+        pm = lib.neural_tensor_data(m._ptr)
+        assert lib.quantize_tensor_f32(x.ctypes.data, pm + 1, n, ctypes.byref(prm)) == 0
+        raw = np.frombuffer(ctypes.string_at(pm, 4 * n), dtype=np.int8)
+        same_bits(raw[1:n + 1], q)
+        assert raw[0] == 0 and not raw[n + 1:].any()
+
+
 def test_raw_pointer_into_tensor_mirror(pn):
     """The reference's Python hands neural_tensor_data() pointers to the
     raw-pointer entry points (training.py:43-79).  Such a pointer resolves to
