@@ -109,7 +109,7 @@ struct Workspace {
     void         *host_small;      // kSmallD2H bytes of coherent pinned host memory
     void         *host_small_dev;  // (device_to_host), and as kernels address them
 };
-constexpr size_t kSmallD2H = size_t(16) << 10;
+constexpr size_t kSmallD2H = size_t(64) << 10;
 constexpr int kMaxPartials = 16384;
 constexpr int kCounters = 1024;
 Workspace   &workspace();
@@ -219,9 +219,14 @@ Ticket       next_ticket();
 int          host_result_wait(unsigned long long ticket, void *dst, size_t bytes);
 // Copy device bytes to the host, done on return.  Up to kSmallD2H bytes one
 // block stores them into pinned host memory with a ticket; more take a copy
-// command and a stream wait, as all sizes did.  Tensor.numpy() whole, copy
-// command -> ticket: 4 B 23.6 -> 12.8 us, 4 KiB 23.2 -> 13.3, 16 KiB 23.7 ->
-// 17.1; at 32 KiB the copy command is the faster one (11.6 against 17.6).
+// command and a stream wait, as all sizes did.  An add and its numpy(), copy
+// command -> ticket: 1 KiB 30.9 -> 20.6 us, 16 KiB 31.0 -> 22.7, 24 KiB 27.5 ->
+// 23.5, 64 KiB 30.0 -> 27.2; at 128 KiB one block's stores leave 33.5 -> 31.7
+// of it.  A copy command also has to retire every launch since the last
+// stream wait, which tickets do not: after a request of some ten launches
+// whose other results came back by ticket, 32000 bytes took 44 us by the copy
+// command and 16.4 by ticket (a limit of 16 KiB left that request at 124 us,
+// now 79).
 int          device_to_host(void *dst, const void *src, size_t bytes);
 
 }  // namespace nh

@@ -109,9 +109,9 @@ def test_torch_stream_interop(pn):
         pn.set_stream(None)
 
 
-@pytest.mark.parametrize("nbytes", [4, 12, 16, 20, 4092, 16380, 16384, 16388, 65536])
+@pytest.mark.parametrize("nbytes", [4, 12, 16, 20, 4092, 16380, 16384, 16388, 65532, 65536, 65540, 131072])
 def test_small_results_to_host(pn, rng, nbytes):
-    """Results of up to 16 KiB come back through pinned host memory, larger
+    """Results of up to 64 KiB come back through pinned host memory, larger
     ones by a copy command: whole tensors, the host mirror, and ranges at
     every alignment, with the bytes beside them left alone."""
     lib = pn.core._lib
