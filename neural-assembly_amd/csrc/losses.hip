@@ -127,7 +127,7 @@ NH_DEV double ce_diff(T x, double m)
 }
 
 // One row per group of NT lanes, VPT 16-byte vectors per lane and the values
-// before and after the vectors in one scalar of the first lanes (RowCut; the
+// past the vectors in one scalar of the first lanes (RowCut; the
 // other lanes' scalar is -inf and adds nothing).  FULL: the row is exactly NT * VPT vectors, so no
 // element needs a bounds check (per-element checks around the exp turn into
 // exec-mask branches).  The lane that
@@ -138,8 +138,12 @@ NH_DEV double ce_diff(T x, double m)
 // vectors for each of 512 lanes: 16 in registers and LV = 9 in LDS (72 KB; a
 // lane reads and writes its own slots only), two blocks per CU.  With all 25
 // in registers the compiler spilled 35-84 of them to scratch memory
-// ([4096, 50257] fused f32 373 us against 318; three passes of 4-byte
-// accesses took 861).
+// ([4096, 50257] fused f32 373 us against 318, both with stores cut at 64-byte
+// boundaries; three passes of 4-byte accesses took 861).  Rows of an odd width
+// start anywhere, and a vector store that starts inside a 64-byte block is
+// slower: 340 us there, 315 with each row cut at the first boundary of its own
+// gradient.  But then the order of a row's sums, and so the result's last
+// bits, went by the buffer's address; equal bits are promised.
 //
 // WAVES: the minimum waves per SIMD the compiler must fit (1: its own
 // choice).  The f64 forward with rows of up to 1024 values takes 5 (83-84
@@ -178,15 +182,15 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
     const int64_t cols = a.cols;
     const T *xr = x + r * cols;
     T *gr = GRAD ? static_cast<T *>(a.grad) + r * cols : nullptr;
-    const RowCut<T, (NT >= 64)> cut(gr, cols);
-    const int nsc = FULL ? 0 : cut.nsc(), head = FULL ? 0 : cut.head;
+    const RowCut<T> cut(cols);
+    const int nsc = FULL ? 0 : cut.rem;
     const auto in_row = [&](int k) { return FULL || lane + k * NT < cut.ncv; };
     // the target first: its load overlaps the row's instead of following the reductions
     int64_t t = 0;
     const bool ok = loss_target(a.tidx, static_cast<const T *>(a.tval), r, cols, t);
     V v[VPT], w[LV > 0 ? LV : 1];
     T vt = -inf_t<T>();
-    const U *xv = reinterpret_cast<const U *>(xr + head);
+    const U *xv = reinterpret_cast<const U *>(xr);
 #pragma unroll
     for (int k = 0; k < VPT; k++)
         if (in_row(k)) v[k] = __builtin_nontemporal_load(xv + lane + k * NT);
@@ -195,8 +199,8 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
         if (in_row(VPT + k)) w[k] = __builtin_nontemporal_load(xv + lane + (VPT + k) * NT);
     if (lane < nsc) vt = xr[cut.sc(lane)];
     // the target's vector and slot, or the scalar that holds it (-1: neither)
-    const bool t_vec = ok && t >= head && t - head < int64_t(FULL ? NT * VPT : cut.ncv) * VN;
-    const int tv = t_vec ? int((t - head) / VN) : -1, tj = int((t - head) % VN);
+    const bool t_vec = ok && t < int64_t(FULL ? NT * VPT : cut.ncv) * VN;
+    const int tv = t_vec ? int(t / VN) : -1, tj = int(t % VN);
     const bool t_mine = ok && !t_vec && lane < nsc && cut.sc(lane) == t;  // in this lane's scalar
     const auto at = [&](const V &q) {  // q[tj]
         T x = q[0];
@@ -291,7 +295,7 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
                 for (int j = 0; j < VN; j++)
                     if (j == tj) g[j] = grad(q[j], true);
             }
-            __builtin_nontemporal_store(g, reinterpret_cast<U *>(gr + head) + lane + k * NT);
+            __builtin_nontemporal_store(g, reinterpret_cast<U *>(gr) + lane + k * NT);
         };
 #pragma unroll
         for (int k = 0; k < VPT; k++)
@@ -447,7 +451,7 @@ static void launch_ce_rows(const T *x, const CeArgs &a)
 // the width was no multiple of the vector, then three passes) -> now, us,
 // smoothed fused form with its summing launches:
 //   f32 [65536, 10] 32.1 -> 10.7, [32768, 256] 24.3 -> 19.2, [30000, 1001] 84.3 -> 49.0, [65536, 1024] 93.2 -> 89.9
-//       [8192, 3000] 107 -> 43.5, [4096, 8192] 115 -> 52.4, [2048, 32000] 267 -> 104, [4096, 50257] 861 -> 317
+//       [8192, 3000] 107 -> 43.5, [4096, 8192] 115 -> 52.4, [2048, 32000] 267 -> 104, [4096, 50257] 861 -> 340
 //       [600, 98000] 517 -> 110, [500, 131072] 682 -> 134 (two reads)
 //   f64 [65536, 10] 33.7 -> 14.3, [30000, 1001] 104 -> 92, [4096, 8553] 203 -> 110, [2000, 24001] 332 -> 167
 template <typename T, int MODE>

@@ -66,28 +66,16 @@ struct RowGrp {
 // 95.0 / 93.9 / 89.9 / 91.6 us.
 constexpr unsigned kFullRowsLds = 40000;
 
-// How a row of `cols` values is cut for a group of NT lanes: `head` values up to
-// the first 64-byte boundary of the row that is written, ncv vectors, `rem`
-// values past them; lane l < nsc() holds value sc(l) as a scalar.  Vector
-// stores that start inside a 64-byte block ran 12% slower (64 M f32 copy, 99.7
-// against 88 us whatever the offset inside the block; loads do not mind).
-// HEAD = false (groups without lanes or work to spare): head = 0.
-template <typename T, bool HEAD>
+// How a row of `cols` values is cut: ncv vectors from its first value, `rem`
+// values past them; lane l < rem holds value sc(l) as a scalar.  The cut goes
+// by index alone: which lane holds a value, and so the order of the row's
+// sums, does not depend on where the row lies in memory.
+template <typename T>
 struct RowCut {
     static constexpr int VN = Vec16<T>::n;
-    int head, ncv, rem;
-    NH_DEV RowCut(const void *written, int64_t cols)
-    {
-        head = 0;
-        if constexpr (HEAD) {
-            const int h = int((64 - (reinterpret_cast<uintptr_t>(written) & 63)) & 63) / int(sizeof(T));
-            head = h < cols ? h : int(cols);
-        }
-        ncv = int((cols - head) / VN);
-        rem = int((cols - head) % VN);
-    }
-    NH_DEV int nsc() const { return head + rem; }
-    NH_DEV int64_t sc(int lane) const { return lane < head ? lane : int64_t(ncv) * VN + lane; }
+    int ncv, rem;
+    NH_DEV explicit RowCut(int64_t cols) : ncv(int(cols / VN)), rem(int(cols % VN)) {}
+    NH_DEV int64_t sc(int lane) const { return int64_t(ncv) * VN + lane; }
 };
 
 }  // namespace nh

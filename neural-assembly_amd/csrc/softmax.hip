@@ -61,7 +61,7 @@ NH_DEV T row_out(T v, double md, double lse, double s, double rs)
 }
 
 // One row per group of NT lanes, held in VPT vectors per lane (and the values
-// before and after the vectors in one scalar of the first lanes, see RowCut;
+// past the vectors in one scalar of the first lanes, see RowCut;
 // the other lanes' scalar is -inf, which adds 0 to the sum, or NaN where the
 // row is NaN anyway).  FULL: the
 // row is exactly NT * VPT vectors, so no element needs a bounds check.
@@ -87,14 +87,14 @@ __global__ __launch_bounds__(NT < kSmBlock ? kSmBlock : NT, NT == 512 ? 4 : 1) v
     if (RPB > 1 && r >= rows) return;  // uniform per group; a block of one row has one
     const T *xr = x + r * cols;
     T *yr = y + r * cols;
-    const RowCut<T, (NT >= 256)> cut(yr, cols);  // in a wave the head costs what it saves: [55392, 577] 45.0 -> 46.7 us
-    const int nsc = FULL ? 0 : cut.nsc(), head = FULL ? 0 : cut.head;
+    const RowCut<T> cut(cols);
+    const int nsc = FULL ? 0 : cut.rem;
     const auto in_row = [&](int k) { return FULL || lane + k * NT < cut.ncv; };
     V v[VPT];
     T vt = neg_inf<T>();
 #pragma unroll
     for (int k = 0; k < VPT; k++)
-        if (in_row(k)) v[k] = __builtin_nontemporal_load(reinterpret_cast<const U *>(xr + head) + lane + k * NT);
+        if (in_row(k)) v[k] = __builtin_nontemporal_load(reinterpret_cast<const U *>(xr) + lane + k * NT);
     if (lane < nsc) vt = xr[cut.sc(lane)];
 
     T m = vt == vt ? vt : neg_inf<T>();
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(NT < kSmBlock ? kSmBlock : NT, NT == 512 ? 4 : 1) v
             V o;
 #pragma unroll
             for (int j = 0; j < VN; j++) o[j] = row_out<T, LOG>(v[k][j], md, lse, s, rs);
-            __builtin_nontemporal_store(o, reinterpret_cast<U *>(yr + head) + lane + k * NT);
+            __builtin_nontemporal_store(o, reinterpret_cast<U *>(yr) + lane + k * NT);
         }
     }
     if (lane < nsc) yr[cut.sc(lane)] = row_out<T, LOG>(vt, md, lse, s, rs);

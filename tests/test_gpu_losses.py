@@ -378,3 +378,43 @@ def test_row_kernel_edges(pn, dt, k):
         assert np.isnan(loss.item()) and bool((G[1] == 7.0).all()) and not bool((G[0] == 7.0).any())
     finally:
         pn.set_stream(None)
+
+
+@pytest.mark.parametrize("k", [257, 513, 1001, 4099, 8193, 33001, 98311])
+@pytest.mark.parametrize("dt", ["float64", "float32"])
+def test_bits_do_not_depend_on_the_address(pn, dt, k):
+    """Loss and gradient bits of the _dev form, whatever element the gradient
+    starts at, equal the host-returning form's (whose gradient is staged in a
+    block of its own) and, in f64, the backward's; equal rows have equal
+    gradients, though rows of an odd width start at different addresses."""
+    import torch
+    lib = pn.core._lib
+    T = getattr(torch, dt)
+    n, a, f64 = 5, 0.1, dt == "float64"
+    rng = np.random.default_rng(k)
+    x = np.repeat(rng.normal(0, 3, (1, k)), n, axis=0).astype(dt)
+    t = np.full(n, k // 3, dtype=np.int64)
+    bits = np.int64 if f64 else np.int32
+    host_g, host_loss = np.empty((n, k), dtype=dt), ctypes.c_double()
+    fused = lib.label_smoothing_ce_fused if f64 else lib.label_smoothing_ce_fused_f32
+    assert fused(x.ctypes.data, t.ctypes.data, n, k, a, ctypes.byref(host_loss), host_g.ctypes.data) == 0
+    for r in range(1, n):
+        assert np.array_equal(host_g[0].view(bits), host_g[r].view(bits))
+    dev = lib.label_smoothing_ce_fused_dev if f64 else lib.label_smoothing_ce_fused_f32_dev
+    pn.set_stream(torch.cuda.current_stream().cuda_stream)
+    try:
+        tt = torch.from_numpy(t).cuda()
+        loss = torch.zeros((), dtype=torch.float64, device="cuda")
+        for oi, og in ((0, 0), (0, 1), (1, 3), (3, 0), (2, 7)):
+            bx, bg = (torch.zeros(n * k + 8, dtype=T, device="cuda") for _ in range(2))
+            X, G = bx[oi:oi + n * k], bg[og:og + n * k]
+            X.copy_(torch.from_numpy(x).flatten())
+            assert dev(X.data_ptr(), tt.data_ptr(), n, k, a, loss.data_ptr(), G.data_ptr()) == 0
+            assert np.array_equal(G.cpu().numpy().view(bits), host_g.ravel().view(bits)), (oi, og)
+            assert loss.item() == host_loss.value
+            if f64:
+                G.zero_()
+                assert lib.label_smoothing_ce_backward(X.data_ptr(), tt.data_ptr(), n, k, a, G.data_ptr()) == 0
+                assert np.array_equal(G.cpu().numpy().view(bits), host_g.ravel().view(bits)), (oi, og)
+    finally:
+        pn.set_stream(None)

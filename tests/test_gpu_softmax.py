@@ -201,3 +201,28 @@ def test_timed_launch(pn):
         lib.neural_hip_reset_stream()
         for e in ev:
             hip.hipEventDestroy(e)
+
+
+@pytest.mark.parametrize("cols", [577, 4099, 8191, 33001, 51203, 98301, 98311])
+@pytest.mark.parametrize("dt", ["float32", "float64"])
+def test_bits_do_not_depend_on_the_address(pn, dt, cols):
+    """Equal rows have equal outputs, wherever the input and output start."""
+    import torch
+    T = getattr(torch, dt)
+    cols = cols if dt == "float32" else (cols + 1) // 2 | 1
+    g = torch.Generator().manual_seed(cols)
+    row = (torch.randn((1, cols), generator=g, dtype=torch.float64) * 3).to(T).cuda()
+    bits = torch.int32 if dt == "float32" else torch.int64
+    pn.set_stream(torch.cuda.current_stream().cuda_stream)
+    try:
+        for f in (pn.core._lib.neural_softmax, pn.core._lib.neural_log_softmax):
+            first = None
+            for oi, oo in ((0, 0), (1, 3), (3, 2)):
+                x, y = (torch.zeros(5 * cols + 8, dtype=T, device="cuda") for _ in range(2))
+                X, Y = x[oi:oi + 5 * cols].view(5, cols), y[oo:oo + 5 * cols].view(5, cols)
+                X.copy_(row.expand(5, cols))
+                assert f(pn.Tensor.from_torch(Y)._ptr, pn.Tensor.from_torch(X)._ptr) == 0
+                first = Y[0].clone() if first is None else first
+                assert torch.equal(Y.contiguous().view(bits), first.view(bits).expand(5, cols)), (oi, oo)
+    finally:
+        pn.set_stream(None)
