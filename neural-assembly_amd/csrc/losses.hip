@@ -446,7 +446,9 @@ static void launch_ce_rows(const T *x, const CeArgs &a)
     });
 }
 
-// The smallest group whose registers hold the row (as launch_softmax).  Before
+// The smallest group whose registers hold the row (as launch_softmax).  A wave
+// ends at exactly 4096 f32 / 2048 f64 values, without the few more that its
+// scalars would hold: wider rows form every term in double (WIDE).  Before
 // (a wave per row up to 4096 f32 / 2048 f64 values, element by element where
 // the width was no multiple of the vector, then three passes) -> now, us,
 // smoothed fused form with its summing launches:
@@ -464,7 +466,7 @@ static int launch_ce(const T *x, const CeArgs &a)
     else if (ncv <= 64 * 2) launch_ce_rows<T, MODE, 64, 2>(x, a);
     else if (ncv <= 64 * 4) launch_ce_rows<T, MODE, 64, 4>(x, a);
     else if (ncv <= 64 * 8) launch_ce_rows<T, MODE, 64, 8>(x, a);
-    else if (ncv <= 64 * 16) launch_ce_rows<T, MODE, 64, 16>(x, a);
+    else if (a.cols <= 64 * 16 * Vec16<T>::n) launch_ce_rows<T, MODE, 64, 16>(x, a);
     else if (ncv <= 256 * 8) launch_ce_rows<T, MODE, 256, 8>(x, a);
     else if (ncv <= 256 * 16) launch_ce_rows<T, MODE, 256, 16>(x, a);
     else if (ncv <= 512 * 16) launch_ce_rows<T, MODE, 512, 16>(x, a);

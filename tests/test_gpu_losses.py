@@ -418,3 +418,47 @@ def test_bits_do_not_depend_on_the_address(pn, dt, k):
                 assert np.array_equal(G.cpu().numpy().view(bits), host_g.ravel().view(bits)), (oi, og)
     finally:
         pn.set_stream(None)
+
+
+@pytest.mark.parametrize("k", [4097, 4098, 4099, 4100, 8193])
+def test_wide_f32_rows_round_once(pn, k):
+    """Rows of more than 4096 f32 classes form the gradient in double and round
+    once.  Equal logits make every e exactly 1 and the sum exactly k, so only
+    that forming is left: (1/n) (1/k - st) in double, rounded to float, where
+    float arithmetic loses the digits that cancel (smoothing 0.9)."""
+    import torch
+    lib = pn.core._lib
+    n, a = 3, 0.9
+    x = torch.full((n, k), 1.25, dtype=torch.float32, device="cuda")
+    g, loss = torch.zeros_like(x), torch.zeros((), dtype=torch.float64, device="cuda")
+    t = torch.tensor([0, k // 2, k - 1], device="cuda")
+    torch.cuda.synchronize()
+    assert lib.label_smoothing_ce_fused_f32_dev(x.data_ptr(), t.data_ptr(), n, k, a, loss.data_ptr(), g.data_ptr()) == 0
+    pn.synchronize()
+    st = np.full((n, k), a / k)
+    st[np.arange(n), t.cpu().numpy()] += 1.0 - a
+    want = ((1.0 / n) * (1.0 / k - st)).astype(np.float32)
+    got = g.cpu().numpy()
+    # double forming: 2^-24 of the value and what double rounding leaves of the cancelled terms
+    assert np.all(np.abs(got.astype(np.float64) - want) <= 2.0 ** -23 * np.abs(want))
+
+
+@pytest.mark.parametrize("k", [2049, 2050, 2051])
+def test_wide_f64_forward_exp(pn, k):
+    """Past 2048 f64 classes the forward takes the library's exp, as the fused
+    form does, and not the table's (about 3 ulp): the same loss bits.  One row
+    a call, two classes that count (loss = log(1 + e^y)), so that a last bit of
+    e^y shows."""
+    import torch
+    lib = pn.core._lib
+    tt = torch.zeros(1, dtype=torch.int64, device="cuda")
+    xt = torch.full((1, k), -800.0, dtype=torch.float64, device="cuda")
+    g = torch.empty_like(xt)
+    fwd, fused = ctypes.c_double(), ctypes.c_double()
+    for y in np.linspace(-1.0, -0.01, 100):
+        xt[0, 0], xt[0, k // 2] = 0.0, y
+        torch.cuda.synchronize()
+        assert lib.label_smoothing_ce_forward(xt.data_ptr(), tt.data_ptr(), 1, k, 0.0, ctypes.byref(fwd)) == 0
+        assert lib.label_smoothing_ce_fused(xt.data_ptr(), tt.data_ptr(), 1, k, 0.0, ctypes.byref(fused),
+                                            g.data_ptr()) == 0
+        assert fwd.value == fused.value, y
