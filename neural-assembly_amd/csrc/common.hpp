@@ -197,6 +197,9 @@ void for_row_launches(int64_t rows, int64_t rpb, L launch)
 }
 int          check_launch();                         // hipGetLastError -> error code
 int          sync();                                 // synchronise the active stream
+// The active stream is being captured (or cannot be asked): no result of its
+// launches can come back to the host, so nothing may wait for a ticket.
+bool         stream_recording();
 // Copy `bytes` (<= 256) of a device result to `dst` (host): one D2H copy into
 // the pinned landing area, a stream sync, then a host memcpy.
 int          result_to_host(void *dst, const void *dev_src, size_t bytes);

@@ -1176,6 +1176,10 @@ static int calibrate_pct(const double *data, int64_t n, double percentile, int s
     if (percentile != percentile) return -1;
     if (percentile < 0.0 || percentile > 0.5) percentile = 0.01;
     if (ensure_init() != NEURAL_OK) return -1;
+    if (stream_recording()) {  // the result cannot come back: refused before anything is recorded
+        set_error(NEURAL_ERR_INTERNAL);
+        return -1;
+    }
     int64_t lo_idx = int64_t(double(n) * percentile);
     int64_t hi_idx = int64_t(double(n) * (1.0 - percentile));
     if (lo_idx < 0) lo_idx = 0;

@@ -225,6 +225,14 @@ int sync()
     return NEURAL_OK;
 }
 
+bool stream_recording()
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream(), &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 int host_result_fetch(void *dst, size_t bytes)
 {
     WsGuard wg;
@@ -299,9 +307,8 @@ __global__ __launch_bounds__(1024) void k_to_host(const uint8_t *__restrict__ sr
 int device_to_host(void *dst, const void *src, size_t bytes)
 {
     if (bytes == 0) return NEURAL_OK;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    // No result can come back while the stream records: the copy and wait refuse it.
-    if (bytes > kSmallD2H || hipStreamIsCapturing(stream(), &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+    // While the stream records the copy and wait refuse the call.
+    if (bytes > kSmallD2H || stream_recording()) {
         NH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream()));
         return sync();
     }

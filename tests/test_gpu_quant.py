@@ -489,3 +489,39 @@ def test_quantized_matmul_full_size_vs_exact_f64(pn):
     exact = torch.matmul(a.double() - pa.zero_point, (b.double() - pb.zero_point).contiguous())
     want = exact * (pa.scale * pb.scale)
     assert torch.equal(c, want)
+
+
+def test_calibrate_percentile_refused_while_recording(pn):
+    """A call whose result goes to the host is refused at once while the stream
+    is being captured (it does not wait for a result that cannot come), and
+    the library works afterwards."""
+    import time
+    import torch
+    lib = pn.core._lib
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipStreamBeginCapture.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    hip.hipStreamEndCapture.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    x = torch.from_numpy(np.random.default_rng(5).normal(0, 1, 100_000)).cuda()
+    got, want = pn.core.QuantParamsC(), pn.core.QuantParamsC()
+    args = (x.data_ptr(), x.numel(), ctypes.c_double(0.01), 0)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    pn.set_stream(s.cuda_stream)
+    try:
+        assert lib.calibrate_percentile(*args, ctypes.byref(want)) == 0  # scratch is at hand below
+        s.synchronize()
+        assert hip.hipStreamBeginCapture(s.cuda_stream, 2) == 0  # relaxed
+        t = time.perf_counter()
+        rc = lib.calibrate_percentile(*args, ctypes.byref(got))
+        took = time.perf_counter() - t
+        graph = ctypes.c_void_p()
+        ended = hip.hipStreamEndCapture(s.cuda_stream, ctypes.byref(graph))
+        assert rc == -1 and lib.neural_get_last_error() == pn.NeuralError.INTERNAL
+        assert ended == 0 and graph.value  # nothing that breaks the recording either
+        hip.hipGraphDestroy.argtypes = [ctypes.c_void_p]
+        assert hip.hipGraphDestroy(graph) == 0
+        assert took < 0.2, took  # the spin on a ticket takes seconds
+    finally:
+        pn.set_stream(None)
+    assert lib.calibrate_percentile(*args, ctypes.byref(got)) == 0
+    assert (got.min_val, got.max_val) == (want.min_val, want.max_val)
