@@ -106,8 +106,8 @@ struct Workspace {
     void         *result;      // 256 bytes of small results
     void         *host_result; // 256 bytes of coherent pinned host memory (host address)
     void         *host_result_dev; // the same bytes as kernels address them
-    void         *host_small;      // kSmallD2H bytes of coherent pinned host memory
-    void         *host_small_dev;  // (device_to_host), and as kernels address them
+    void         *host_small;      // kSmallD2H bytes of coherent pinned host memory and a ticket
+    void         *host_small_dev;  // word after them (device_to_host), and as kernels address them
 };
 constexpr size_t kSmallD2H = size_t(64) << 10;
 constexpr int kMaxPartials = 16384;
@@ -229,7 +229,9 @@ int          host_result_wait(unsigned long long ticket, void *dst, size_t bytes
 // stream wait, which tickets do not: after a request of some ten launches
 // whose other results came back by ticket, 32000 bytes took 44 us by the copy
 // command and 16.4 by ticket (a limit of 16 KiB left that request at 124 us,
-// now 79).
+// now 79).  The pinned bytes and their ticket have a lock of their own, so that
+// a wait here holds up no other thread's launches; a thread that finds them
+// taken uses the copy command.
 int          device_to_host(void *dst, const void *src, size_t bytes);
 
 }  // namespace nh

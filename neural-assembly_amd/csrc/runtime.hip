@@ -116,9 +116,11 @@ int ensure_init()
                 hipMalloc(&r.ws.result, 256) != hipSuccess ||
                 hipHostMalloc(&r.ws.host_result, 256, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
                 hipHostGetDevicePointer(&r.ws.host_result_dev, r.ws.host_result, 0) != hipSuccess ||
-                hipHostMalloc(&r.ws.host_small, kSmallD2H, hipHostMallocCoherent | hipHostMallocMapped) != hipSuccess ||
+                hipHostMalloc(&r.ws.host_small, kSmallD2H + 64, hipHostMallocCoherent | hipHostMallocMapped) !=
+                    hipSuccess ||
                 hipHostGetDevicePointer(&r.ws.host_small_dev, r.ws.host_small, 0) != hipSuccess ||
                 std::memset(r.ws.host_result, 0, 256) == nullptr ||
+                std::memset(r.ws.host_small, 0, kSmallD2H + 64) == nullptr ||
                 hipMemset(r.ws.counter, 0, sizeof(unsigned) * kCounters) != hipSuccess ||
                 hipMemset(r.ws.result, 0, 256) != hipSuccess ||
                 hipDeviceSynchronize() != hipSuccess) {
@@ -245,6 +247,8 @@ int host_result_fetch(void *dst, size_t bytes)
 namespace {
 constexpr size_t kTicketOffset = 248;  // last 8 bytes of the 256-byte host result area
 unsigned long long g_ticket = 0;       // last ticket handed out (under WsGuard)
+std::mutex g_small_mu;                 // host_small, from a download's launch to the host's copy of it
+unsigned long long g_small_ticket = 0; // last ticket of host_small (under g_small_mu)
 }  // namespace
 
 Ticket next_ticket()
@@ -255,11 +259,10 @@ Ticket next_ticket()
     return t;
 }
 
-// Until the ticket shows in host memory.
-static int wait_ticket(unsigned long long ticket)
+// Until the ticket shows in the host word at p.
+static int wait_ticket(const void *p, unsigned long long ticket)
 {
-    const volatile unsigned long long *word = reinterpret_cast<const volatile unsigned long long *>(
-        static_cast<const char *>(workspace().host_result) + kTicketOffset);
+    const volatile unsigned long long *word = static_cast<const volatile unsigned long long *>(p);
     // Spin on the ticket for a while (a kernel that ends normally stores it
     // within microseconds of finishing), then fall back to the stream wait,
     // which also surfaces a fault.
@@ -274,7 +277,7 @@ static int wait_ticket(unsigned long long ticket)
 int host_result_wait(unsigned long long ticket, void *dst, size_t bytes)
 {
     if (bytes > kTicketOffset) return set_error(NEURAL_ERR_INTERNAL);
-    NH_TRY(wait_ticket(ticket));
+    NH_TRY(wait_ticket(static_cast<const char *>(workspace().host_result) + kTicketOffset, ticket));
     std::memcpy(dst, workspace().host_result, bytes);
     return NEURAL_OK;
 }
@@ -307,18 +310,21 @@ __global__ __launch_bounds__(1024) void k_to_host(const uint8_t *__restrict__ sr
 int device_to_host(void *dst, const void *src, size_t bytes)
 {
     if (bytes == 0) return NEURAL_OK;
+    std::unique_lock<std::mutex> mine(g_small_mu, std::defer_lock);
     // While the stream records the copy and wait refuse the call.
-    if (bytes > kSmallD2H || stream_recording()) {
+    if (bytes > kSmallD2H || stream_recording() || !mine.try_lock()) {
         NH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream()));
         return sync();
     }
-    WsGuard wg;
-    const Ticket tk = next_ticket();
+    Workspace &ws = workspace();
+    Ticket tk;
+    tk.slot = reinterpret_cast<unsigned long long *>(static_cast<char *>(ws.host_small_dev) + kSmallD2H);
+    tk.value = ++g_small_ticket;
     NH_LAUNCH(k_to_host, dim3(1), dim3(1024), 0, stream(), static_cast<const uint8_t *>(src),
-              static_cast<uint8_t *>(workspace().host_small_dev), unsigned(bytes), tk);
+              static_cast<uint8_t *>(ws.host_small_dev), unsigned(bytes), tk);
     NH_TRY(check_launch());
-    NH_TRY(wait_ticket(tk.value));
-    std::memcpy(dst, workspace().host_small, bytes);
+    NH_TRY(wait_ticket(static_cast<const char *>(ws.host_small) + kSmallD2H, tk.value));
+    std::memcpy(dst, ws.host_small, bytes);
     return NEURAL_OK;
 }
 

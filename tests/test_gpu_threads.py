@@ -88,3 +88,40 @@ def test_two_threads_share_the_workspace(pn):
     assert not any(t.is_alive() for t in th), "a worker thread did not finish"
     assert not bad, bad[:5]
     assert not bad_err, bad_err[:5]
+
+
+def test_waiting_download_holds_up_no_launch(pn):
+    """While one thread waits for a small result behind a long queue, another
+    thread's calls that only enqueue (here a reduction whose partials lie in
+    the shared workspace) return at once, and its own download is right."""
+    import time
+
+    import torch
+    lib = pn.core._lib
+    big = pn.Tensor.create([1 << 26], dtype=pn.float64)
+    rows = pn.Tensor.from_numpy(np.ones((2, 1 << 20), dtype=np.float32))
+    out = pn.Tensor.create([2])
+    small = pn.Tensor.from_numpy(np.arange(8, dtype=np.float32))
+    assert lib.neural_reduce_sum(rows._ptr, 1, out._ptr) == 0
+    out.numpy()
+    for _ in range(3000):  # about half a second of work
+        assert lib.neural_gelu(big._ptr, big._ptr) == 0
+    y = small + small
+    done = []
+
+    def wait():
+        done.append((y.numpy().copy(), time.perf_counter()))
+
+    th = threading.Thread(target=wait)
+    th.start()
+    time.sleep(0.03)
+    t0 = time.perf_counter()
+    assert lib.neural_reduce_sum(rows._ptr, 1, out._ptr) == 0
+    took = time.perf_counter() - t0
+    waiting = not done
+    got = out.numpy()
+    th.join()
+    assert took < 0.02, took
+    assert waiting, "the queue was too short to tell"
+    assert np.array_equal(got, np.full(2, 1 << 20, dtype=np.float32))
+    assert np.array_equal(done[0][0], np.arange(8, dtype=np.float32) * 2)
