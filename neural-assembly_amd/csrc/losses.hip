@@ -486,6 +486,7 @@ static int launch_ce(const T *x, const CeArgs &a)
 // the host makes otherwise.
 template <bool F32>
 struct RedCeLoss {
+    static constexpr bool kCostly = true;
     using L = double;
     using B = double;
     double div = 0.0;
@@ -509,6 +510,7 @@ struct RedCeLoss {
 // and s_r = sum_c exp(x_c - m); its loss is log(s_r) * S - A_r with
 // S = sum_c st_c = st0 (cols - 1) + st1.  div as in RedCeLoss.
 struct RedLsLoss {
+    static constexpr bool kCostly = true;
     using L = double;
     using B = double;
     const double *s;

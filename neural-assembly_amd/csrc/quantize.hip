@@ -94,6 +94,7 @@ struct RedMinMax {
 struct QErrOut { double sig, noise; };
 template <typename T>
 struct RedQErr {
+    static constexpr bool kCostly = true;
     using L = QErrOut;
     using B = QErrOut;
     double inv, scale;

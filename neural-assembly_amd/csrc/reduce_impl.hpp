@@ -375,7 +375,7 @@ struct ReducePlan {
 };
 
 template <typename T>
-ReducePlan reduce_plan(int64_t rows, int64_t cols)
+ReducePlan reduce_plan(int64_t rows, int64_t cols, bool costly = false)
 {
     constexpr int VN = Vec16<T>::n;
     const int64_t want = int64_t(num_cus()) * 4;  // blocks that keep every CU streaming (measured: 4/CU >= 8/CU here)
@@ -388,8 +388,12 @@ ReducePlan reduce_plan(int64_t rows, int64_t cols)
     // [64, 32000] 9 -> 5 us; the four of [62, 17600] with the bias add 33.5 ->
     // 19.5; a whole tensor of 60000 f32,
     // min and max, 17.0 -> 13.2 us with its quantize and dequantize.
+    // Not for reducers that compute a function per element (costly): over 32768
+    // double logarithms one CU takes 18 us longer than segments do (tensor loss
+    // f32 [32768, 512] 43 us against 25; quantization error of 65536 values 24
+    // against 12.6).
     constexpr int64_t kWideBytes = 256 << 10;
-    if (rows < want && cols * int64_t(sizeof(T)) <= kWideBytes && cols > (rows <= num_cus() ? 2048 : 2 * kGran)) {
+    if (!costly && rows < want && cols * int64_t(sizeof(T)) <= kWideBytes && cols > (rows <= num_cus() ? 2048 : 2 * kGran)) {
         p.tpr = kRWide;
     } else if (rows < want && cols > 2 * kGran) {
         p.gx = ceil_div(want, rows);
@@ -405,6 +409,13 @@ ReducePlan reduce_plan(int64_t rows, int64_t cols)
     return p;
 }
 
+// Reducers whose lacc() evaluates a function per element (a logarithm, a value
+// quantized and back) declare kCostly.
+template <class Red, typename = void> struct CostlyElem { static constexpr bool value = false; };
+template <class Red> struct CostlyElem<Red, std::void_t<decltype(Red::kCostly)>> {
+    static constexpr bool value = Red::kCostly;
+};
+
 // Blocks of a row-per-group launch (rpb rows per block), capped at kMaxGridBlocks.
 inline unsigned rows_grid(int64_t rows, int rpb)
 {
@@ -419,7 +430,7 @@ int launch_reduce(const T *x, int64_t rows, int64_t cols, int64_t ld, const Red 
     if (tk.slot && rows != 1) return set_error(NEURAL_ERR_INTERNAL);
     static_assert(sizeof(typename Red::B) <= 64, "segment summary must fit a 64-byte partial slot");
     if (rows <= 0 || cols <= 0) return NEURAL_OK;
-    const ReducePlan plan = reduce_plan<T>(rows, cols);
+    const ReducePlan plan = reduce_plan<T>(rows, cols, CostlyElem<Red>::value);
     const int64_t gx = plan.gx, chunk = plan.chunk;
     if (RelIndex<Red>::value && chunk >= (int64_t(1) << 31)) return set_error(NEURAL_ERR_TENSOR_TOO_LARGE);
     if (gx > 1) {
@@ -435,9 +446,10 @@ int launch_reduce(const T *x, int64_t rows, int64_t cols, int64_t ld, const Red 
     } else if (plan.tpr == 64) {
         NH_LAUNCH((k_reduce_rows<T, Red, 64>), dim3(rows_grid(rows, kRBlock / 64)), dim3(kRBlock), 0, stream(), x,
                   rows, cols, ld, red, out, tk);
-    } else if (plan.tpr == kRWide) {
-        NH_LAUNCH((k_reduce_rows<T, Red, kRWide>), dim3(rows_grid(rows, 1)), dim3(kRWide), 0, stream(), x, rows, cols,
-                  ld, red, out, tk);
+    } else if (!CostlyElem<Red>::value && plan.tpr == kRWide) {
+        if constexpr (!CostlyElem<Red>::value)
+            NH_LAUNCH((k_reduce_rows<T, Red, kRWide>), dim3(rows_grid(rows, 1)), dim3(kRWide), 0, stream(), x, rows,
+                      cols, ld, red, out, tk);
     } else {
         NH_LAUNCH((k_reduce_rows<T, Red, kRBlock>), dim3(rows_grid(rows, 1)), dim3(kRBlock), 0, stream(), x, rows,
                   cols, ld, red, out, tk);

@@ -19,7 +19,7 @@ import math
 import numpy as np
 import pytest
 
-from conftest import GPU, rel_close
+from conftest import GPU, rel_close, same_bits
 
 pytestmark = GPU
 
@@ -236,7 +236,6 @@ def test_ls_ce_loss_left_in_device_memory(pn, k):
     queue without waiting; a target out of range gives a NaN loss and does
     not reach the next host-returning call; argument errors return -1."""
     torch = pytest.importorskip("torch")
-    from conftest import same_bits
     lib = pn.core._lib
     b = 4096
     x, t = _case(b, k, 91)  # finite logits: a NaN loss below can only come from the bad target
@@ -462,3 +461,39 @@ def test_wide_f64_forward_exp(pn, k):
         assert lib.label_smoothing_ce_fused(xt.data_ptr(), tt.data_ptr(), 1, k, 0.0, ctypes.byref(fused),
                                             g.data_ptr()) == 0
         assert fwd.value == fused.value, y
+
+
+@pytest.mark.parametrize("b", [2048, 2049, 4096, 4097, 8191, 32768, 32769])
+def test_loss_sum_over_batches(pn, b):
+    """The mean over the rows' losses at the batch sizes where the summing pass
+    changes form (a wave, a block, segments); the _dev form gives the same
+    bits.  Bounds: those of the module."""
+    import torch
+    lib = pn.core._lib
+    k, a = 5, 0.1
+    x, t = _case(b, k, b)
+    xt, tt = torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda()
+    g, dev = torch.empty_like(xt), torch.zeros(2, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    fwd, fused, ce = (ctypes.c_double() for _ in range(3))
+    args = (xt.data_ptr(), tt.data_ptr(), b, k, a)
+    assert lib.label_smoothing_ce_forward(*args, ctypes.byref(fwd)) == 0
+    assert lib.label_smoothing_ce_fused(*args, ctypes.byref(fused), g.data_ptr()) == 0
+    assert lib.label_smoothing_ce_forward_dev(*args, dev.data_ptr()) == 0
+    assert lib.label_smoothing_ce_fused_dev(*args, dev.data_ptr() + 8, g.data_ptr()) == 0
+    pn.synchronize()
+    same_bits(dev.cpu().numpy(), np.array([fwd.value, fused.value]))
+    lsm = x - x.max(axis=1, keepdims=True)
+    lsm -= np.log(np.exp(lsm).sum(axis=1, keepdims=True))
+    st = np.full((b, k), a / k)
+    st[np.arange(b), t] += 1 - a
+    want = -(st * lsm).sum() / b
+    for got in (fwd.value, fused.value):
+        assert abs(got - want) <= 1e-12 * _bound(x, t, a)
+    for dt, rel, floor in ((np.float64, 1e-12, 0.0), (np.float32, 2e-6, 2e-7)):
+        tx, tv = pn.Tensor.from_numpy(x.astype(dt)), pn.Tensor.from_numpy(t.astype(dt))
+        assert lib.neural_cross_entropy_loss(tx._ptr, tv._ptr, ctypes.byref(ce)) == 0
+        x64 = x.astype(dt).astype(np.float64)
+        p = np.exp(x64 - x64.max(axis=1, keepdims=True))
+        want_ce = np.mean(-np.log((p / p.sum(axis=1, keepdims=True))[np.arange(b), t] + 1e-7))
+        assert abs(ce.value - want_ce) <= rel * abs(want_ce) + floor
