@@ -2,7 +2,7 @@
 //
 // Every reduction here is a reduction of R rows of C elements (a whole tensor
 // is one row).  A row is split into contiguous segments; each segment is
-// reduced by one group of lanes (a wave64 or a 256-lane block):
+// reduced by one group of lanes (a wave64, or a block of 256 or 1024 lanes):
 //
 //   lanes     walk the segment in 128-bit vectors (U vectors in flight per
 //             lane), keeping a small lane state in the input's own precision
@@ -355,11 +355,11 @@ __global__ __launch_bounds__(kRBlock) void k_reduce_combine(const T *__restrict_
 // ---- launch policy --------------------------------------------------------------------------
 
 // Reduce `rows` rows of `cols` elements (row r at x + r*ld) and store through
-// Red::store into `out` (device memory).  Many rows: one wave (cols <= 2048)
-// or one block per row.  Few rows of up to kWideBytes: a block of 1024 lanes
-// per row, one launch.  Few longer rows: ~4 blocks per CU spread over the
-// rows, each block one contiguous segment of a multiple of 16 KiB, then the
-// one-block-per-row combine.
+// Red::store into `out` (device memory).  Many rows, or few of up to
+// kWideBytes: one wave (cols <= 2048) or one block per row, of 1024 lanes for
+// up to as many long rows as CUs.  Few longer rows: ~4 blocks per CU spread
+// over the rows, each block one contiguous segment of a multiple of 16 KiB,
+// then the one-block-per-row combine.
 //
 // The segment summaries go to the shared workspace (under WsGuard), or to
 // `scratch` (scratch_bytes long) when the caller brings its own buffer; a
@@ -381,20 +381,23 @@ ReducePlan reduce_plan(int64_t rows, int64_t cols, bool costly = false)
     const int64_t want = int64_t(num_cus()) * 4;  // blocks that keep every CU streaming (measured: 4/CU >= 8/CU here)
     constexpr int64_t kGran = int64_t(kRBlock) * kRUnroll * VN;
     ReducePlan p{1, cols, cols <= 2048 ? 64 : kRBlock};
-    // A row of up to kWideBytes keeps a block of 1024 lanes busy for 3-5 us, less
-    // than segments and their second launch take; with more rows than CUs only
-    // where there would be segments ([900, 4096] with the step's four reductions
-    // 21 us with 256 lanes per row, 31 with 1024).  The argmax of a decode step
-    // [64, 32000] 9 -> 5 us; the four of [62, 17600] with the bias add 33.5 ->
-    // 19.5; a whole tensor of 60000 f32,
-    // min and max, 17.0 -> 13.2 us with its quantize and dequantize.
+    // Few rows of up to kWideBytes, past the width that 256 lanes read in two
+    // rounds: one launch, less than segments and their second launch take.  Up
+    // to a row per CU a block of 1024 lanes each (argmax of a decode step
+    // [64, 32000] 9 -> 5 us; bias add and four reductions [62, 17600] 33.5 -> 19.5;
+    // a whole tensor of 60000 f32, min and max, 17.0 -> 13.2 us with its quantize
+    // and dequantize); narrower rows gain nothing from it (statistics of
+    // [128, 4096] 3.7 us with 256 lanes, 4.6 with 1024).  With more rows than CUs
+    // the usual 256 lanes, several blocks to a CU: row statistics f32
+    // [838, 20000] 12.6 us, with 1024 lanes, one block to a CU in a fourth round,
+    // 21.3, in segments 16.5; the sum alone 11.2 / 11.8 / 12.5.
     // Not for reducers that compute a function per element (costly): over 32768
     // double logarithms one CU takes 18 us longer than segments do (tensor loss
     // f32 [32768, 512] 43 us against 25; quantization error of 65536 values 24
     // against 12.6).
     constexpr int64_t kWideBytes = 256 << 10;
-    if (!costly && rows < want && cols * int64_t(sizeof(T)) <= kWideBytes && cols > (rows <= num_cus() ? 2048 : 2 * kGran)) {
-        p.tpr = kRWide;
+    if (!costly && rows < want && cols * int64_t(sizeof(T)) <= kWideBytes && cols > 2 * kGran) {
+        if (rows <= num_cus()) p.tpr = kRWide;
     } else if (rows < want && cols > 2 * kGran) {
         p.gx = ceil_div(want, rows);
         p.chunk = ceil_div(ceil_div(cols, p.gx), kGran) * kGran;

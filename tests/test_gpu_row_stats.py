@@ -200,3 +200,11 @@ def test_tensor_methods(pn):
     want = _separate(pn, pn.Tensor.from_numpy(x + b), 64)
     for got, w in zip([s.numpy(), m.numpy(), mx.numpy(), idx], want):
         same_bits(got, w)
+
+
+@pytest.mark.parametrize("rows,cols", [(256, 8193), (257, 8192), (257, 8193), (257, 4097), (1023, 8193), (300, 32769)])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_long_rows_around_a_row_per_cu(pn, ora, rows, cols, dt):
+    """Long rows up to and past one per CU (blocks of 1024 or of 256 lanes)."""
+    test_row_stats_equal_separate_calls(pn, ora, rows, cols, dt)
+    test_bias_add_row_stats_equal_separate_calls(pn, ora, rows, cols, dt)
