@@ -236,7 +236,7 @@ struct BiasRow {
 
 // One group of TPR lanes per row, as k_reduce_rows: the row of x is read
 // once, y = x + b written once, and the statistics of y stored.
-template <typename T, int TPR>
+template <typename T, int TPR, int NARROW = 0>
 __global__ __launch_bounds__(Grp<TPR>::kBlock) void k_bias_row_stats(const T *__restrict__ x,
                                                                      const T *__restrict__ bias, T *__restrict__ y,
                                                                      int64_t rows, int64_t cols, RedStats<T> red)
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(Grp<TPR>::kBlock) void k_bias_row_stats(const T *__
         const T *xr = x + r * cols;
         const BiasPre<T> pre{bias, y + r * cols};
         T y0 = T(0);  // y[r][0] as lane 0 computed it
-        const typename RedStats<T>::L l = seg_walk<T, RedStats<T>, TPR, true>(red, xr, 0, cols, pre, &y0);
+        const typename RedStats<T>::L l = seg_walk<T, RedStats<T>, TPR, true, NARROW>(red, xr, 0, cols, pre, &y0);
         const BiasRow<T> row{xr, bias};
         const typename RedStats<T>::B b = red.template finish<TPR>(l, row, 0, cols);
         if (Grp<TPR>::lane() == 0) red.store(nullptr, r, b, FirstOnly<T>{y0}, cols);
@@ -264,7 +264,13 @@ static int row_stats_launch(const T *x, const T *bias, T *y, int64_t rows, int64
     if (!bias) return launch_reduce(x, rows, cols, cols, red, nullptr);
     const ReducePlan plan = reduce_plan<T>(rows, cols);
     if (plan.gx > 1) return NEURAL_ERR_NOT_IMPLEMENTED;  // the caller takes the two-pass route
-    if (plan.tpr == 64)
+    if (plan.tpr == 64 && narrow_of<T>(cols) == 2)
+        NH_LAUNCH((k_bias_row_stats<T, 64, 2>), dim3(rows_grid(rows, kRBlock / 64)), dim3(kRBlock), 0, stream(), x,
+                  bias, y, rows, cols, red);
+    else if (plan.tpr == 64 && narrow_of<T>(cols) == 4)
+        NH_LAUNCH((k_bias_row_stats<T, 64, 4>), dim3(rows_grid(rows, kRBlock / 64)), dim3(kRBlock), 0, stream(), x,
+                  bias, y, rows, cols, red);
+    else if (plan.tpr == 64)
         NH_LAUNCH((k_bias_row_stats<T, 64>), dim3(rows_grid(rows, kRBlock / 64)), dim3(kRBlock), 0, stream(), x,
                   bias, y, rows, cols, red);
     else if (plan.tpr == kRWide)

@@ -40,6 +40,16 @@ namespace nh {
 constexpr int kRBlock = 256;
 constexpr int kRWide = 1024;  // lanes of a block that has a whole longer row to itself
 constexpr int kRUnroll = 4;
+// Scalars per lane of a wave for rows of up to 128 and of up to 256 elements
+// (seg_walk's NARROW form); 0: vectors.  Even f64 rows past 192 fill three
+// quarters of the lanes with vectors: row statistics [65536, 256] 23.3 us, 24.6 in
+// scalars ([65536, 255] 27.4 and 25.4).
+template <typename T>
+inline int narrow_of(int64_t cols)
+{
+    if (sizeof(T) == 8 && cols > 3 * 64 && cols % 2 == 0) return 0;
+    return cols <= 2 * 64 ? 2 : cols <= 4 * 64 ? 4 : 0;
+}
 
 // ---- generic cross-lane helpers ---------------------------------------------------------
 
@@ -154,7 +164,8 @@ struct NoPre {
 // of the vector width; the row may start anywhere (16-byte loads at the
 // element's own alignment: rows of a width that is no multiple of the vector
 // took 4-byte loads, one in flight per lane: bias add and four row reductions
-// [8192, 3001] f32 125 us, now 99; [20000, 1241] 192 -> 99).  NT:
+// [8192, 3001] f32 125 us, now 99; [20000, 1241] 192 -> 99).  NARROW: the
+// segment has at most NARROW * TPR elements, read as scalars (0: any size).  NT:
 // the vector loads are non-temporal.  A prologue `pre` (Pre::kActive) maps
 // each loaded vector / element (by its index in the row) before it is reduced;
 // the fused producers use it to compute and store a value and reduce it in the
@@ -162,7 +173,7 @@ struct NoPre {
 // reduction accumulates exactly what the stand-alone one does.
 // `first` (optional) receives the first value the lane walked: for the
 // group's lane 0 that is element lo (after the prologue).
-template <typename T, class Red, int TPR, bool NT, class Pre = NoPre>
+template <typename T, class Red, int TPR, bool NT, int NARROW = 0, class Pre = NoPre>
 NH_DEV typename Red::L seg_walk(const Red &red, const T *__restrict__ row, int64_t lo, int64_t hi,
                                 const Pre &pre = Pre{}, T *first = nullptr)
 {
@@ -171,61 +182,77 @@ NH_DEV typename Red::L seg_walk(const Red &red, const T *__restrict__ row, int64
     constexpr bool kRel = RelIndex<Red>::value;
     L st = red.linit();
     const int lane = G::lane();
-    using V = typename Vec16<T>::type;
-    constexpr int VN = Vec16<T>::n;
-    using U = typename VecU<T>::type;
-    const U *xv = reinterpret_cast<const U *>(row);
-    // a segment of at most TPR elements: one per lane, one load
-    const int64_t v0 = lo / VN, v1 = hi - lo <= TPR ? v0 : hi / VN;
-    for (int64_t c = v0 + lane; c < v1; c += int64_t(TPR) * kRUnroll) {
-        V r[kRUnroll];
-        decltype(pre.load(0)) aux[kRUnroll];
+    if constexpr (NARROW > 0) {
+        // Vectors would leave many lanes idle, and the walk below takes registers
+        // that rows in flight can use.  hi - lo is uniform.
+        T x[NARROW];
 #pragma unroll
-        for (int u = 0; u < kRUnroll; u++) {
-            const int64_t i = c + int64_t(u) * TPR;
-            if (i < v1) r[u] = NT ? V(__builtin_nontemporal_load(xv + i)) : V(xv[i]);
+        for (int k = 0; k < NARROW; k++)
+            if ((k == 0 || hi - lo > k * TPR) && lo + lane + k * TPR < hi) x[k] = row[lo + lane + k * TPR];
+#pragma unroll
+        for (int k = 0; k < NARROW; k++) {
+            const int64_t j = lo + lane + k * TPR;
+            if ((k == 0 || hi - lo > k * TPR) && j < hi) {
+                const T y = pre.one(x[k], j);
+                if (first && k == 0) *first = y;
+                red.lacc(st, y, kRel ? j - lo : j);
+            }
         }
-        if constexpr (Pre::kActive) {
+    } else {
+        using V = typename Vec16<T>::type;
+        constexpr int VN = Vec16<T>::n;
+        using U = typename VecU<T>::type;
+        const U *xv = reinterpret_cast<const U *>(row);
+        const int64_t v0 = lo / VN, v1 = hi / VN;
+        for (int64_t c = v0 + lane; c < v1; c += int64_t(TPR) * kRUnroll) {
+            V r[kRUnroll];
+            decltype(pre.load(0)) aux[kRUnroll];
 #pragma unroll
             for (int u = 0; u < kRUnroll; u++) {
                 const int64_t i = c + int64_t(u) * TPR;
-                if (i < v1) aux[u] = pre.load(i);
+                if (i < v1) r[u] = NT ? V(__builtin_nontemporal_load(xv + i)) : V(xv[i]);
             }
+            if constexpr (Pre::kActive) {
+#pragma unroll
+                for (int u = 0; u < kRUnroll; u++) {
+                    const int64_t i = c + int64_t(u) * TPR;
+                    if (i < v1) aux[u] = pre.load(i);
+                }
+#pragma unroll
+                for (int u = 0; u < kRUnroll; u++) {
+                    const int64_t i = c + int64_t(u) * TPR;
+                    if (i < v1) r[u] = pre.vec(r[u], aux[u], i);
+                }
+            }
+            if (first && c == v0 + lane) *first = r[0][0];
+            const int32_t rb = kRel ? int32_t(c - v0) * VN : 0;  // lo is a multiple of VN here
 #pragma unroll
             for (int u = 0; u < kRUnroll; u++) {
                 const int64_t i = c + int64_t(u) * TPR;
-                if (i < v1) r[u] = pre.vec(r[u], aux[u], i);
-            }
-        }
-        if (first && c == v0 + lane) *first = r[0][0];
-        const int32_t rb = kRel ? int32_t(c - v0) * VN : 0;  // lo is a multiple of VN here
+                if (i < v1) {
 #pragma unroll
-        for (int u = 0; u < kRUnroll; u++) {
-            const int64_t i = c + int64_t(u) * TPR;
-            if (i < v1) {
-#pragma unroll
-                for (int k = 0; k < VN; k++) {
-                    if constexpr (kRel) red.lacc(st, r[u][k], rb + (u * TPR * VN + k));
-                    else red.lacc(st, r[u][k], i * VN + k);
+                    for (int k = 0; k < VN; k++) {
+                        if constexpr (kRel) red.lacc(st, r[u][k], rb + (u * TPR * VN + k));
+                        else red.lacc(st, r[u][k], i * VN + k);
+                    }
                 }
             }
         }
-    }
-    const int64_t tail = v1 * VN > lo ? v1 * VN : lo;
-    for (int64_t j = tail + lane; j < hi; j += TPR) {
-        const T x = pre.one(row[j], j);
-        if (first && j == tail + lane && tail == lo) *first = x;
-        red.lacc(st, x, kRel ? j - lo : j);
+        for (int64_t j = (v1 * VN > lo ? v1 * VN : lo) + lane; j < hi; j += TPR) {
+            const T x = pre.one(row[j], j);
+            if (first && j == lo) *first = x;
+            red.lacc(st, x, kRel ? j - lo : j);
+        }
     }
     return G::reduce(st, [&](const L &a, const L &b) { return red.lcomb(a, b); });
 }
 
 // Reduce row elements [lo, hi) to the segment summary (`first`: see seg_walk).
-template <typename T, class Red, int TPR, bool NT>
+template <typename T, class Red, int TPR, bool NT, int NARROW = 0>
 NH_DEV typename Red::B seg_reduce(const Red &red, const T *__restrict__ row, int64_t lo, int64_t hi,
                                   T *first = nullptr)
 {
-    return red.template finish<TPR>(seg_walk<T, Red, TPR, NT>(red, row, lo, hi, NoPre{}, first), row, lo, hi);
+    return red.template finish<TPR>(seg_walk<T, Red, TPR, NT, NARROW>(red, row, lo, hi, NoPre{}, first), row, lo, hi);
 }
 
 // Reducers whose store() reads only element 0 of the row (argmax: x0 NaN
@@ -293,8 +320,16 @@ NH_DEV void publish(const Ticket &tk)
     }
 }
 
-// One group (wave or block) per row; a block of waves takes 4 rows.
-template <typename T, class Red, int TPR>
+// One group (wave or block) per row; a block of waves takes 4 rows.  Waves over
+// rows of up to 256 elements have forms of their own (NARROW, see narrow_of),
+// with 16-42 registers instead of 38-93: one walk for all widths left half the
+// lanes idle at 65 to 128 elements and kept 5 waves per SIMD busy at best.  Row
+// sum, row statistics, bias add with statistics, in vectors -> so, us: f32
+// [1 M, 2] 136, 267, 362 -> 131, 203, 194; [258111, 65] 47.7, 84, 148 -> 35.5, 54,
+// 59; [131072, 128] 23.0, 39.5, 70.9 -> 20.0, 28.6, 35.0; [65536, 256] 13.7, 21.3, 38.9
+// -> 13.9, 18.3, 25.7; f64 [131072, 128] 24.2, 37.0, 64.7 -> 24.4, 33.6, 52.6.  Four
+// scalars for the narrowest rows too: [1 M, 2] 158, 237, 212.
+template <typename T, class Red, int TPR, int NARROW = 0>
 __global__ __launch_bounds__(Grp<TPR>::kBlock) void k_reduce_rows(const T *__restrict__ x, int64_t rows, int64_t cols,
                                                                   int64_t ld, Red red, void *out, Ticket tk)
 {
@@ -308,13 +343,13 @@ __global__ __launch_bounds__(Grp<TPR>::kBlock) void k_reduce_rows(const T *__res
         // for the whole sequence than non-temporal ones
         if constexpr (StoreReadsFirst<Red>::value) {
             T x0 = T(0);
-            const typename Red::B b = seg_reduce<T, Red, TPR, false>(red, xr, 0, cols, &x0);
+            const typename Red::B b = seg_reduce<T, Red, TPR, false, NARROW>(red, xr, 0, cols, &x0);
             if (Grp<TPR>::lane() == 0) {
                 red.store(out, r, b, FirstOnly<T>{x0}, cols);
                 publish(tk);  // tickets are used with a single row only
             }
         } else {
-            const typename Red::B b = seg_reduce<T, Red, TPR, false>(red, xr, 0, cols);
+            const typename Red::B b = seg_reduce<T, Red, TPR, false, NARROW>(red, xr, 0, cols);
             if (Grp<TPR>::lane() == 0) {
                 red.store(out, r, b, xr, cols);
                 publish(tk);  // tickets are used with a single row only
@@ -446,6 +481,12 @@ int launch_reduce(const T *x, int64_t rows, int64_t cols, int64_t ld, const Red 
         NH_LAUNCH((k_reduce_seg<T, Red>), grid, dim3(kRBlock), 0, stream(), x, cols, ld, chunk, red, part);
         NH_LAUNCH((k_reduce_combine<T, Red>), dim3(unsigned(rows)), dim3(kRBlock), 0, stream(), x, cols, ld,
                            int(gx), red, part, out, tk);
+    } else if (plan.tpr == 64 && narrow_of<T>(cols) == 2) {
+        NH_LAUNCH((k_reduce_rows<T, Red, 64, 2>), dim3(rows_grid(rows, kRBlock / 64)), dim3(kRBlock), 0, stream(), x,
+                  rows, cols, ld, red, out, tk);
+    } else if (plan.tpr == 64 && narrow_of<T>(cols) == 4) {
+        NH_LAUNCH((k_reduce_rows<T, Red, 64, 4>), dim3(rows_grid(rows, kRBlock / 64)), dim3(kRBlock), 0, stream(), x,
+                  rows, cols, ld, red, out, tk);
     } else if (plan.tpr == 64) {
         NH_LAUNCH((k_reduce_rows<T, Red, 64>), dim3(rows_grid(rows, kRBlock / 64)), dim3(kRBlock), 0, stream(), x,
                   rows, cols, ld, red, out, tk);

@@ -208,3 +208,12 @@ def test_long_rows_around_a_row_per_cu(pn, ora, rows, cols, dt):
     """Long rows up to and past one per CU (blocks of 1024 or of 256 lanes)."""
     test_row_stats_equal_separate_calls(pn, ora, rows, cols, dt)
     test_bias_add_row_stats_equal_separate_calls(pn, ora, rows, cols, dt)
+
+
+@pytest.mark.parametrize("cols", [2, 64, 65, 127, 128, 129, 191, 192, 193, 255, 256, 257])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_narrow_rows(pn, ora, cols, dt):
+    """Rows that a wave reads as up to 2 or 4 scalars per lane, and the first
+    width past them: fused and separate calls agree bit for bit."""
+    test_row_stats_equal_separate_calls(pn, ora, 517, cols, dt)
+    test_bias_add_row_stats_equal_separate_calls(pn, ora, 517, cols, dt)
