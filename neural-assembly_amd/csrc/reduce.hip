@@ -294,9 +294,12 @@ static int row_stats_launch(const T *x, const T *bias, T *y, int64_t rows, int64
 // a second stage of one serial lane per column took 116 + 20 us at f32
 // [16384, 4096]; bias + GELU and these column sums 218 -> 144 us there, bias +
 // swish and column sums f64 [65536, 512] 286 -> 136 us.
+// WR: the block's waves that share a column group (4), or 1: each wave has a
+// group of its own (whole waves of columns, R = 1) and nothing to fold.
 constexpr int kColU = 8;
+constexpr int kColFewRows = 16;
 
-template <typename T, typename O>
+template <typename T, typename O, int WR>
 __global__ __launch_bounds__(256) void k_colsum(const T *__restrict__ x, int64_t rows, int64_t cols, int64_t chunk,
                                                 int LR, int64_t div, O *__restrict__ out)
 {
@@ -307,14 +310,15 @@ __global__ __launch_bounds__(256) void k_colsum(const T *__restrict__ x, int64_t
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int R = 64 / LR, ro = lane / LR, lc = lane % LR;
     const int64_t r0 = int64_t(blockIdx.y) * chunk, r1 = r0 + chunk < rows ? r0 + chunk : rows;
-    const int64_t groups = (cols + int64_t(LR) * VN - 1) / (int64_t(LR) * VN), step = 4 * int64_t(R);
+    const int64_t span = int64_t(LR) * VN * (4 / WR);  // columns of a block
+    const int64_t groups = (cols + span - 1) / span, step = WR * int64_t(R);
     for (int64_t cg = blockIdx.x; cg < groups; cg += gridDim.x) {
-        const int64_t c0 = (cg * LR + lc) * VN;
+        const int64_t c0 = ((WR == 4 ? cg : cg * 4 + w) * LR + lc) * VN;
         double s[VN];
 #pragma unroll
         for (int j = 0; j < VN; j++) s[j] = 0.0;
         if (ro < R && c0 < cols) {
-            int64_t r = r0 + int64_t(w) * R + ro;
+            int64_t r = r0 + (WR == 4 ? int64_t(w) * R : 0) + ro;
             if (c0 + VN <= cols) {
                 for (; r + (kColU - 1) * step < r1; r += kColU * step) {
                     V v[kColU];
@@ -339,6 +343,12 @@ __global__ __launch_bounds__(256) void k_colsum(const T *__restrict__ x, int64_t
                         if (c0 + j < cols) s[j] += double(x[r * cols + c0 + j]);
                 }
             }
+        }
+        if constexpr (WR == 1) {
+#pragma unroll
+            for (int j = 0; j < VN; j++)
+                if (c0 + j < cols) out[int64_t(blockIdx.y) * cols + c0 + j] = O(div > 1 ? s[j] / double(div) : s[j]);
+            continue;
         }
         // the block's 4 R row streams of column lane lc, folded by halves
         const int e = w * R + ro;
@@ -376,25 +386,35 @@ static int colsum(const T *src, int64_t rows, int64_t cols, bool mean, T *dst)
         return unsigned(g < kMaxGridBlocks ? g : kMaxGridBlocks);
     };
     constexpr int VN = Vec16<T>::n;
-    // about 4 blocks per CU over the column groups, each chunk at least two
-    // batches of rows
     const int LR = lanes(VN);
-    int64_t nchunks = ceil_div(int64_t(num_cus()) * 4, int64_t(grid_x(VN)));
+    const int64_t div = mean ? rows : 1;
+    // Up to 16 rows leave a block's four waves four rows each at most and the
+    // fold more work than the sums: a wave per column group.  f32 [1, 1000000]
+    // 9.8 -> 4.1 us, [8, 1000000] 12.0 -> 5.8, f64 [4, 1000000] 14.7 -> 7.5.
+    if (LR == 64 && rows <= kColFewRows) {
+        NH_LAUNCH((k_colsum<T, T, 1>), dim3(unsigned(ceil_div(int64_t(grid_x(VN)), 4))), dim3(256), 0, stream(), src,
+                  rows, cols, rows, LR, div, dst);
+        return check_launch();
+    }
+    // about 4 blocks per CU (what it holds) over the column groups, to the
+    // nearest chunk, each chunk at least two batches of rows; one chunk more left
+    // a second round nearly empty and paid for its partials: f32 [67, 250000]
+    // 19.5 -> 11.5 us, [333, 50257] 21.7 -> 16.2, f64 [170, 98304] 26.2 -> 19.8
+    int64_t nchunks = (int64_t(num_cus()) * 4 + grid_x(VN) / 2) / int64_t(grid_x(VN));
     const int64_t most = ceil_div(rows, int64_t(4 * (64 / LR)) * kColU * 2);
     nchunks = nchunks > most ? most : nchunks;
     nchunks = nchunks < 1 ? 1 : (nchunks > 65535 ? 65535 : nchunks);
     const int64_t chunk = ceil_div(rows > 0 ? rows : 1, nchunks);
     nchunks = ceil_div(rows > 0 ? rows : 1, chunk);
-    const int64_t div = mean ? rows : 1;
     if (nchunks == 1) {
-        NH_LAUNCH((k_colsum<T, T>), dim3(grid_x(VN)), dim3(256), 0, stream(), src, rows, cols, chunk, LR, div, dst);
+        NH_LAUNCH((k_colsum<T, T, 4>), dim3(grid_x(VN)), dim3(256), 0, stream(), src, rows, cols, chunk, LR, div, dst);
         return check_launch();
     }
     double *part = static_cast<double *>(dev_alloc(size_t(nchunks * cols) * sizeof(double)));
     if (!part) return set_error(NEURAL_ERR_OUT_OF_MEMORY);
-    NH_LAUNCH((k_colsum<T, double>), dim3(grid_x(VN), unsigned(nchunks)), dim3(256), 0, stream(), src, rows, cols,
+    NH_LAUNCH((k_colsum<T, double, 4>), dim3(grid_x(VN), unsigned(nchunks)), dim3(256), 0, stream(), src, rows, cols,
               chunk, LR, int64_t(1), part);
-    NH_LAUNCH((k_colsum<double, T>), dim3(grid_x(2)), dim3(256), 0, stream(), part, nchunks, cols, nchunks, lanes(2),
+    NH_LAUNCH((k_colsum<double, T, 4>), dim3(grid_x(2)), dim3(256), 0, stream(), part, nchunks, cols, nchunks, lanes(2),
               div, dst);
     const int rc = check_launch();
     dev_free(part);

@@ -323,3 +323,34 @@ def test_row_reductions_unaligned_edges(pn, ora, dt, cols):
             same_bits(at, at2)
     finally:
         pn.set_stream(None)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 8, 15, 16, 17, 67])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_colsum_few_rows(pn, dt, rows):
+    """Few rows of many columns, where each wave has columns of its own (up to
+    16 rows): widths around a wave's and a block's columns and over several
+    blocks, buffers that start inside a vector; bounds of test_colsum_edges."""
+    import torch
+    rng = np.random.default_rng(rows)
+    tol = 1e-5 if dt == np.float32 else 1e-13
+    pn.set_stream(torch.cuda.current_stream().cuda_stream)
+    try:
+        for cols in (127, 128, 129, 255, 256, 257, 511, 512, 1023, 1025, 70_003):
+            x = rng.normal(0, 3, (rows, cols)).astype(dt)
+            buf = torch.zeros(rows * cols + 3, dtype=torch.float32 if dt == np.float32 else torch.float64,
+                              device="cuda")
+            e = x.astype(np.float64).sum(axis=0)
+            bound = tol * np.abs(x.astype(np.float64)).sum(axis=0)
+            for off in (0, 1):
+                v = buf[off:off + rows * cols].view(rows, cols)
+                v.copy_(torch.from_numpy(x))
+                o = torch.full((cols + 2,), 7.0, dtype=buf.dtype, device="cuda")
+                t, out = pn.Tensor.from_torch(v), pn.Tensor.from_torch(o[1:cols + 1])
+                assert pn.core._lib.neural_reduce_sum(t._ptr, 0, out._ptr) == 0
+                got = o.cpu().numpy()
+                assert np.all(np.abs(got[1:-1] - e) <= bound) and got[0] == 7.0 and got[-1] == 7.0, (cols, off)
+                assert pn.core._lib.neural_reduce_mean(t._ptr, 0, out._ptr) == 0
+                assert np.all(np.abs(o.cpu().numpy()[1:-1] - e / rows) <= bound / rows), (cols, off)
+    finally:
+        pn.set_stream(None)
