@@ -146,16 +146,36 @@ struct StepTab {
 };
 static_assert(sizeof(StepTab) + sizeof(AdamArgs) + 64 <= 4096, "kernel arguments");
 
-// One element per lane, `tiles` 256-lane tiles per block (1 unless the grid
-// would pass kMaxGridBlocks); a block finds its tensor with one compare of its
-// index per lane and two ballots.
+// One element per lane.
+template <typename T, int TYPE>
+NH_DEV void step_elem(const StepEntry &e, int64_t j, const AdamArgs &a)
+{
+    T *__restrict__ p = static_cast<T *>(e.p);
+    const T *__restrict__ g = static_cast<const T *>(e.g);
+    if constexpr (TYPE == OPT_SGD) {  // sgd_step_impl (optimizers_c.c:218-249)
+        const T pv = ld_nt(p + j);  // with the other loads: after the store to m it waits (50 M f64 302 us, 310)
+        const double nv = a.b1 * ld_nt(e.m + j) + double(ld_nt(g + j));
+        st_nt(e.m + j, nv);
+        st_nt(p + j, pv - T(a.lr * nv));
+    } else {
+        const T pd = ld_nt(p + j), gd = ld_nt(g + j);
+        double mm = ld_nt(e.m + j), vq = ld_nt(e.v + j);
+        T r;
+        if constexpr (sizeof(T) == 4) r = TYPE == OPT_ADAMW ? adamw_f32(pd, gd, mm, vq, a) : adam_f32(pd, gd, mm, vq, a);
+        else r = TYPE == OPT_ADAMW ? adamw_f64(pd, gd, mm, vq, a) : adam_f64(pd, gd, mm, vq, a);
+        st_nt(p + j, r);
+        st_nt(e.m + j, mm);
+        st_nt(e.v + j, vq);
+    }
+}
+
+// `tiles` 256-lane tiles per block (1 unless the grid would pass
+// kMaxGridBlocks); a block finds its tensor with one compare of its index per
+// lane and two ballots.
 // Bound by HBM, 44 B per element (f32 Adam).  A launch per tensor let the chip
 // drain and refill between tensors: norm pass and step over 85 M values in 144
 // tensors 1072 -> 718 us (70 of them the norm), 1.2 M values in 288 tensors
-// 1033 -> 90 us, 50 M in 12 413 -> 389 us; large tensors gain little.
-// Measured at 100 M f32 params with f64 moments, one tensor: 698 us with one
-// element per lane, 710-725 us for 2 or 4 in flight per lane, 825 us for a grid
-// of 16 blocks per CU striding over the tensor.
+// 1033 -> 90 us, 50 M in 12 413 -> 389 us.
 template <typename T, int TYPE>
 __global__ __launch_bounds__(kOBlock) void k_opt_step(const StepTab tab, AdamArgs a)
 {
@@ -169,35 +189,40 @@ __global__ __launch_bounds__(kOBlock) void k_opt_step(const StepTab tab, AdamArg
         i = __builtin_amdgcn_readfirstlane(int(__popcll(__ballot(c0)) + __popcll(__ballot(c1))) - 1);
     }
     const StepEntry &e = tab.e[i];
-    T *__restrict__ p = static_cast<T *>(e.p);
-    const T *__restrict__ g = static_cast<const T *>(e.g);
     const int64_t j0 = int64_t(b - tab.first[i]) * tab.tiles * kOBlock + threadIdx.x;
     for (int k = 0; k < tab.tiles; k++) {
         const int64_t j = j0 + int64_t(k) * kOBlock;
         if (j >= e.n) return;
-        if constexpr (TYPE == OPT_SGD) {  // sgd_step_impl (optimizers_c.c:218-249)
-            const double nv = a.b1 * ld_nt(e.m + j) + double(ld_nt(g + j));
-            st_nt(e.m + j, nv);
-            st_nt(p + j, ld_nt(p + j) - T(a.lr * nv));
-        } else {
-            const T pd = ld_nt(p + j), gd = ld_nt(g + j);
-            double mm = ld_nt(e.m + j), vq = ld_nt(e.v + j);
-            T r;
-            if constexpr (sizeof(T) == 4) r = TYPE == OPT_ADAMW ? adamw_f32(pd, gd, mm, vq, a) : adam_f32(pd, gd, mm, vq, a);
-            else r = TYPE == OPT_ADAMW ? adamw_f64(pd, gd, mm, vq, a) : adam_f64(pd, gd, mm, vq, a);
-            st_nt(p + j, r);
-            st_nt(e.m + j, mm);
-            st_nt(e.v + j, vq);
-        }
+        step_elem<T, TYPE>(e, j, a);
     }
+}
+
+// One tensor whose grid fits a launch: no table to look up before the first
+// load.  100 M f32 values, AdamW 682 -> 679 us, SGD 477 -> 450; 2 or 4 elements in
+// flight per lane or a grid of 16 blocks per CU striding over the tensor took
+// 2-18% longer than one element per lane.
+template <typename T, int TYPE>
+__global__ __launch_bounds__(kOBlock) void k_opt_step_one(const StepEntry e, AdamArgs a)
+{
+    const int64_t j = int64_t(blockIdx.x) * kOBlock + threadIdx.x;
+    if (j < e.n) step_elem<T, TYPE>(e, j, a);
+}
+
+template <typename T, int TYPE>
+static void launch_step_of(const StepTab &tab, unsigned blocks, const AdamArgs &a)
+{
+    if (tab.count == 1 && tab.tiles == 1)
+        NH_LAUNCH((k_opt_step_one<T, TYPE>), dim3(blocks), dim3(kOBlock), 0, stream(), tab.e[0], a);
+    else
+        NH_LAUNCH((k_opt_step<T, TYPE>), dim3(blocks), dim3(kOBlock), 0, stream(), tab, a);
 }
 
 template <typename T>
 static int launch_step(int type, const StepTab &tab, unsigned blocks, const AdamArgs &a)
 {
-    if (type == OPT_SGD) NH_LAUNCH((k_opt_step<T, OPT_SGD>), dim3(blocks), dim3(kOBlock), 0, stream(), tab, a);
-    else if (type == OPT_ADAM) NH_LAUNCH((k_opt_step<T, OPT_ADAM>), dim3(blocks), dim3(kOBlock), 0, stream(), tab, a);
-    else NH_LAUNCH((k_opt_step<T, OPT_ADAMW>), dim3(blocks), dim3(kOBlock), 0, stream(), tab, a);
+    if (type == OPT_SGD) launch_step_of<T, OPT_SGD>(tab, blocks, a);
+    else if (type == OPT_ADAM) launch_step_of<T, OPT_ADAM>(tab, blocks, a);
+    else launch_step_of<T, OPT_ADAMW>(tab, blocks, a);
     return check_launch();
 }
 
