@@ -130,8 +130,10 @@ NH_DEV double ce_diff(T x, double m)
 // past the vectors in one scalar of the first lanes (RowCut; the
 // other lanes' scalar is -inf and adds nothing).  FULL: the row is exactly NT * VPT vectors, so no
 // element needs a bounds check (per-element checks around the exp turn into
-// exec-mask branches).  The lane that
-// holds the target picks x_t or e_t up as it passes; e_c replaces x_c.
+// exec-mask branches).  e_c replaces x_c.  x_t is read again from memory, beside
+// the row (a pick from the registers, with an exp of its own for the tensor
+// loss: f64 [65536, 256] 44.0 us, now 40.0); the tensor loss's lane that holds the
+// target keeps the e_t it computes.
 //
 // What bounds it: HBM where enough rows are in flight, so that one block loads
 // or stores while another computes.  A 201 KB row of 50257 f32 classes is 25
@@ -139,16 +141,17 @@ NH_DEV double ce_diff(T x, double m)
 // lane reads and writes its own slots only), two blocks per CU.  With all 25
 // in registers the compiler spilled 35-84 of them to scratch memory
 // ([4096, 50257] fused f32 373 us against 318, both with stores cut at 64-byte
-// boundaries; three passes of 4-byte accesses took 861).  Rows of an odd width
-// start anywhere, and a vector store that starts inside a 64-byte block is
-// slower: 340 us there, 315 with each row cut at the first boundary of its own
-// gradient.  But then the order of a row's sums, and so the result's last
-// bits, went by the buffer's address; equal bits are promised.
+// boundaries; three passes of 4-byte accesses took 861); this form spills 4 in
+// f32 and 13 in f64.  Rows of an odd width start anywhere, and a vector store
+// that starts inside a 64-byte block is slower: 331 us there, 314 with each row
+// cut at the first boundary of its own gradient.  But then the order of a row's
+// sums, and so the result's last bits, went by the buffer's address; equal bits
+// are promised.
 //
 // WAVES: the minimum waves per SIMD the compiler must fit (1: its own
-// choice).  The f64 forward with rows of up to 1024 values takes 5 (83-84
-// VGPRs, no spills; 103 and 4 waves otherwise): 88.8-90.1 -> 82.9 us at
-// [65536,1024] (A/B in one run).  The fused and backward forms keep every
+// choice).  The f64 forward with rows of up to 1024 values takes 5 (no
+// spills; 103 VGPRs and 4 waves otherwise when it was measured): 88.8-90.1 -> 82.9
+// us at [65536,1024] (A/B in one run).  The fused and backward forms keep every
 // exp for the gradient and spill under that bound (fused f64 180 -> 331 us),
 // as do rows of 2048 doubles.
 template <typename T, int NT, int VPT, int LV, int MODE, bool FULL, int WAVES>
@@ -198,16 +201,11 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
     for (int k = 0; k < LV; k++)
         if (in_row(VPT + k)) w[k] = __builtin_nontemporal_load(xv + lane + (VPT + k) * NT);
     if (lane < nsc) vt = xr[cut.sc(lane)];
+    T xt = LOSS && ok ? xr[t] : T(0);
     // the target's vector and slot, or the scalar that holds it (-1: neither)
     const bool t_vec = ok && t < int64_t(FULL ? NT * VPT : cut.ncv) * VN;
     const int tv = t_vec ? int(t / VN) : -1, tj = int(t % VN);
     const bool t_mine = ok && !t_vec && lane < nsc && cut.sc(lane) == t;  // in this lane's scalar
-    const auto at = [&](const V &q) {  // q[tj]
-        T x = q[0];
-#pragma unroll
-        for (int j = 1; j < VN; j++) x = j == tj ? q[j] : x;
-        return x;
-    };
     T mx = vt == vt ? vt : -inf_t<T>();
 #pragma unroll
     for (int k = 0; k < VPT; k++)
@@ -235,20 +233,22 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
     using Acc = typename std::conditional<MODE == CE_ASM && sizeof(T) == 4 && !WIDE, float, double>::type;
     Acc sl = Acc(0);
     double acc = 0.0;
-    double pick = 0.0;  // the lane that holds the target: x_t - m (the losses' A) or e_t (tensor CE)
+    double e_t = 0.0;  // tensor CE: the lane that holds the target has its e here
     bool mine = t_mine;
     const auto sum_vec = [&](V &q, int k) {  // vector lane + k NT of the row
-        if (MODE != CE_LS_BWD && lane + k * NT == tv) {
-            const T x1 = at(q);
-            pick = MODE == CE_ASM ? row_exp(x1) : ce_diff<T, WIDE>(x1, m);
-            mine = true;
-        }
+        double e[VN];
 #pragma unroll
         for (int j = 0; j < VN; j++) {
-            const double e = row_exp(q[j]);
+            e[j] = row_exp(q[j]);
             if constexpr (LOSS) acc += ce_diff<T, WIDE>(q[j], m);
-            if constexpr (GRAD) q[j] = T(e);
-            sl += Acc(e);
+            if constexpr (GRAD) q[j] = T(e[j]);
+            sl += Acc(e[j]);
+        }
+        if (MODE == CE_ASM && lane + k * NT == tv) {
+            e_t = e[0];
+#pragma unroll
+            for (int j = 1; j < VN; j++) e_t = j == tj ? e[j] : e_t;
+            mine = true;
         }
     };
 #pragma unroll
@@ -264,11 +264,13 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
     if (nsc) {  // uniform
         const double e = row_exp(vt);
         if (LOSS && lane < nsc) acc += ce_diff<T, WIDE>(vt, m);
-        if (t_mine) pick = MODE == CE_ASM ? e : ce_diff<T, WIDE>(vt, m);
+        if (MODE == CE_ASM && t_mine) e_t = e;
         if constexpr (GRAD) vt = T(e);
         sl += Acc(e);
     }
     const double s = G::sum(double(sl), lds_s);
+    // x_t is read before any gradient is written, which may be over the logits
+    if constexpr (LOSS && GRAD) asm volatile("" : "+v"(xt) : : "memory");
     if (!ok) {
         if (lane == 0) {
             __hip_atomic_store(a.bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -280,7 +282,7 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
         // p_t = e_t / sum (f32: e_t, sum and p_t rounded to float); the row's
         // loss -log(p_t + 1e-7) is taken in the summing pass (RedCeLoss), where
         // the double log runs on all lanes instead of on lane 0 of every row.
-        if (mine) a.row_loss[r] = sizeof(T) == 4 ? double(float(pick) / float(s)) : pick / s;
+        if (mine) a.row_loss[r] = sizeof(T) == 4 ? double(float(e_t) / float(s)) : e_t / s;
         return;
     }
     const double st0 = a.alpha / double(cols), st1 = st0 + (1.0 - a.alpha);
@@ -306,9 +308,9 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
         if (lane < nsc) gr[cut.sc(lane)] = grad(vt, t_mine);
     }
     if constexpr (LOSS) {
-        acc = G::sum(st0 * acc + (mine ? (st1 - st0) * pick : 0.0), lds_a);
+        acc = G::sum(acc, lds_a);
         if (lane == 0) {
-            a.row_loss[r] = acc;
+            a.row_loss[r] = st0 * acc + (st1 - st0) * ce_diff<T, WIDE>(xt, m);
             a.row_s[r] = s;
         }
     }
@@ -336,7 +338,7 @@ __global__ __launch_bounds__(kCeWide) void k_ce_stream(const T *__restrict__ x, 
     const U *xv = reinterpret_cast<const U *>(xr);
     int64_t t = 0;
     const bool ok = loss_target(a.tidx, static_cast<const T *>(a.tval), r, cols, t);
-    const T xt = ok ? xr[t] : T(0);
+    T xt = ok ? xr[t] : T(0);
     const auto row_exp = [](T xv, double m) {
         return sizeof(T) == 8 ? row_exp_d(double(xv), m) : row_exp_f(float(xv), m);
     };
@@ -378,6 +380,7 @@ __global__ __launch_bounds__(kCeWide) void k_ce_stream(const T *__restrict__ x, 
     // a row of only -inf is NaN, as exp(-inf - -inf) makes it
     s = G::sum(s == 0.0 ? s : s * exp(mr - m), lds_s);
     if (m == -__builtin_inf()) s = __builtin_nan("");
+    if constexpr (LOSS && GRAD) asm volatile("" : "+v"(xt) : : "memory");  // before any gradient is written
     if (!ok) {
         if (threadIdx.x == 0) {
             __hip_atomic_store(a.bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -437,7 +440,9 @@ static void launch_ce_rows(const T *x, const CeArgs &a)
     for_row_launches(a.rows, block / NT, [&](unsigned g, int64_t base) {
         if constexpr (NT <= 64) {
             if (a.cols == int64_t(NT) * VPT * Vec16<T>::n) {
-                constexpr unsigned lds = sizeof(T) == 4 && VPT >= 4 ? kFullRowsLds : 0;
+                // (the tensor loss, which stores nothing, wants it from 8 vectors: f32
+                // [65536, 1024] 57.6 us with it, 50.4 without, [32768, 2048] 49.4, 51.1)
+                constexpr unsigned lds = sizeof(T) == 4 && VPT >= (MODE == CE_ASM ? 8 : 4) ? kFullRowsLds : 0;
                 NH_LAUNCH((k_ce_rows<T, NT, VPT, LV, MODE, true, W>), dim3(g), dim3(block), lds, stream(), x, a, base);
                 return;
             }

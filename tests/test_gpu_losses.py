@@ -497,3 +497,23 @@ def test_loss_sum_over_batches(pn, b):
         p = np.exp(x64 - x64.max(axis=1, keepdims=True))
         want_ce = np.mean(-np.log((p / p.sum(axis=1, keepdims=True))[np.arange(b), t] + 1e-7))
         assert abs(ce.value - want_ce) <= rel * abs(want_ce) + floor
+
+
+@pytest.mark.parametrize("k", [10, 64, 513, 1001, 2048, 4099, 8193, 33001, 49152, 98311])
+@pytest.mark.parametrize("dt", ["float64", "float32"])
+def test_fused_in_place(pn, dt, k):
+    """The gradient written over the logits: same loss and gradient bits."""
+    import torch
+    lib = pn.core._lib
+    n, f64 = 9, dt == "float64"
+    fn = lib.label_smoothing_ce_fused_dev if f64 else lib.label_smoothing_ce_fused_f32_dev
+    rng = np.random.default_rng(k)
+    x = torch.from_numpy(rng.normal(0, 3, (n, k)).astype(dt)).cuda()
+    t = torch.from_numpy(rng.integers(0, k, n)).cuda()
+    g, loss = torch.empty_like(x), torch.zeros(2, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    assert fn(x.data_ptr(), t.data_ptr(), n, k, 0.1, loss.data_ptr(), g.data_ptr()) == 0
+    assert fn(x.data_ptr(), t.data_ptr(), n, k, 0.1, loss.data_ptr() + 8, x.data_ptr()) == 0
+    pn.synchronize()
+    assert loss[0].item() == loss[1].item()
+    same_bits(x.cpu().numpy(), g.cpu().numpy())
