@@ -17,9 +17,9 @@
 // softmax.  A NaN anywhere in a row makes the whole row NaN, as in the
 // reference (the NaN reaches the sum).
 //
-// A row is held in registers by one group of lanes -- a wave up to 4096 f32 /
-// 2048 f64 values, a block of 256 to 1024 lanes beyond, up to 98304 / 49152
-// values -- so it is read once and written once at any width and alignment:
+// A row is held in registers by one group of lanes -- part of a wave or a wave up
+// to 2048 f32 / 1024 f64 values and at exactly twice that, else a block of 256 to
+// 1024 lanes, up to 98304 / 49152 values -- so it is read once and written once at any width and alignment:
 // 16-byte accesses at the element's own alignment and one scalar per lane for
 // the values at the row's ends.  Wider rows are read twice.
 #include <cmath>
@@ -128,7 +128,10 @@ __global__ __launch_bounds__(NT < kSmBlock ? kSmBlock : NT, NT == 512 ? 4 : 1) v
         s += double(e);
     }
     s = G::sum(s, lds_s);
-    double lse = 0.0;  // s >= 1: the maximum contributes 1
+    // s >= 1: the maximum contributes 1.  f64 rows of whole vectors within a wave
+    // take log_ge1 (about 3 ulp, fewer instructions per row); the others, whose
+    // rows are longer or were always logged by the library, its log.
+    double lse = 0.0;
     if constexpr (LOG && sizeof(T) == 4) lse = log_ge1(s);
     else if constexpr (LOG) lse = NT <= 64 && cols % VN == 0 ? log_ge1(s) : log(s);
     const double rs = LOG ? 0.0 : 1.0 / s;
@@ -243,7 +246,10 @@ static void launch_rows(const T *x, T *y, int64_t rows, int64_t cols)
 // most rows are in flight.  Narrow rows share a wave, 16 rows of up to 4
 // vectors, 4 of up to 64, 2 of up to 128; where the rows' ends are not vector
 // ends the last take a whole wave (its longer stores: [100000, 511] 73 against
-// 84 us).  Before (a wave per aligned row of up to 4096 values, else three
+// 84 us).  16 vectors per lane only where every one is full: between 2048 and
+// 4096 f32 values 256 lanes with up to 4 or 8 vectors answer few rows sooner and
+// many alike (f32 [131, 4000] 6.2 -> 3.6 us, [4194, 4000] 24.5 -> 23.3, f64 [255, 2049]
+// 8.1 -> 4.8).  Before (a wave per aligned row of up to 4096 values, else three
 // passes of 4-byte accesses) -> now, us:
 //   f32 [55392, 577] softmax / log-softmax  159 -> 45 / 160 -> 47 (256 MB, 5.7 TB/s)
 //       [200000, 16] 42.2 -> 6.0, [200000, 64] 47.4 -> 18.1, [200000, 63] 203 -> 23.7
@@ -263,7 +269,8 @@ static int launch_softmax(const T *x, T *y, int64_t rows, int64_t cols)
     else if (ncv <= 64 * 2) launch_rows<T, LOG, 64, 2>(x, y, rows, cols);
     else if (ncv <= 64 * 4) launch_rows<T, LOG, 64, 4>(x, y, rows, cols);
     else if (ncv <= 64 * 8) launch_rows<T, LOG, 64, 8>(x, y, rows, cols);
-    else if (ncv <= 64 * 16) launch_rows<T, LOG, 64, 16>(x, y, rows, cols);
+    else if (cols == 64 * 16 * Vec16<T>::n) launch_rows<T, LOG, 64, 16>(x, y, rows, cols);
+    else if (ncv <= 256 * 4) launch_rows<T, LOG, 256, 4>(x, y, rows, cols);
     else if (ncv <= 256 * 8) launch_rows<T, LOG, 256, 8>(x, y, rows, cols);
     else if (ncv <= 256 * 16) launch_rows<T, LOG, 256, 16>(x, y, rows, cols);
     else if (ncv <= 512 * 16) launch_rows<T, LOG, 512, 16>(x, y, rows, cols);
