@@ -426,12 +426,15 @@ ReducePlan reduce_plan(int64_t rows, int64_t cols, bool costly = false)
     // the usual 256 lanes, several blocks to a CU: row statistics f32
     // [838, 20000] 12.6 us, with 1024 lanes, one block to a CU in a fourth round,
     // 21.3, in segments 16.5; the sum alone 11.2 / 11.8 / 12.5.
-    // Not for reducers that compute a function per element (costly): over 32768
-    // double logarithms one CU takes 18 us longer than segments do (tensor loss
-    // f32 [32768, 512] 43 us against 25; quantization error of 65536 values 24
-    // against 12.6).
+    // Reducers that compute a function per element (costly) take them up to 4096
+    // elements only, where 256 lanes would make 16 rounds (fused loss f64
+    // [4096, 128] 8.8 us, 10.3): over 32768 double logarithms one CU takes 18 us
+    // longer than segments do (tensor loss f32 [32768, 512] 43 us against 25;
+    // quantization error of 65536 values 24 against 12.6).
     constexpr int64_t kWideBytes = 256 << 10;
-    if (!costly && rows < want && cols * int64_t(sizeof(T)) <= kWideBytes && cols > 2 * kGran) {
+    if (costly && rows <= num_cus() && cols > 2048 && cols <= 4096) {
+        p.tpr = kRWide;
+    } else if (!costly && rows < want && cols * int64_t(sizeof(T)) <= kWideBytes && cols > 2 * kGran) {
         if (rows <= num_cus()) p.tpr = kRWide;
     } else if (rows < want && cols > 2 * kGran) {
         p.gx = ceil_div(want, rows);
@@ -490,10 +493,9 @@ int launch_reduce(const T *x, int64_t rows, int64_t cols, int64_t ld, const Red 
     } else if (plan.tpr == 64) {
         NH_LAUNCH((k_reduce_rows<T, Red, 64>), dim3(rows_grid(rows, kRBlock / 64)), dim3(kRBlock), 0, stream(), x,
                   rows, cols, ld, red, out, tk);
-    } else if (!CostlyElem<Red>::value && plan.tpr == kRWide) {
-        if constexpr (!CostlyElem<Red>::value)
-            NH_LAUNCH((k_reduce_rows<T, Red, kRWide>), dim3(rows_grid(rows, 1)), dim3(kRWide), 0, stream(), x, rows,
-                      cols, ld, red, out, tk);
+    } else if (plan.tpr == kRWide) {
+        NH_LAUNCH((k_reduce_rows<T, Red, kRWide>), dim3(rows_grid(rows, 1)), dim3(kRWide), 0, stream(), x, rows, cols,
+                  ld, red, out, tk);
     } else {
         NH_LAUNCH((k_reduce_rows<T, Red, kRBlock>), dim3(rows_grid(rows, 1)), dim3(kRBlock), 0, stream(), x, rows,
                   cols, ld, red, out, tk);
