@@ -940,7 +940,7 @@ def _cfg5(torch, pn, lib, clock, dev, g, cpu_on, out, detail):
            *clock.op(scan), host_call_us=clock.host_call_us(scan))
     flags = (hn.value, hi.value)
     opt = pn.AdamW(1e-3, 0.9, 0.999, 1e-8, 0.01)
-    cf.add("adamw", "k_opt_step<float, AdamW>", 44 * NA, NA, *clock.op(lambda: opt.step([tp], [tg])))
+    cf.add("adamw", "k_opt_step_one<float, AdamW>", 44 * NA, NA, *clock.op(lambda: opt.step([tp], [tg])))
     lib.neural_tensor_scan(tcl._ptr, ctypes.byref(hn), ctypes.byref(hi), ctypes.byref(ss))
     clean_norm = ss.value ** 0.5
     cpu = cpu_cfg5(p, clean, gr) if cpu_on else None
