@@ -175,6 +175,7 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
     __shared__ T lds_m[G::kWaves];
     __shared__ double lds_s[G::kWaves], lds_a[G::kWaves];
     __shared__ V more[LV > 0 ? LV : 1][LV > 0 ? NT : 1];
+    __shared__ T lds_xt;
     if constexpr (kTab) {
         if (threadIdx.x < 64) etab[threadIdx.x] = exp2(double(threadIdx.x) * (1.0 / 64.0));
         __syncthreads();
@@ -220,6 +221,10 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
             for (int j = 0; j < VN; j++) mx = fmax_nn(mx, w[k][j]);
             more[k][lane] = w[k];
         }
+    // x_t waits in LDS where a block holds the row (a register kept for it spilled
+    // others: fused f32 [256, 65536] 30.8 -> 43.4 us); lane 0 alone uses it
+    if constexpr (LOSS && WIDE)
+        if (lane == 0) lds_xt = xt;
     const double m = double(G::max(mx, lds_m));
     const auto row_exp = [&](T xv) {
         if constexpr (kTab) return exp_tab(double(xv) - m, etab);
@@ -270,7 +275,7 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
     }
     const double s = G::sum(double(sl), lds_s);
     // x_t is read before any gradient is written, which may be over the logits
-    if constexpr (LOSS && GRAD) asm volatile("" : "+v"(xt) : : "memory");
+    if constexpr (LOSS && GRAD && !WIDE) asm volatile("" : "+v"(xt) : : "memory");
     if (!ok) {
         if (lane == 0) {
             __hip_atomic_store(a.bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -310,7 +315,7 @@ __global__ __launch_bounds__(NT < 256 ? 256 : NT, WAVES) void k_ce_rows(const T 
     if constexpr (LOSS) {
         acc = G::sum(acc, lds_a);
         if (lane == 0) {
-            a.row_loss[r] = st0 * acc + (st1 - st0) * ce_diff<T, WIDE>(xt, m);
+            a.row_loss[r] = st0 * acc + (st1 - st0) * ce_diff<T, WIDE>(WIDE ? lds_xt : xt, m);
             a.row_s[r] = s;
         }
     }
