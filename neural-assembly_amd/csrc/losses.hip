@@ -142,7 +142,7 @@ NH_DEV double ce_diff(T x, double m)
 // in registers the compiler spilled 35-84 of them to scratch memory
 // ([4096, 50257] fused f32 373 us against 318, both with stores cut at 64-byte
 // boundaries; three passes of 4-byte accesses took 861); this form spills 4 in
-// f32 and 13 in f64.  Rows of an odd width start anywhere, and a vector store
+// f32 and 11 in f64.  Rows of an odd width start anywhere, and a vector store
 // that starts inside a 64-byte block is slower: 331 us there, 314 with each row
 // cut at the first boundary of its own gradient.  But then the order of a row's
 // sums, and so the result's last bits, went by the buffer's address; equal bits
